@@ -236,10 +236,10 @@ int vmc_ensemble_get_inverse(vmc_ensemble *e, double *inv, void *stream);
  * registers (7, 19, 27, 33, 57 or 81 electrons per spin, FP32 also 123 and
  * 147; equal spins or polarised); VMC_KERNEL_DELAYED (FP64, at most 160
  * electrons per spin) keeps the inverse in HBM and applies accepted moves
- * as delayed rank-8 Woodbury updates on the matrix cores.
+ * as delayed Woodbury updates on the matrix cores, a block of moves at a time.
  * VMC_KERNEL_AUTO (default) takes the register kernel whenever it applies,
- * else, in FP64, the delayed-update kernel when the inverses do not fit the
- * generic kernel's LDS.  No reference counterpart: the reference has a
+ * else, in FP64, the delayed-update kernel (any spins, up to about 500
+ * electrons per spin), else the generic kernel.  No reference counterpart: the reference has a
  * single CPU code path (its rank-1 update, slater_plane_wave.cpp:367-423);
  * this is the autotuner's knob.  VMC_ERR_INVALID if the system does not fit
  * the requested kernel. */

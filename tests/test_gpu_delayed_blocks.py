@@ -1,0 +1,64 @@
+"""GPU parity of the FP64 delayed-update sweep's blocks (vmc_sweep_du.hip).
+
+A block takes up to 32 movers per determinant, 16 below 17 electrons, and
+flushes at most 16 accepted moves in row tiles of 16; sizes below sit at the
+edges of blocks, tiles and instantiations, with equal spins, unequal spins
+(one determinant per block) and one determinant (above 160 electrons the row
+tile is read twice).  The device follows the oracle's Philox twin move for
+move: positions equal to the rounding of the FP64 proposal (1e-12 L), and the
+local energy after each sweep within 1e-9 of the oracle's, the bound the
+delayed-update kernel has at its other sizes.
+"""
+import numpy as np
+import pytest
+
+from helpers import oracle_system
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 0), (2, 1), (8, 1), (16, 16), (17, 17), (19, 7), (7, 19), (32, 32), (34, 33), (48, 48), (49, 49),
+         (64, 64), (65, 65), (96, 96), (97, 97), (128, 0), (129, 129), (160, 160), (161, 0), (177, 5)]
+
+
+@pytest.mark.parametrize("n_up,n_dn", SIZES, ids=[f"{a}+{b}" for a, b in SIZES])
+def test_blocks_follow_the_oracle_twin(vmc, oracle, n_up, n_dn):
+    N = n_up + n_dn
+    L = vmc.box_length_from_rs(2.0, N)
+    s = vmc.System(n_up, n_dn, L, 0.25, 0.5, 1.0, 5.0 / L, 25, 0.5 * L, vmc.ERFC_EXACT, vmc.MOVE_GAUSSIAN,
+                   vmc.PREC_FP64, 0)
+    W, seed, step = 2, 700 + N, 0.8
+    ens = vmc.Ensemble(s, W, seed, step0=step)
+    assert ens.kernel() == vmc.KERNEL_DELAYED
+    ens.init_positions()
+    osys = oracle_system(oracle, s)
+    walkers = [oracle.Walker(osys, oracle.init_positions(osys, seed, w)[0]) for w in range(W)]
+    sweeps = 3 if N < 130 else 1
+    total = np.zeros(W)
+    for sweep in range(sweeps):
+        ens.sweep(1, measure=True, adapt=False)
+        st, pos = ens.stats(), ens.positions()
+        for w in range(W):
+            acc, _, e = walkers[w].sweep(seed, w, sweep, step, move_kind=s.move_kind, adapt=False, measure=True)
+            total[w] += acc
+            np.testing.assert_allclose(pos[w], walkers[w].positions(), rtol=0, atol=1e-12 * L)
+            assert st[w, vmc.STAT["ACCEPTED"]] == total[w]
+            assert abs(st[w, vmc.STAT["LAST_E"]] - e) <= 1e-9 * max(abs(e), 1e-3 * N), (w, sweep)
+    ens.close()
+
+
+def test_several_sweeps_in_one_launch_are_those_of_single_launches(vmc):
+    """Unmeasured sweeps share a launch: the same chain, bit for bit, as one
+    launch per sweep, step adaptation included."""
+    L = vmc.box_length_from_rs(3.0, 26)
+    s = vmc.System(19, 7, L, 0.25, 0.5, 1.0, 5.0 / L, 25, 0.5 * L, vmc.ERFC_EXACT, vmc.MOVE_GAUSSIAN,
+                   vmc.PREC_FP64, 0)
+    out = []
+    for calls, n in ((1, 5), (5, 1)):
+        e = vmc.Ensemble(s, 67, 9, step0=0.7)
+        e.init_positions()
+        for _ in range(calls):
+            e.sweep(n, adapt=True)
+        out.append((e.positions(), e.stats(), e.steps(), e.inverse()))
+        e.close()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)

@@ -30,6 +30,7 @@ struct DevSys {
     int inv_off[2];  // offset of the determinant's inverse in a walker's block
     int ninv;        // n[0]^2 + n[1]^2
     int nmax;
+    int kmax;        // largest component of an orbital's n vector
     int ng;
     int erfc_kind;   // 0 = Abramowitz-Stegun 7.1.26, 1 = erfc
     int move_kind;   // 0 = uniform cube, 1 = Gaussian

@@ -1,30 +1,45 @@
-// vmc_sweep_du.hip -- FP64 sweep with delayed (Woodbury) inverse updates for
-// determinants of up to 160 electrons, the FP64 sizes above the
-// register-resident kernels (123 and 147 electrons per spin among them).
+// vmc_sweep_du.hip -- FP64 sweep with delayed (Woodbury) inverse updates, a
+// block of up to 32 moves per determinant at a time.
 //
-// One 256-thread workgroup per walker.  The transposed inverse invT_0 of each
-// determinant stays in the walker's HBM block and changes only at a flush.
-// Between flushes the accepted moves of a determinant form a window of at
-// most KD entries: the row change delta_a = phi(r'_a) - phi(r_a) of mover
-// p_a and a copy P_a of the row invT_0[p_a], both in LDS.  With
-// C[a][b] = [a == b] + delta_a . P_b, Woodbury gives the current inverse
-//   invT[k][j] = invT_0[k][j] - sum_ab P_a[j] Cinv[a][b] (delta_b . invT_0[k])
-// (the reference's rank-1 update, slater_plane_wave.cpp:367-423, applied KD
-// at a time).  A move of electron q needs only row q.  With Q = invT_0[q],
-//   R = phi'.Q - sum_ab (phi'.P_a) Cinv[a][b] (delta_b . Q)
-// (the ratio of slater_plane_wave.cpp:351-365), so each move forms one 16 x 16
-// block of dot products on the FP64 matrix cores -- rows phi', phi(r_q),
-// delta_0..; columns Q, P_0.. -- and an accepted move borders Cinv with its
-// Schur complement.  A flush applies the window to invT_0 on the matrix
-// cores, 16 rows of invT_0 per step:
-//   Z = -(Cinv Delta) invT_0[rows]^T, then invT_0[rows] += Z^T P,
-// each row read once and written once.  Per proposed move the kernel reads
-// one row of invT_0 from memory instead of updating all n rows per accepted
-// move; the n^2 update is paid once per KD accepted moves, as matrix products.
+// One workgroup per walker; the transposed inverse invT of each determinant
+// stays in the walker's HBM block.  Every proposal of a sweep is known before
+// the sweep starts (each electron moves once), so a block of consecutive
+// movers is prepared as matrix work and decided afterwards:
+//   - T[k][q] = phi'_q . invT[k] for the block's movers q and their inverse
+//     rows k, on the FP64 matrix cores.  The ratio of the first move is T[0][0];
+//     each accepted move a updates the block's rows by
+//       T[k] -= (T[k][a] / R_a) T[a],  T[a] /= R_a,
+//     the row operations of Sherman-Morrison (slater_plane_wave.cpp:367-423)
+//     on the 32 columns that later moves of the block read, so R_q = T[q][q]
+//     (slater_plane_wave.cpp:351-365) when q's turn comes.  One wavefront holds
+//     T in registers, one row per lane, both determinants in its two halves,
+//     and the dead column of each mover collects the row operations
+//     themselves: after the block it holds Cinv of the accepted movers.
+//   - The Jastrow change of every mover against the block's starting
+//     positions, by all wavefronts, and for each pair of movers (p, a) the
+//     correction X[a][p] that p's change takes when a is accepted first.
+//   - The chain of decisions is then a wavefront's: two lane reads, the accept
+//     test, one row of X, one row broadcast and 31 FMAs per pair of moves.
+//   - A flush applies the m <= 16 accepted moves to all n rows of invT on the
+//     matrix cores, 16 rows per wavefront at a time:
+//       Z = Phi'_acc invT[rows]^T - E, Y = Cinv Z, invT[rows] -= Y^T P_acc,
+//     each row read once and written once (E: unit entries at the movers' own
+//     rows; P_acc: the accepted movers' old rows, copied to LDS first).
+// A block ends early when 16 moves are accepted in one determinant or when
+// the product of its accepted ratios exceeds 16 (kDuGrowth).
+//
+// What bounds it (N = 294, 1024 walkers, 1.70 ms a sweep): FP64 VALU work (43 %
+// of the cycles, the pair terms above all) and FP64 MFMA issue (24 %) of two
+// resident workgroups; alone on its CU a walker takes 0.51 ms, of which the
+// decisions are a fifth, the flushes a third and T beside the pair terms 30 %.
+// Against one inverse row read, five barriers and an 8-entry window solved by
+// serial lane reads per move: 7.84 -> 1.70 ms a sweep at N = 294 and 3.88 -> 1.14
+// at N = 246 (1024 walkers), 0.46 -> 0.07 ms at 19 + 7 electrons (777 walkers,
+// against the generic kernel), 138 -> 3.5 ms at 485 (8 walkers, the same).
 //
 // The chain is the generic kernel's (vmc_hip.hip sweep_walker): the same
-// Philox draws, sweep order, FP64 accept test and Jastrow bookkeeping, so the
-// FP64 trajectory follows the oracle twin move for move.
+// Philox draws, sweep order and FP64 accept test, so the FP64 trajectory
+// follows the oracle twin move for move.
 #include "../../include/vmc_hip.h"
 #include "vmc_device.hpp"
 #include "vmc_rr_launch.hpp"
@@ -35,33 +50,54 @@
 namespace vmc {
 
 typedef double du_v4d __attribute__((ext_vector_type(4)));
+// Four consecutive doubles at an 8-byte boundary (rows of odd length).
+typedef double du_v4u __attribute__((ext_vector_type(4), aligned(8)));
 
-constexpr int kDuThreads = 256;
-constexpr int kDuWaves = kDuThreads / kWave;
-constexpr int kDuWindow = 8;  // accepted moves per determinant between flushes
-// A window is also applied once the product of its Schur complements (the
-// determinant's growth since the last flush) exceeds kDuGrowth: the flush then
-// forms a small inverse as the difference of larger terms, and its rounding
-// grows with that ratio (walkers leaving a near-singular start accept ratios
-// of 5 to 12; in equilibrium this adds about 3 % to the flushes).
-constexpr double kDuGrowth = 4.0;
+constexpr int kG = 8;  // decisions per unrolled group
+constexpr int kDuMaxAcc = 16;  // accepted moves per determinant between flushes: one MFMA tile
+// A flush forms invT as the difference of terms that grow with the product of
+// the accepted ratios since the last one (the determinant's growth); walkers
+// leaving a near-singular start accept ratios of 5 to 12.  In 1/256 of log2:
+// the block ends above a growth of 16.
+constexpr int kDuGrowth = 4 * 256;
 
-// P: row length padded to a multiple of 16 (n <= P); at most 2P electrons.
-template <int P, int KD>
-struct DuShared {
-    static constexpr int NE = 2 * P;
-    double px[NE], py[NE], pz[NE], U[NE], uj[NE];
-    double draw[4][NE];                  // proposal (dx, dy, dz) and accept uniform per electron
-    alignas(16) double phin[P];          // orbital row at the proposal
-    alignas(16) double phio[P];          // orbital row at the mover's position
-    alignas(16) double qrow[P];          // invT_0 row of the mover
-    alignas(16) double delta[2][KD][P];  // window row changes (a flush overwrites them)
-    alignas(16) double prow[2][KD][P];   // window copies of invT_0 rows
-    double cinv[2][16][16];              // inverse of the window's C, per determinant
-    double gpart[kDuWaves][48];          // per-wave G rows 0, 1 and column 0
-    double jpart[kDuWaves];
-    double dec[4];                       // decision, ratio, new Jastrow row sum, Schur complement
+// Dynamic LDS of a walker, in doubles from its start.  TH > 0: rows of up to
+// 16 TH columns (n > 16 (TH - 2)), so every offset but those of the arrays
+// over electrons and orbitals is a constant.
+template <int NB, int TH, bool kTwo, int NW>
+struct DuLds {
+    static constexpr int ND = kTwo ? 2 : 1;
+    static constexpr int kSlots = kTwo ? 64 : 32;  // movers of a block
+    static constexpr int NB16 = (NB + 15) / 16 * 16;
+    // Powers 0 .. K1 - 1 of an axis phasor: the largest component of the
+    // orbitals is 1 up to 16 per spin, 2 up to 64, 3 up to 160 and 5 up to 512.
+    static constexpr int K1 = TH == 0 ? 6 : TH <= 1 ? 2 : TH <= 4 ? 3 : 4;
+    static constexpr int prop = 0;
+    static constexpr int cinv = prop + 4 * kSlots;
+    static constexpr int ctl = cinv + 2 * kDuMaxAcc * (kDuMaxAcc + 1);  // 48 ints
+    static constexpr int book = ctl + 24;
+    static constexpr int pw = book + 6;
+    // Phi' and P of the flush, or X, T and the wavefronts' Jastrow sums of the
+    // block's decisions.
+    static constexpr int big = pw + 3 * K1 * kSlots * 2;
+    static constexpr int part = big + ND * NB * kSlots + ND * NB16 * 32;
+    static constexpr int kBlock = part - big + (kTwo ? NW : 2 * NW) * kSlots;
+    int pitch;  // LDS row pitch (16-byte steps, rows spread over the banks)
+    int px, orb, total;
+    __host__ __device__ DuLds(int N, int n, int norb) {
+        pitch = TH > 0 ? 16 * TH + 2 : (n + 15) / 16 * 16 + 2;
+        const int flush = 2 * kDuMaxAcc * pitch;
+        px = big + (flush > kBlock ? flush : kBlock);
+        orb = px + 3 * ((N + 1) & ~1);
+        total = orb + (norb + 1) / 2;
+    }
 };
+
+// book: step width, log|det| of both determinants, accepted moves of the launch
+// and of the sweep, accepted moves since the last re-inversion (kept here, not
+// in registers through every phase).
+// ctl ints: [0..1] accepted masks, [2] moves decided, [4 + 16 h + i] slot (row
+// in the block) of determinant h's i-th accepted mover.
 
 __device__ __forceinline__ double du_readlane(double v, int l) {
     union { double d; int i[2]; } u;
@@ -71,362 +107,726 @@ __device__ __forceinline__ double du_readlane(double v, int l) {
     return u.d;
 }
 
-// Applies the m-entry window of determinant h to its inverse inv (n x n, row
-// k = invT_0[k][.]) and leaves the window empty.  Called by every thread.
-template <int P, int KD>
-__device__ void du_flush(DuShared<P, KD> &sh, double *inv, int n, int h, int m) {
-    const int t = threadIdx.x, wave = t >> 6, lane = t & (kWave - 1);
-    // delta_a <- -(Cinv Delta)_a in place, each thread one column j (rows a >= m
-    // become zero).
-    if (t < P) {
-        double d[KD];
+// The thread index as a value of its own in each phase, so that a phase's
+// addresses are formed there and not carried in registers through the others.
+__device__ __forceinline__ int du_thread() {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
+// LDS traffic between lanes of one wavefront: the LDS serves a wavefront's
+// accesses in order, so only the compiler has to keep them in order.
+__device__ __forceinline__ void du_wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Metropolis test u < R^2 exp(2 dJ) (simulation.cpp:125-131) of every lane's
+// values, as lane masks: `yes`, and `near` where the hardware exp2 does not
+// decide it (u within 1e-5 of the threshold, or |dJ| beyond its range) and the
+// FP64 exp has to.
+__device__ __forceinline__ void du_test(double R, double dj, double ua, unsigned long long &yes,
+                                        unsigned long long &near) {
+    const double approx = R * R * (double)__builtin_amdgcn_exp2f((float)(2.0 * dj * 1.4426950408889634));
+    yes = __ballot(ua < approx);
+    near = __ballot(!(fabs(ua - approx) > 1e-5 * approx) || !(fabs(dj) < 40.0));
+}
+// Bit `l` of the test's outcome.
+__device__ __forceinline__ int du_decide(double R, double dj, double ua, int l) {
+    unsigned long long yes, near;
+    du_test(R, dj, ua, yes, near);
+    if ((near >> l) & 1ull) yes = __ballot(ua < R * R * exp(2.0 * dj));
+    return (int)((yes >> l) & 1ull);
+}
+
+// log2 |R| of lane l in 1/256, from the exponent and the leading mantissa bits
+// (at most 0.09 low).
+__device__ __forceinline__ int du_log2(double R, int l) {
+    return ((__builtin_amdgcn_readlane(__double2hiint(R), l) & 0x7fffffff) >> 12) - (1023 << 8);
+}
+
+// Factor of the mover's row in a row's update: the row's entry in the mover's
+// column over R, and 1 - 1/R for the mover's own row.  Both sides are formed
+// (a branch costs more).
+__device__ __forceinline__ double du_factor(bool pivot, double t, double ir) {
+    double own = 1.0 - ir, other = t * ir;
+    asm volatile("" : "+v"(own), "+v"(other));
+    return pivot ? own : other;
+}
+
+// T[q] -= f T_l[q] for every column, T_l the row of lane l (lane reads into
+// scalar registers: no LDS round trip on the chain).
+template <int NB>
+__device__ __forceinline__ void du_row_op(double (&T)[NB], double f, int l) {
 #pragma unroll
-        for (int i = 0; i < KD; ++i) d[i] = i < m ? sh.delta[h][i][t] : 0.0;
+    for (int q0 = 0; q0 < NB; q0 += 8) {
+        // (eight lane reads, then their uses: a use right behind its read waits)
+        double v[8];
 #pragma unroll
-        for (int a = 0; a < KD; ++a) {
-            double acc = 0.0;
+        for (int q = 0; q < 8; ++q) v[q] = du_readlane(T[q0 + q], l);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < KD; ++i)
-                if (a < m && i < m) acc += sh.cinv[h][a][i] * d[i];
-            sh.delta[h][a][t] = -acc;
+        for (int q = 0; q < 8; ++q) T[q0 + q] = fma(-f, v[q], T[q0 + q]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// Orbital o (packed, du_pack) of the mover in `slot` from the axis powers.
+__device__ __forceinline__ int du_pack(int4 o) {
+    const int y = o.y < 0 ? -o.y : o.y, z = o.z < 0 ? -o.z : o.z;
+    return o.x | (y << 8) | (z << 16) | (o.y < 0 ? 1 << 24 : 0) | (o.z < 0 ? 1 << 25 : 0) | (o.w ? 1 << 26 : 0);
+}
+template <int kSlots, int K1>
+__device__ __forceinline__ double du_orbital(const double2 *pw, int slot, int o) {
+    const double2 X = pw[(o & 255) * kSlots + slot];
+    double2 Y = pw[(K1 + ((o >> 8) & 255)) * kSlots + slot];
+    double2 Z = pw[(2 * K1 + ((o >> 16) & 255)) * kSlots + slot];
+    Y.y = (o & (1 << 24)) ? -Y.y : Y.y;
+    Z.y = (o & (1 << 25)) ? -Z.y : Z.y;
+    const double re = X.x * Y.x - X.y * Y.y, im = X.x * Y.y + X.y * Y.x;
+    return (o & (1 << 26)) ? re * Z.y + im * Z.x : re * Z.x - im * Z.y;
+}
+
+// Length of the minimum image of a separation in units of L: sqrt(x) from
+// v_rsq_f64 (2^-24 relative) y and one third-order step: with h = x y and
+// e = 1 - h y, sqrt(x) = h (1 + e/2 + 3/8 e^2) to e^3 = 2^-70.
+__device__ __forceinline__ double du_dist(double dx, double dy, double dz) {
+    dx -= rint(dx);
+    dy -= rint(dy);
+    dz -= rint(dz);
+    const double x = fmax(fma(dz, dz, fma(dy, dy, dx * dx)), 1e-280);
+    const double y = __builtin_amdgcn_rsq(x), h = x * y, e = fma(-h, y, 1.0);
+    return fma(h * e, fma(e, 0.375, 0.5), h);
+}
+
+// (u(rn) - u(ro)) / (a L) of the Pade pair function r / (1 + b r), distances in
+// units of L and bl = b L: over the common denominator (one reciprocal, from
+// v_rcp_f64 and a third-order step, and no cancellation).
+__device__ __forceinline__ double du_pade_diff(double rn, double ro, double bl) {
+    const double d = fma(bl, rn, 1.0) * fma(bl, ro, 1.0);
+    const double y = __builtin_amdgcn_rcp(d), e = fma(-d, y, 1.0);
+    return (rn - ro) * fma(y, fma(e, e, e), y);
+}
+
+// This sweep's proposals of the block's movers (vmc_hip.hip sweep_walker):
+// Philox tags MOVE and ACCP, counter {electron, walker, sweep}; or the
+// caller's moves.  One wavefront, one lane per mover.
+template <bool kTwo>
+__device__ __forceinline__ void du_propose(const DevSys &s, double *prop, const double *gp, const SweepGiven &given, int w,
+                           uint32_t sweep, double sigma, int hb, int q0, int cnt, int lane) {
+    asm volatile("" : "+v"(lane));
+    const int r = lane & 31, h = kTwo ? lane >> 5 : hb;
+    if (r >= cnt || (!kTwo && lane >= 32)) return;
+    const int e = s.first[h] + q0 + r, slot = kTwo ? lane : r;
+    constexpr int kSlots = kTwo ? 64 : 32;
+    if (given.prop) {
+        const size_t g = (size_t)w * s.N + e;
+        for (int c = 0; c < 3; ++c) prop[c * kSlots + slot] = given.prop[3 * g + c];
+        prop[3 * kSlots + slot] = given.u[g];
+        return;
+    }
+    const uint4 rm = philox4x32_10(make_uint4((uint32_t)e, (uint32_t)w, sweep, kTagMove), s.key0, s.key1);
+    const uint4 ra = philox4x32_10(make_uint4((uint32_t)e, (uint32_t)w, sweep, kTagAccept), s.key0, s.key1);
+    double d[3];
+    if (s.move_kind == 1) {
+        const double rho0 = sqrt(-2.0 * log(u01(rm.x)));
+        const double rho1 = sqrt(-2.0 * log(u01(rm.z)));
+        double s0, c0, s1, c1;
+        sincospi(2.0 * u01(rm.y), &s0, &c0);
+        sincospi(2.0 * u01(rm.w), &s1, &c1);
+        d[0] = rho0 * c0;
+        d[1] = rho0 * s0;
+        d[2] = rho1 * c1;
+    } else {
+        d[0] = 2.0 * u01(rm.x) - 1.0;
+        d[1] = 2.0 * u01(rm.y) - 1.0;
+        d[2] = 2.0 * u01(rm.z) - 1.0;
+    }
+    for (int c = 0; c < 3; ++c) {
+        const double x = gp[c * s.N + e] + sigma * d[c];
+        prop[c * kSlots + slot] = x - s.L * floor(x * s.inv_L);
+    }
+    prop[3 * kSlots + slot] = u01(ra.x);
+}
+
+// Applies determinant h's m accepted moves to its inverse inv (n x n, row k =
+// invT[k][.]).  TH: 16-column tiles of a row tile held in registers between
+// its read and its write; 0 reads the row tile twice (n > 160).  Called by
+// every thread.
+template <int NB, int TH, bool kTwo, int NW>
+__device__ __forceinline__ void du_flush(const DuLds<NB, TH, kTwo, NW> &l, double *sm, double *inv, int n, int h,
+                                         int q0, int m, const int *orb) {
+    using Lay = DuLds<NB, TH, kTwo, NW>;
+    const int t = du_thread(), wave = wave_uniform(t >> 6), lane = t & (kWave - 1);
+    const int *list = reinterpret_cast<const int *>(sm + Lay::ctl) + 4 + 16 * h;
+    const double2 *pw = reinterpret_cast<const double2 *>(sm + Lay::pw);
+    double *phi = sm + Lay::big, *prow = phi + kDuMaxAcc * l.pitch;
+    const int r = lane & 15, g = lane >> 4;
+    const int T = TH > 0 ? TH : (n + 15) / 16, TF = n / 16;  // column tiles, whole ones
+    const int R = (n + 15) / 16;                               // row tiles
+    const auto load = [&](const double *row, int jt) {
+        du_v4d c = {0.0, 0.0, 0.0, 0.0};
+        if (jt < TH - 2 || jt < TF) {
+            const du_v4u u = *reinterpret_cast<const du_v4u *>(row + 16 * jt);
+            c = u;
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (16 * jt + 4 * g + q < n) c[q] = row[16 * jt + q];
+        }
+        return c;
+    };
+    const auto row_of = [&](int kt) {
+        const int k = 16 * kt + r;
+        return inv + (size_t)(k < n ? k : n - 1) * n + 4 * g;
+    };
+    // The first row tile is on its way while the movers' rows are gathered.
+    constexpr int TR = TH > 0 ? TH : 1;
+    du_v4d c[TR];
+    if (TH > 0 && wave < R) {
+        const double *row = row_of(wave);
+#pragma unroll
+        for (int jt = 0; jt < TR; ++jt) c[jt] = load(row, jt);
+    }
+    // The accepted movers' new orbital rows and old inverse rows (rows past m
+    // and columns past n keep finite values that meet zeros).
+    for (int a = wave; a < m; a += NW) {
+        const int rs = list[a], slot = kTwo ? h * 32 + rs : rs;
+        const double *src = inv + (size_t)(q0 + rs) * n;
+        for (int j = lane; j < l.pitch - 2; j += kWave) {
+            const bool in = j < n;
+            prow[a * l.pitch + j] = in ? src[j] : 0.0;
+            phi[a * l.pitch + j] = in ? du_orbital<Lay::kSlots, Lay::K1>(pw, slot, orb[j]) : 0.0;
         }
     }
     __syncthreads();
-    // Row tiles of 16 rows per wave: Z = -(Cinv Delta) invT_0[rows]^T on the
-    // matrix cores, then invT_0[rows] += Z^T P.  The output registers of the
-    // first product are the A operands of the second (register q of lane l
-    // holds Z[4q + (l >> 4)][k0 + (l & 15)]).
-    const int r = lane & 15, g = lane >> 4;
-    constexpr int T = P / 16;
-    constexpr int SJ = P / 4;
-    const double *arow = sh.delta[h][r < KD ? r : 0];
-    for (int kt = wave; kt < T; kt += kDuWaves) {
-        const int k0 = 16 * kt;
-        const int kr = k0 + r < n ? k0 + r : n - 1;
-        const double *brow = inv + (size_t)kr * n;
-        du_v4d z = {0.0, 0.0, 0.0, 0.0};
-        const int jb = g * SJ;
-#pragma unroll 4
-        for (int s = 0; s < SJ; ++s) {
-            const int j = jb + s;
-            const double a = r < KD ? arow[j] : 0.0;
-            const double b = brow[j < n ? j : n - 1];
-            z = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, z, 0, 0, 0);
-        }
-        for (int jt = 0; jt < T; ++jt) {
-            const int jj = 16 * jt + r;
-            du_v4d c;
+    const double *cinv = sm + Lay::cinv + h * kDuMaxAcc * (kDuMaxAcc + 1);
+    const double *phr = phi + r * l.pitch + 4 * g;
+    // Column 16 jt + 4 (r & 3) + (r >> 2) is what output row r of the update
+    // stands for: register q of group g then holds column 16 jt + 4 g + q, so
+    // a lane's four values are consecutive in memory.
+    const double *pr = prow + g * l.pitch + 4 * (r & 3) + (r >> 2);
+    int own[4];  // the row of mover 4 q + g, where Z loses 1
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int k = k0 + 4 * q + g;
-                c[q] = (k < n && jj < n) ? inv[(size_t)k * n + jj] : 0.0;
+    for (int q = 0; q < 4; ++q) own[q] = 4 * q + g < m ? q0 + list[4 * q + g] : -1;
+    for (int kt = wave; kt < R; kt += NW) {
+        const int k = 16 * kt + r;
+        double *row = row_of(kt);
+        du_v4d z = {0.0, 0.0, 0.0, 0.0}, y = {0.0, 0.0, 0.0, 0.0};
+        const auto store = [&](int jt, const du_v4d &c) {
+            if (k >= n) return;
+            if (jt < TH - 2 || jt < TF) {
+                *reinterpret_cast<du_v4u *>(row + 16 * jt) = c;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (16 * jt + 4 * g + q < n) row[16 * jt + q] = c[q];
+            }
+        };
+        const auto dot = [&](int jt, const du_v4d &c) {
+            const du_v4d a = *reinterpret_cast<const du_v4u *>(phr + 16 * jt);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) z = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], c[q], z, 0, 0, 0);
+        };
+        const auto update = [&](int jt, du_v4d &c) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                c = __builtin_amdgcn_mfma_f64_16x16x4f64(pr[4 * q * l.pitch + 16 * jt], y[q], c, 0, 0, 0);
+        };
+        const auto solve = [&]() {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) z[q] = own[q] == k ? z[q] - 1.0 : z[q];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                y = __builtin_amdgcn_mfma_f64_16x16x4f64(cinv[r * (kDuMaxAcc + 1) + 4 * q + g], z[q], y, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[q] = -y[q];
+        };
+        if constexpr (TH > 0) {
+#pragma unroll
+            for (int jt = 0; jt < TH; ++jt) {
+                dot(jt, c[jt]);
+                if (jt % 2) __builtin_amdgcn_sched_barrier(0);
+            }
+            solve();
+#pragma unroll
+            for (int jt = 0; jt < TH; ++jt) {
+                update(jt, c[jt]);
+                if (jt % 2) __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
-            for (int s = 0; s < (KD + 3) / 4; ++s) {
-                const int a = 4 * s + g;
-                const double b = sh.prow[h][a < KD ? a : 0][jj];
-                c = __builtin_amdgcn_mfma_f64_16x16x4f64(z[s], b, c, 0, 0, 0);
-            }
+            for (int jt = 0; jt < TH; ++jt) store(jt, c[jt]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (kt + NW < R) {
+                const double *next = row_of(kt + NW);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int k = k0 + 4 * q + g;
-                if (k < n && jj < n) inv[(size_t)k * n + jj] = c[q];
+                for (int jt = 0; jt < TH; ++jt) c[jt] = load(next, jt);
+            }
+        } else {
+            // The next column tile is on its way while this one is used.
+            du_v4d cc = load(row, 0);
+#pragma unroll 1
+            for (int jt = 0; jt < T; ++jt) {
+                const du_v4d nx = load(row, jt + 1 < T ? jt + 1 : jt);
+                dot(jt, cc);
+                cc = nx;
+            }
+            solve();
+            cc = load(row, 0);
+#pragma unroll 1
+            for (int jt = 0; jt < T; ++jt) {
+                const du_v4d nx = load(row, jt + 1 < T ? jt + 1 : jt);
+                update(jt, cc);
+                store(jt, cc);
+                cc = nx;
             }
         }
     }
     __syncthreads();
 }
 
-template <int P, int KD>
+// kTwo: equal spins, the block's movers are up q0.., down q0.. in turn; else
+// the block's movers are of one determinant.
+template <int NB, int TH, bool kTwo, int NW>
 __device__ void du_sweep_walker(const DevSys &s, const DevState &st, int w, int n_sweeps,
                                 unsigned long long sweep0, int flags, const SweepGiven &given) {
-    __shared__ DuShared<P, KD> sh;
-    const int t = threadIdx.x, wave = t >> 6, lane = t & (kWave - 1);
-    const int N = s.N;
+    extern __shared__ __align__(16) double sm[];
+    constexpr int NT = NW * kWave;
+    constexpr int kSlots = kTwo ? 64 : 32;
+    constexpr int ND = kTwo ? 2 : 1;
+    constexpr int NB16 = (NB + 15) / 16 * 16;
+    constexpr int kSub = kTwo ? NW : 2 * NW;  // subsets of the electrons in the pair sums
+    const int t = threadIdx.x, wave = wave_uniform(t >> 6), lane = t & (kWave - 1);
+    const int N = s.N, NP = (N + 1) & ~1;
+    const int norb = kTwo ? s.nmax : s.n[0] + (s.ndet == 2 ? s.n[1] : 0);
+    using Lay = DuLds<NB, TH, kTwo, NW>;
+    const Lay l(N, s.nmax, norb);
+    double *px = sm + l.px, *py = px + NP, *pz = py + NP;
+    double *prop = sm + Lay::prop;
+    double *X = sm + Lay::big;                        // [ND NB][kSlots]
+    double *Ts = X + ND * NB * kSlots;             // [ND][NB16][32]
+    double2 *pw = reinterpret_cast<double2 *>(sm + Lay::pw);
+    double *part = sm + Lay::part;
+    int *orbs = reinterpret_cast<int *>(sm + l.orb);
+    int *ctl = reinterpret_cast<int *>(sm + Lay::ctl);
     double *invw = reinterpret_cast<double *>(st.inv) + (size_t)w * s.ninv;
     double *gp = st.pos + (size_t)w * 3 * N;
-    WalkerView<double> v{};
-    v.inv = invw;
-    v.px = sh.px;
-    v.py = sh.py;
-    v.pz = sh.pz;
-    v.U = sh.U;
-    v.uj = sh.uj;
-    for (int j = t; j < P; j += kDuThreads) {
-        sh.phin[j] = 0.0;
-        sh.phio[j] = 0.0;
-        sh.qrow[j] = 0.0;
-    }
-    for (int e = t; e < 2 * KD * P; e += kDuThreads) {
-        (&sh.delta[0][0][0])[e] = 0.0;
-        (&sh.prow[0][0][0])[e] = 0.0;
-    }
-    for (int i = t; i < N; i += kDuThreads) {
-        sh.px[i] = gp[i];
-        sh.py[i] = gp[N + i];
-        sh.pz[i] = gp[2 * N + i];
+    for (int i = t; i < l.orb; i += NT) sm[i] = 0.0;
+    for (int j = t; j < norb; j += NT) {
+        const int d = !kTwo && j >= s.n[0] ? 1 : 0;
+        orbs[j] = du_pack(s.orb[d * s.nmax + (d ? j - s.n[0] : j)]);
     }
     __syncthreads();
-    jastrow_rows<double>(s, v, t);
-
-    double *ws = st.stats + (size_t)w * kStatCount;
-    double stat[kStatCount];
-#pragma unroll
-    for (int k = 0; k < kStatCount; ++k) stat[k] = ws[k];
-    double sigma = st.sigma[w];
-    int since = st.since[w];
-    if (s.reinv_k > 0 && since >= s.reinv_k) since = 0;  // re-inverted after the last sweep
-    double ld0 = st.logdet[2 * w + 0], ld1 = st.logdet[2 * w + 1];
-    const double b = s.b;
+    for (int i = t; i < N; i += NT) {
+        px[i] = gp[i] * s.inv_L;
+        py[i] = gp[N + i] * s.inv_L;
+        pz[i] = gp[2 * N + i] * s.inv_L;
+    }
+    double *book = sm + Lay::book;
+    if (t == 0) {
+        const int since = st.since[w];
+        book[0] = st.sigma[w];
+        book[1] = st.logdet[2 * w + 0];
+        book[2] = st.logdet[2 * w + 1];
+        book[3] = 0.0;
+        book[4] = 0.0;
+        book[5] = s.reinv_k > 0 && since >= s.reinv_k ? 0.0 : (double)since;  // re-inverted after the last sweep
+    }
+    __syncthreads();
 
     for (int sw = 0; sw < n_sweeps; ++sw) {
         const uint32_t sweep = (uint32_t)(sweep0 + (unsigned long long)sw);
-        // This sweep's draws (vmc_hip.hip sweep_walker): Philox tag MOVE and
-        // ACCP, counter {electron, walker, sweep}; or the caller's moves.
-        for (int q = t; q < N; q += kDuThreads) {
-            if (given.prop) {
-                const size_t g = (size_t)w * N + q;
-                sh.draw[0][q] = given.prop[3 * g];
-                sh.draw[1][q] = given.prop[3 * g + 1];
-                sh.draw[2][q] = given.prop[3 * g + 2];
-                sh.draw[3][q] = given.u[g];
-                continue;
+        for (int hb = 0; hb < (kTwo ? 1 : s.ndet); ++hb) {
+            const int n = s.n[hb];
+            if (wave == NW - 1) du_propose<kTwo>(s, prop, gp, given, w, sweep, book[0], hb, 0, n < NB ? n : NB, lane);
+            __syncthreads();
+            int cnt = 0;
+            for (int q0 = 0; q0 < n;) {
+                cnt = n - q0 < NB ? n - q0 : NB;
+                // Axis phasor powers of the block's proposals.
+                for (int i = du_thread(); i < 3 * kSlots; i += NT) {
+                    const int ax = i / kSlots, slot = i - ax * kSlots;
+                    if ((slot & 31) >= cnt) continue;
+                    double f = prop[ax * kSlots + slot] * s.inv_L;
+                    f -= rint(f);
+                    double sn, cs;
+                    sincos_2pi<double>(f, &sn, &cs);
+                    double2 p = make_double2(1.0, 0.0);
+                    for (int k = 0; k < Lay::K1; ++k) {
+                        pw[(ax * Lay::K1 + k) * kSlots + slot] = p;
+                        p = make_double2(p.x * cs - p.y * sn, p.x * sn + p.y * cs);
+                    }
+                }
+                __syncthreads();
+                // T of the block on the first ND MT wavefronts, 16 movers
+                // each; the other wavefronts start with the pair terms, of
+                // which these take a share that evens the two (a column tile
+                // of T costs about 1.4 electrons' pair terms).
+                constexpr int MT = NB16 / 16, NTask = ND * MT;
+                {
+                    const int t = du_thread(), wave = wave_uniform(t >> 6), lane = t & (kWave - 1);
+                    const int r = lane & 15, g = lane >> 4;
+                    const int P16 = (n + 15) / 16;
+                    for (int task = wave; task < NTask; task += NW) {
+                        const int h = task / MT, mt = task % MT;
+                        if (16 * mt >= cnt) continue;
+                        const int hd = kTwo ? h : hb;
+                        const int slot = (kTwo ? h * 32 : 0) + 16 * mt + r;
+                        const int *orb = orbs + (!kTwo && hb ? s.n[0] : 0) + 4 * g;
+                        const double *row[MT];
+#pragma unroll
+                        for (int kt = 0; kt < MT; ++kt) {
+                            const int k = q0 + 16 * kt + r;
+                            row[kt] = invw + s.inv_off[hd] + (size_t)(k < n ? k : n - 1) * n + 4 * g;
+                        }
+                        const auto load = [&](int kt, int jt) {
+                            du_v4d c;
+                            if (16 * jt + 16 <= n) {
+                                const du_v4u u = *reinterpret_cast<const du_v4u *>(row[kt] + 16 * jt);
+                                c = u;
+                            } else {
+#pragma unroll
+                                for (int q = 0; q < 4; ++q)
+                                    c[q] = 16 * jt + 4 * g + q < n ? row[kt][16 * jt + q] : 0.0;
+                            }
+                            return c;
+                        };
+                        du_v4d z[MT], c0[MT], c1[MT];
+#pragma unroll
+                        for (int kt = 0; kt < MT; ++kt) {
+                            z[kt] = du_v4d{0.0, 0.0, 0.0, 0.0};
+                            c0[kt] = load(kt, 0);
+                            c1[kt] = load(kt, P16 > 1 ? 1 : 0);
+                        }
+                        const auto orbitals = [&](int jt, double (&av)[4]) {
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                const int j = 16 * jt + 4 * g + q;
+                                av[q] = du_orbital<kSlots, Lay::K1>(pw, slot, orb[j < n ? 16 * jt + q : -4 * g]);
+                            }
+                        };
+                        double av[4];
+                        orbitals(0, av);
+#pragma unroll 1
+                        for (int jt = 0; jt < P16; ++jt) {
+                            double an[4];
+                            orbitals(jt + 1 < P16 ? jt + 1 : jt, an);
+#pragma unroll
+                            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                                for (int kt = 0; kt < MT; ++kt)
+                                    z[kt] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[q], c0[kt][q], z[kt], 0, 0, 0);
+#pragma unroll
+                            for (int kt = 0; kt < MT; ++kt) {
+                                c0[kt] = c1[kt];
+                                c1[kt] = load(kt, jt + 2 < P16 ? jt + 2 : P16 - 1);
+                            }
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) av[q] = an[q];
+                        }
+#pragma unroll
+                        for (int kt = 0; kt < MT; ++kt)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q)
+                                Ts[(h * NB16 + 16 * mt + 4 * q + g) * 32 + 16 * kt + r] = z[kt][q];
+                    }
+                }
+                // Jastrow change of the lane's mover against the electrons of
+                // the wavefront's share, at the block's starting positions,
+                // and the corrections by the movers among them.
+                {
+                    const int t = du_thread(), wave = wave_uniform(t >> 6), lane = t & (kWave - 1);
+                    const double inv_L = s.inv_L, bl = s.b * s.L;
+                    const int r = lane & 31, slot = kTwo ? lane : r;
+                    const int h = kTwo ? lane >> 5 : hb;
+                    const int half = kTwo ? 0 : lane >> 5;
+                    const int e = s.first[h] + q0 + (r < cnt ? r : 0);
+                    const double xo = px[e], yo = py[e], zo = pz[e];
+                    const double xn = prop[slot] * inv_L, yn = prop[kSlots + slot] * inv_L,
+                                 zn = prop[2 * kSlots + slot] * inv_L;
+                    // u at the lane's mover's new place less u at its old one,
+                    // against the point (x, y, z).
+                    const double a0 = (h == 0 ? s.a_same : s.a_anti) * s.L, a1 = (h == 1 ? s.a_same : s.a_anti) * s.L;
+                    const auto change = [&](double x, double y, double z, double a) {
+                        const double rn = du_dist(xn - x, yn - y, zn - z);
+                        const double ro = du_dist(xo - x, yo - y, zo - z);
+                        return a * du_pade_diff(rn, ro, bl);
+                    };
+                    // Electrons come in rounds of V: four to a wavefront, `few`
+                    // to one with a tile of T.
+                    int few = 4;
+                    if constexpr (NTask < NW) {
+                        const int tc = 14 * ((n + 15) / 16) / (kTwo ? 10 : 20);
+                        const int J = (N + ND * cnt) / (kTwo ? 1 : 2);
+                        const int y = (J + NTask * tc) / NW;
+                        few = y > tc ? (4 * (y - tc) + y / 2) / y : 0;
+                    }
+                    const int tw = wave < NTask ? wave : NTask;
+                    const int share = NTask < NW && wave < NTask ? few : 4;
+                    const int first = NTask < NW ? tw * few + (wave - tw) * 4 : wave * 4;
+                    const int V = NTask < NW ? NTask * few + (NW - NTask) * 4 : NW * 4;
+                    double acc = 0.0;
+                    // The block's movers: at their old places for the mover's
+                    // own change, and what it changes by when they move first.
+                    const int nm = ND * cnt;
+#pragma unroll 1
+                    for (int v0 = 0; v0 * (kTwo ? 1 : 2) < nm; v0 += V)
+#pragma unroll 1
+                        for (int v = 0; v < share; ++v) {
+                            const int jj = kTwo ? v0 + first + v : 2 * (v0 + first + v) + half;
+                            const int j = jj < nm ? jj : 0;
+                            const int hj = kTwo && j >= cnt ? 1 : 0, jl = j - (hj ? cnt : 0);
+                            const int js = hj * 32 + jl, ej = s.first[kTwo ? hj : hb] + q0 + jl;
+                            const double a = (kTwo ? hj : hb) ? a1 : a0;
+                            const double d = change(px[ej], py[ej], pz[ej], a);
+                            const double dn = change(prop[js] * inv_L, prop[kSlots + js] * inv_L,
+                                                     prop[2 * kSlots + js] * inv_L, a);
+                            if (jj < nm) X[(hj * NB + jl) * kSlots + slot] = dn - d;
+                            acc += jj < nm && ej != e ? d : 0.0;
+                        }
+                    // The other electrons, two at a time (past the last one
+                    // with a weight of zero).
+                    const int no = N - nm;
+                    for (int v0 = 0; v0 * (kTwo ? 1 : 2) < no; v0 += V)
+#pragma unroll 1
+                        for (int v = 0; v < share; v += 2) {
+                            double d[2];
+#pragma unroll
+                            for (int u = 0; u < 2; ++u) {
+                                const int jj = kTwo ? v0 + first + v + u : 2 * (v0 + first + v + u) + half;
+                                const bool in = v + u < share && jj < no;
+                                int j = in ? jj : 0;
+                                j += j >= s.first[hb] + q0 ? cnt : 0;
+                                if constexpr (kTwo) j += j >= s.first[1] + q0 ? cnt : 0;
+                                j = j < N ? j : 0;
+                                d[u] = change(px[j], py[j], pz[j], spin_of(s, j) ? a1 : a0);
+                                d[u] = in ? d[u] : 0.0;
+                            }
+                            acc += d[0] + d[1];
+                        }
+                    part[(kTwo ? wave : 2 * wave + half) * kSlots + slot] = acc;
+                }
+                __syncthreads();
+                if (wave == 0) {
+                    const int lane = du_thread() & (kWave - 1);
+                    const int r = lane & 31, h = kTwo ? lane >> 5 : 0, slot = kTwo ? lane : r;
+                    double T[NB];
+#pragma unroll
+                    for (int q = 0; q < NB; ++q) T[q] = Ts[(h * NB16 + q) * 32 + r];
+                    double dj = 0.0;
+#pragma unroll
+                    for (int i = 0; i < kSub; ++i) dj += part[i * kSlots + slot];
+                    const double ua = prop[3 * kSlots + slot];
+                    unsigned mask[2] = {0u, 0u};
+                    int grow[2] = {0, 0};  // log2 of the accepted ratios' product, in 1/256
+                    double rec_r = 1.0, rec_j = 0.0;
+                    int steps = cnt;
+                    // Eight columns at a time by their registers, then the
+                    // columns move on by eight: after all groups column a's
+                    // row operations sit in T[a].
+#pragma unroll 1
+                    for (int i0 = 0; i0 < NB; i0 += kG) {
+#pragma unroll
+                        for (int k = 0; k < kG; ++k) {
+                            const int i = i0 + k;
+                            if (i >= steps) break;
+                            const double R = T[k], irl = rcp_nr(R);
+                            const bool pivot = r == i;
+                            const int au = du_decide(R, dj, ua, i);
+                            rec_r = pivot ? R : rec_r;
+                            rec_j = pivot && h == 0 ? dj : rec_j;
+                            double f = 0.0;
+                            if (au) {
+                                mask[0] |= 1u << i;
+                                grow[0] += du_log2(R, i);
+                                dj += X[i * kSlots + slot];
+                                const double ir = du_readlane(irl, i);
+                                f = kTwo && h ? 0.0 : du_factor(pivot, R, ir);
+                                du_row_op<NB>(T, f, i);
+                            }
+                            if constexpr (kTwo) {
+                                const int ad = du_decide(R, dj, ua, 32 + i);
+                                rec_j = pivot && h == 1 ? dj : rec_j;
+                                if (ad) {
+                                    mask[1] |= 1u << i;
+                                    grow[1] += du_log2(R, 32 + i);
+                                    dj += X[(NB + i) * kSlots + slot];
+                                    const double ir = du_readlane(irl, 32 + i);
+                                    const double fd = h ? du_factor(pivot, R, ir) : 0.0;
+                                    du_row_op<NB>(T, fd, 32 + i);
+                                    f = h ? fd : f;
+                                }
+                            }
+                            // The mover's column is done: it takes the row
+                            // operations' own column.
+                            T[k] = pivot ? 1.0 - f : -f;
+                            const int full = (int)(__popc(mask[0]) >= kDuMaxAcc) | (int)(__popc(mask[1]) >= kDuMaxAcc) |
+                                             (int)(grow[0] > kDuGrowth) | (int)(grow[1] > kDuGrowth);
+                            steps = full ? i + 1 : steps;
+                        }
+                        double head[kG];
+#pragma unroll
+                        for (int k = 0; k < kG; ++k) head[k] = T[k];
+#pragma unroll
+                        for (int k = 0; k + kG < NB; ++k) T[k] = T[k + kG];
+#pragma unroll
+                        for (int k = 0; k < kG; ++k) T[NB - kG + k] = head[k];
+                    }
+                    const unsigned mh = mask[h];
+                    const bool mine = ((mh >> r) & 1u) && (kTwo || lane < 32);
+                    const int pb = __popc(mh & ((1u << r) - 1u));
+                    for (int i = lane; i < ND * kDuMaxAcc * (kDuMaxAcc + 1); i += kWave) sm[Lay::cinv + i] = 0.0;
+                    du_wave_fence();
+#pragma unroll
+                    for (int hh = 0; hh < ND; ++hh) {
+                        double *ci = sm + Lay::cinv + hh * kDuMaxAcc * (kDuMaxAcc + 1) + pb;
+                        const bool put = mine && (!kTwo || h == hh);
+#pragma unroll
+                        for (int q = 0; q < NB; ++q) {
+                            if ((mask[hh] >> q) & 1u) {
+                                if (put) *ci = T[q];
+                                ci += kDuMaxAcc + 1;
+                            }
+                        }
+                    }
+                    const int e = s.first[kTwo ? h : hb] + q0 + r;
+                    if (mine) {
+                        ctl[4 + 16 * h + pb] = r;
+                        const double x = prop[slot], y = prop[kSlots + slot], z = prop[2 * kSlots + slot];
+                        gp[e] = x;
+                        gp[N + e] = y;
+                        gp[2 * N + e] = z;
+                        px[e] = x * s.inv_L;
+                        py[e] = y * s.inv_L;
+                        pz[e] = z * s.inv_L;
+                    }
+                    if (lane == 0) {
+                        ctl[0] = (int)mask[0];
+                        ctl[1] = (int)mask[1];
+                        ctl[2] = steps;
+                    }
+                    if (given.trace && r < steps && (kTwo || lane < 32)) {
+                        double *tr = given.trace + ((size_t)w * N + e) * kTraceCount;
+                        tr[0] = rec_r;
+                        tr[1] = rec_j;
+                        tr[2] = mine ? 1.0 : 0.0;
+                    }
+                    const double lg = mine ? log(fabs(rec_r)) : 0.0;
+                    const double l0 = wave_sum(!kTwo || h == 0 ? lg : 0.0), l1 = kTwo ? wave_sum(h == 1 ? lg : 0.0) : 0.0;
+                    if (lane == 0) {
+                        const double na = (double)(__popc(mask[0]) + __popc(mask[1]));
+                        book[1 + hb] += l0;
+                        if (kTwo) book[2] += l1;
+                        book[3] += na;
+                        book[4] += na;
+                        book[5] += na;
+                    }
+                }
+                __syncthreads();
+                const int m0 = __popc((unsigned)ctl[0]), m1 = __popc((unsigned)ctl[1]);
+                const int next = q0 + ctl[2];
+                // The next block's proposals, beside the flush.
+                if (wave == NW - 1 && next < n)
+                    du_propose<kTwo>(s, prop, gp, given, w, sweep, book[0], hb, next, n - next < NB ? n - next : NB, lane);
+#pragma unroll 1
+                for (int h = 0; h < ND; ++h) {
+                    const int m = h ? m1 : m0, d = kTwo ? h : hb;
+                    if (m > 0)
+                        du_flush<NB, TH, kTwo, NW>(l, sm, invw + s.inv_off[d], n, h, q0, m,
+                                                   orbs + (!kTwo && hb ? s.n[0] : 0));
+                }
+                __syncthreads();
+                q0 = next;
             }
-            const uint4 r = philox4x32_10(make_uint4((uint32_t)q, (uint32_t)w, sweep, kTagMove), s.key0, s.key1);
-            const uint4 ra = philox4x32_10(make_uint4((uint32_t)q, (uint32_t)w, sweep, kTagAccept), s.key0, s.key1);
-            double dx, dy, dz;
-            if (s.move_kind == 1) {
-                const double rho0 = sqrt(-2.0 * log(u01(r.x)));
-                const double rho1 = sqrt(-2.0 * log(u01(r.z)));
-                double s0, c0, s1, c1;
-                sincospi(2.0 * u01(r.y), &s0, &c0);
-                sincospi(2.0 * u01(r.w), &s1, &c1);
-                dx = rho0 * c0;
-                dy = rho0 * s0;
-                dz = rho1 * c1;
-            } else {
-                dx = 2.0 * u01(r.x) - 1.0;
-                dy = 2.0 * u01(r.y) - 1.0;
-                dz = 2.0 * u01(r.z) - 1.0;
+        }
+        if (t == 0) {
+            if (flags & VMC_SWEEP_ADAPT) {
+                const double sigma = book[0] * exp(0.25 * (book[4] / (double)N - 0.5));
+                book[0] = sigma > 0.5 * s.L ? 0.5 * s.L : sigma;
             }
-            sh.draw[0][q] = dx;
-            sh.draw[1][q] = dy;
-            sh.draw[2][q] = dz;
-            sh.draw[3][q] = u01(ra.x);
+            book[4] = 0.0;
         }
         __syncthreads();
-        int acc = 0;
-        int m0 = 0, m1 = 0;           // window entries per determinant
-        double g0 = 1.0, g1 = 1.0;    // |product of the window's Schur complements|
-        for (int tt = 0; tt < N; ++tt) {
-            const int p = sweep_visit(s.n_up, s.n_dn, tt);
-            const int h = spin_of(s, p);
-            const int n = s.n[h];
-            const int q = p - s.first[h];
-            const int mh = h ? m1 : m0;
-            const double xo = sh.px[p], yo = sh.py[p], zo = sh.pz[p];
-            double x, y, z;
-            if (given.prop) {
-                x = sh.draw[0][p];
-                y = sh.draw[1][p];
-                z = sh.draw[2][p];
-            } else {
-                x = xo + sigma * sh.draw[0][p];
-                y = yo + sigma * sh.draw[1][p];
-                z = zo + sigma * sh.draw[2][p];
-                x -= s.L * floor(x * s.inv_L);
-                y -= s.L * floor(y * s.inv_L);
-                z -= s.L * floor(z * s.inv_L);
-            }
-            // The orbital rows at the proposal and at the mover's position, the
-            // mover's invT_0 row, and the new Jastrow pair terms.
-            double *invh = invw + s.inv_off[h];
-            if (t < n) {
-                sh.phin[t] = orbital<double>(s, h, t, x * s.inv_L, y * s.inv_L, z * s.inv_L);
-                sh.phio[t] = orbital<double>(s, h, t, xo * s.inv_L, yo * s.inv_L, zo * s.inv_L);
-                sh.qrow[t] = invh[(size_t)q * n + t];
-            }
-            double jp = 0.0;
-            for (int e = t; e < N; e += kDuThreads) {
-                double u = 0.0;
-                if (e != p) {
-                    const double r = pair_dist<double>(s, x, y, z, v, e, nullptr, nullptr, nullptr);
-                    u = pade_u<double>(r, pair_a<double>(s, p, e), b);
-                }
-                sh.uj[e] = u;
-                jp += u;
-            }
-            jp = wave_sum(jp);
-            if (lane == 0) sh.jpart[wave] = jp;
-            __syncthreads();
-            // G = L R^T over the wave's quarter of the row: L rows phi', phi(r_q),
-            // delta_0..; R rows Q, P_0..  (rows past the window hold finite
-            // values whose products are not read).
-            {
-                const int r = lane & 15, g = lane >> 4;
-                const double *arow = r == 0 ? sh.phin : r == 1 ? sh.phio : sh.delta[h][r - 2 < KD ? r - 2 : 0];
-                const double *brow = r == 0 ? sh.qrow : sh.prow[h][r - 1 < KD ? r - 1 : 0];
-                constexpr int S = P / 16;
-                const int j0 = wave * (P / 4) + g * S;
-                du_v4d gacc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                for (int k = 0; k < S; ++k)
-                    gacc = __builtin_amdgcn_mfma_f64_16x16x4f64(arow[j0 + k], brow[j0 + k], gacc, 0, 0, 0);
-                // register q of lane l holds G[4q + (l >> 4)][l & 15]
-                if (lane < 32) sh.gpart[wave][lane] = gacc[0];
-                if (r == 0) {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) sh.gpart[wave][32 + 4 * k + g] = gacc[k];
-                }
-            }
-            __syncthreads();
-            if (wave == 0) {
-                // val: lanes 0..15 G[0][l] (phi'.Q, phi'.P_a), 16..31 G[1][l-16]
-                // (phi(r_q).Q, phi(r_q).P_a), 32..47 G[l-32][0] (delta_a.Q at 34 + a).
-                double val = 0.0;
-                if (lane < 48) {
-#pragma unroll
-                    for (int wv = 0; wv < kDuWaves; ++wv) val += sh.gpart[wv][lane];
-                }
-                // z = Cinv c on lanes a < mh, then R = phi'.Q - sum_a (phi'.P_a) z_a.
-                double za = 0.0;
-                for (int k = 0; k < mh; ++k) {
-                    const double ck = du_readlane(val, 34 + k);
-                    if (lane < mh) za += sh.cinv[h][lane][k] * ck;
-                }
-                double R = du_readlane(val, 0);
-                for (int a = 0; a < mh; ++a) R -= du_readlane(val, 1 + a) * du_readlane(za, a);
-                double jn = 0.0;
-#pragma unroll
-                for (int wv = 0; wv < kDuWaves; ++wv) jn += sh.jpart[wv];
-                const double dj = jn - sh.U[p];
-                const double prob = R * R * exp(2.0 * dj);
-                const int accept = wave_uniform((int)(sh.draw[3][p] < prob));
-                double sc = 0.0;
-                if (accept) {
-                    // Border Cinv with the new entry mh: column c (delta_a.Q),
-                    // row rr_a = (phi' - phi(r_q)).P_a, corner 1 + (phi' - phi(r_q)).Q,
-                    // Schur complement sc = corner - rr.z (= R in exact arithmetic).
-                    const double corner = 1.0 + du_readlane(val, 0) - du_readlane(val, 16);
-                    double rz = 0.0, wk = 0.0;
-                    for (int a = 0; a < mh; ++a) {
-                        const double rra = du_readlane(val, 1 + a) - du_readlane(val, 17 + a);
-                        rz += rra * du_readlane(za, a);
-                        if (lane < mh) wk += rra * sh.cinv[h][a][lane];
-                    }
-                    sc = corner - rz;
-                    const double isc = 1.0 / sc;
-                    for (int a = 0; a < mh; ++a) {
-                        const double zi = du_readlane(za, a);
-                        if (lane < mh) sh.cinv[h][a][lane] += zi * wk * isc;
-                    }
-                    if (lane < mh) {
-                        sh.cinv[h][lane][mh] = -za * isc;
-                        sh.cinv[h][mh][lane] = -wk * isc;
-                    }
-                    if (lane == 0) sh.cinv[h][mh][mh] = isc;
-                }
-                if (lane == 0) {
-                    sh.dec[0] = (double)accept;
-                    sh.dec[1] = R;
-                    sh.dec[2] = jn;
-                    sh.dec[3] = sc;
-                    if (given.trace) {
-                        double *tr = given.trace + ((size_t)w * N + p) * kTraceCount;
-                        tr[0] = R;
-                        tr[1] = dj;
-                        tr[2] = (double)accept;
-                    }
-                }
-            }
-            __syncthreads();
-            if (sh.dec[0] != 0.0) {
-                const double R = sh.dec[1];
-                for (int j = t; j < P; j += kDuThreads) {
-                    sh.delta[h][mh][j] = sh.phin[j] - sh.phio[j];
-                    sh.prow[h][mh][j] = sh.qrow[j];
-                }
-                // Jastrow row sums (simulation.cpp:133-145 via the cached pair terms).
-                for (int e = t; e < N; e += kDuThreads) {
-                    if (e == p) continue;
-                    const double r = pair_dist<double>(s, xo, yo, zo, v, e, nullptr, nullptr, nullptr);
-                    sh.U[e] += sh.uj[e] - pade_u<double>(r, pair_a<double>(s, p, e), b);
-                }
-                if (t == 0) {
-                    sh.U[p] = sh.dec[2];
-                    sh.px[p] = x;
-                    sh.py[p] = y;
-                    sh.pz[p] = z;
-                }
-                ++acc;
-                ++since;
-                if (h) ld1 += log(fabs(R)); else ld0 += log(fabs(R));
-                int mn = mh + 1;
-                const double gn = (h ? g1 : g0) * fabs(sh.dec[3]);
-                if (mn == KD || gn > kDuGrowth) {
-                    __syncthreads();
-                    du_flush<P, KD>(sh, invh, n, h, mn);
-                    mn = 0;
-                }
-                if (h) {
-                    m1 = mn;
-                    g1 = mn ? gn : 1.0;
-                } else {
-                    m0 = mn;
-                    g0 = mn ? gn : 1.0;
-                }
-            }
-            __syncthreads();
-        }
-        // Apply the open windows: the inverse in memory is current between sweeps.
-        if (m0 > 0) du_flush<P, KD>(sh, invw + s.inv_off[0], s.n[0], 0, m0);
-        if (m1 > 0) du_flush<P, KD>(sh, invw + s.inv_off[1], s.n[1], 1, m1);
-        stat[6] += (double)acc;
-        stat[7] += (double)N;
-        if (flags & VMC_SWEEP_ADAPT) {
-            sigma *= exp(0.25 * ((double)acc / (double)N - 0.5));
-            if (sigma > 0.5 * s.L) sigma = 0.5 * s.L;
-        }
-    }
-    for (int i = t; i < N; i += kDuThreads) {
-        gp[i] = sh.px[i];
-        gp[N + i] = sh.py[i];
-        gp[2 * N + i] = sh.pz[i];
     }
     if (t == 0) {
-#pragma unroll
-        for (int k = 0; k < kStatCount; ++k) ws[k] = stat[k];
-        st.sigma[w] = sigma;
-        st.since[w] = since;
+        double *ws = st.stats + (size_t)w * kStatCount;
+        ws[6] += book[3];
+        ws[7] += (double)N * (double)n_sweeps;
+        st.sigma[w] = book[0];
+        st.since[w] = (int)book[5];
         st.flags[w] = st.flags[w] & ~kFlagJrowValid;  // this kernel keeps no row sums
-        st.logdet[2 * w + 0] = ld0;
-        st.logdet[2 * w + 1] = ld1;
+        st.logdet[2 * w + 0] = book[1];
+        st.logdet[2 * w + 1] = book[2];
     }
 }
 
-template <int P, int KD>
-__global__ __launch_bounds__(kDuThreads) void k_sweep_du(DevSys s, DevState st, int n_sweeps,
-                                                        unsigned long long sweep0, int flags, SweepGiven given) {
-    du_sweep_walker<P, KD>(s, st, blockIdx.x, n_sweeps, sweep0, flags, given);
+// Four wavefronts per SIMD: two resident walkers of eight wavefronts, so one
+// walker's decisions overlap with the other's matrix work.  (Five wavefronts
+// at 147 per spin, two row tiles each and 168 registers, took 2.52 ms against
+// 1.70; six at 81, 0.84 against 0.60.)
+template <int NB, int TH, bool kTwo, int NW>
+__global__ __launch_bounds__(NW * kWave, 4) void k_sweep_du(DevSys s, DevState st, int n_sweeps,
+                                                            unsigned long long sweep0, int flags, SweepGiven given) {
+    du_sweep_walker<NB, TH, kTwo, NW>(s, st, blockIdx.x, n_sweeps, sweep0, flags, given);
 }
+
+namespace {
+
+constexpr size_t kDuLdsLimit = 160 * 1024;
+
+// Calls f.template operator()<NB, TH, kTwo, NW>() with the instantiation of a
+// size: a block of 32 moves per determinant (16 up to 16 per spin), the row
+// tile in registers up to 160 per spin (beyond, 16 rows of n doubles exceed a
+// wavefront's registers).  Wavefronts per walker: four where a row tile
+// has at most four column tiles, eight to 160, sixteen above, where few
+// walkers have to fill the chip.
+template <bool kTwo, typename F>
+auto du_dispatch(int n, F f) {
+    if (n <= 16) return f.template operator()<16, 1, kTwo, 4>();
+    if (n <= 32) return f.template operator()<32, 2, kTwo, 4>();
+    if (n <= 48) return f.template operator()<32, 3, kTwo, 4>();
+    if (n <= 64) return f.template operator()<32, 4, kTwo, 4>();
+    if (n <= 96) return f.template operator()<32, 6, kTwo, 8>();
+    if (n <= 128) return f.template operator()<32, 8, kTwo, 8>();
+    if (n <= 160) return f.template operator()<32, 10, kTwo, 8>();
+    return f.template operator()<32, 0, kTwo, 16>();
+}
+
+bool du_two(const DevSys &d) { return d.ndet == 2 && d.n_up == d.n_dn; }
+
+size_t du_lds(const DevSys &d) {
+    const int norb = du_two(d) ? d.nmax : d.n[0] + (d.ndet == 2 ? d.n[1] : 0);
+    const auto size = [&]<int NB, int TH, bool kTwo, int NW>() {
+        using Lay = DuLds<NB, TH, kTwo, NW>;
+        return d.kmax < Lay::K1 ? sizeof(double) * (size_t)Lay(d.N, d.nmax, norb).total : ~size_t(0);
+    };
+    return du_two(d) ? du_dispatch<true>(d.nmax, size) : du_dispatch<false>(d.nmax, size);
+}
+
+}  // namespace
 
 bool du_supported(const DevSys &d) {
     return d.nmax <= 160 && (d.ndet == 1 || d.n_dn == d.n_up) && d.N <= 2 * 160;
 }
 
+bool du_fits(const DevSys &d) { return du_lds(d) <= kDuLdsLimit; }
+
 bool du_launch(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps, unsigned long long s0, int flags,
                const SweepGiven &given, hipStream_t stream) {
-    if (!du_supported(d)) return false;
-    if (d.nmax <= 64)
-        hipLaunchKernelGGL((k_sweep_du<64, kDuWindow>), dim3(grid), dim3(kDuThreads), 0, stream, d, st, n_sweeps,
-                           s0, flags, given);
-    else if (d.nmax <= 128)
-        hipLaunchKernelGGL((k_sweep_du<128, kDuWindow>), dim3(grid), dim3(kDuThreads), 0, stream, d, st,
-                           n_sweeps, s0, flags, given);
-    else
-        hipLaunchKernelGGL((k_sweep_du<160, kDuWindow>), dim3(grid), dim3(kDuThreads), 0, stream, d, st,
-                           n_sweeps, s0, flags, given);
-    return true;
+    if (!du_fits(d)) return false;
+    const size_t lds = du_lds(d);
+    const auto run = [&]<int NB, int TH, bool kTwo, int NW>() {
+        const auto k = k_sweep_du<NB, TH, kTwo, NW>;
+        if (lds > 64 * 1024 &&
+            hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds) != hipSuccess)
+            return false;
+        hipLaunchKernelGGL(k, dim3(grid), dim3(NW * kWave), lds, stream, d, st, n_sweeps, s0, flags, given);
+        return true;
+    };
+    return du_two(d) ? du_dispatch<true>(d.nmax, run) : du_dispatch<false>(d.nmax, run);
 }
 
 }  // namespace vmc
