@@ -52,6 +52,13 @@ struct DevSys {
     int nseg;
     const int4 *sfseg;
     const double *sfw;
+    // And as the operands of the matrix-core structure factor (vmc_tables.hpp
+    // sf_matrix): [8 sf_tiles] columns {mx, my} and [8 sf_tiles][8 sf_nz8][2]
+    // weights of (mx, my, +a) and (mx, my, -a).
+    int sf_tiles, sf_nz8;
+    int pmax;  // highest power of an axis phasor of any G vector or orbital
+    const int2 *sf_col;
+    const double *sf_w;
 };
 
 // Per-ensemble device state (walker-major SoA in HBM).
@@ -157,6 +164,7 @@ struct BatchItem {
     DevSys s;
     DevState st;
     int inv_lds;
+    int generic_energy;  // the FP64 local energy is the generic one (measure64 does not fit)
     int walker_begin;
     int walker_end;
 };

@@ -329,10 +329,12 @@ __global__ __launch_bounds__(256) void k_measure_parts(DevSys s, DevState st, do
 }
 
 // The FP64 local energy of a mixed batch's generic group after its measured
-// sweep: one workgroup per walker of the group, st.inv the FP64 inverses.
+// sweep, of the systems that measure64 does not take: one workgroup per walker
+// of the group, st.inv the FP64 inverses.
 __global__ __launch_bounds__(256) void k_measure_batch64(const BatchItem *items, int n_items, int block_size) {
     extern __shared__ __align__(16) unsigned char smem[];
     const BatchItem &it = items[batch_find(items, n_items, blockIdx.x)];
+    if (!it.generic_energy) return;
     measure_walker<double>(it.s, it.st, blockIdx.x - it.walker_begin, false, nullptr, block_size, smem);
 }
 
@@ -640,19 +642,11 @@ struct SystemTables {
     std::vector<int4> orb;
     std::vector<int4> gvec;
     std::vector<double> gw;
-    int4 *d_orb = nullptr;
-    int4 *d_gvec = nullptr;
-    double *d_gw = nullptr;
-    int4 *d_sfseg = nullptr;
-    double *d_sfw = nullptr;
+    unsigned char *d_tables = nullptr;  // every device table of `dev`, one allocation
     int real_bytes = 8;
 
     ~SystemTables() {
-        if (d_orb) (void)hipFree(d_orb);
-        if (d_gvec) (void)hipFree(d_gvec);
-        if (d_gw) (void)hipFree(d_gw);
-        if (d_sfseg) (void)hipFree(d_sfseg);
-        if (d_sfw) (void)hipFree(d_sfw);
+        if (d_tables) (void)hipFree(d_tables);
     }
 };
 
@@ -739,29 +733,32 @@ int build_tables(const vmc_system *sys, uint64_t seed, SystemTables &t) {
     for (size_t i = 0; i < g.m.size(); ++i) t.gvec[i] = make_int4(g.m[i][0], g.m[i][1], g.m[i][2], 0);
     t.gw = g.w;
     t.real_bytes = sys->precision == VMC_PREC_FP64 ? 8 : 4;
-    VMC_HIP_TRY(hipMalloc(&t.d_orb, sizeof(int4) * std::max<size_t>(t.orb.size(), 1)));
-    VMC_HIP_TRY(hipMemcpy(t.d_orb, t.orb.data(), sizeof(int4) * t.orb.size(), hipMemcpyHostToDevice));
-    VMC_HIP_TRY(hipMalloc(&t.d_gvec, sizeof(int4) * std::max<size_t>(t.gvec.size(), 1)));
-    VMC_HIP_TRY(hipMalloc(&t.d_gw, sizeof(double) * std::max<size_t>(t.gw.size(), 1)));
-    if (!t.gvec.empty()) {
-        VMC_HIP_TRY(hipMemcpy(t.d_gvec, t.gvec.data(), sizeof(int4) * t.gvec.size(), hipMemcpyHostToDevice));
-        VMC_HIP_TRY(hipMemcpy(t.d_gw, t.gw.data(), sizeof(double) * t.gw.size(), hipMemcpyHostToDevice));
-    }
-    d.orb = t.d_orb;
-    d.gvec = t.d_gvec;
-    d.gw = t.d_gw;
     const SfSegments sg = sf_segments(g);
-    std::vector<int4> seg(sg.seg.size());
-    for (size_t i = 0; i < seg.size(); ++i) seg[i] = make_int4(sg.seg[i][0], sg.seg[i][1], sg.seg[i][2], sg.seg[i][3]);
-    VMC_HIP_TRY(hipMalloc(&t.d_sfseg, sizeof(int4) * std::max<size_t>(seg.size(), 1)));
-    VMC_HIP_TRY(hipMalloc(&t.d_sfw, sizeof(double) * std::max<size_t>(sg.w.size(), 1)));
-    if (!seg.empty()) {
-        VMC_HIP_TRY(hipMemcpy(t.d_sfseg, seg.data(), sizeof(int4) * seg.size(), hipMemcpyHostToDevice));
-        VMC_HIP_TRY(hipMemcpy(t.d_sfw, sg.w.data(), sizeof(double) * sg.w.size(), hipMemcpyHostToDevice));
-    }
-    d.nseg = static_cast<int>(seg.size());
-    d.sfseg = t.d_sfseg;
-    d.sfw = t.d_sfw;
+    const SfMatrix sm = sf_matrix(g);
+    // One allocation and one copy for all tables (a served request pays for
+    // each call).
+    std::vector<unsigned char> blob;
+    const auto put = [&blob](const auto &v) {
+        const size_t at = (blob.size() + 255) & ~size_t(255), bytes = sizeof(v[0]) * v.size();
+        blob.resize(at + bytes);
+        if (bytes) std::memcpy(blob.data() + at, v.data(), bytes);
+        return at;
+    };
+    const size_t o_orb = put(t.orb), o_gvec = put(t.gvec), o_gw = put(t.gw), o_seg = put(sg.seg), o_segw = put(sg.w),
+                 o_col = put(sm.col), o_colw = put(sm.w);
+    VMC_HIP_TRY(hipMalloc(&t.d_tables, blob.size()));
+    VMC_HIP_TRY(hipMemcpy(t.d_tables, blob.data(), blob.size(), hipMemcpyHostToDevice));
+    d.orb = reinterpret_cast<const int4 *>(t.d_tables + o_orb);
+    d.gvec = reinterpret_cast<const int4 *>(t.d_tables + o_gvec);
+    d.gw = reinterpret_cast<const double *>(t.d_tables + o_gw);
+    d.nseg = static_cast<int>(sg.seg.size());
+    d.sfseg = reinterpret_cast<const int4 *>(t.d_tables + o_seg);
+    d.sfw = reinterpret_cast<const double *>(t.d_tables + o_segw);
+    d.sf_tiles = sm.tiles;
+    d.sf_nz8 = sm.nz8;
+    d.pmax = std::max(d.kmax, sm.reach);
+    d.sf_col = reinterpret_cast<const int2 *>(t.d_tables + o_col);
+    d.sf_w = reinterpret_cast<const double *>(t.d_tables + o_colw);
     return VMC_OK;
 }
 
@@ -866,10 +863,8 @@ int sweep_family(const vmc_ensemble *e) {
 }
 
 // Delayed-update sweeps (FP64), one launch per sweep when each is measured
-// or followed by the periodic re-inversion.  The local energy is the FP64
-// multi-wavefront measurement where that has an instantiation (123 and 147
-// per spin among them: it reads the inverse rows from memory), else the
-// generic one; both take the inverse the sweep left current in HBM.
+// or followed by the periodic re-inversion.  The local energy (measure64)
+// takes the inverse the sweep left current in HBM.
 int launch_sweep_du(vmc_ensemble *e, int n_sweeps, int flags, int block_size, hipStream_t stream) {
     const DevSys &d = e->tables.dev;
     const unsigned grid = static_cast<unsigned>(e->W);
@@ -891,7 +886,7 @@ int launch_sweep_du(vmc_ensemble *e, int n_sweeps, int flags, int block_size, hi
         }
         if (measure) {
             timed = e->timer.begin(stream, ev);
-            if (!rrw_measure64(d, e->st, grid, block_size, nullptr, stream))
+            if (!measure64(d, e->st, grid, block_size, nullptr, stream))
                 hipLaunchKernelGGL((k_measure_parts<double, false>), dim3(grid),
                                    dim3(static_cast<unsigned>(e->walker_threads)), lds_for(d, 8, false), stream, d,
                                    e->st, static_cast<double *>(nullptr), block_size);
@@ -1031,7 +1026,7 @@ int launch_sweep(vmc_ensemble *e, int n_sweeps, int flags, int block_size, hipSt
     // With periodic re-inversion, one sweep per launch, each followed by the
     // FP64 re-inversion of the walkers that came due.  In mixed precision a
     // measured sweep re-inverts every walker with its FP64 result in inv64
-    // and takes the local energy from that in FP64 (k_measure_parts).
+    // and takes the local energy from that in FP64 (measure64).
     const bool exact = sizeof(Real) == 4 && (flags & VMC_SWEEP_MEASURE) && e->inv64;
     const bool reinv = d.reinv_k > 0 || exact;
     const int per_launch = reinv ? 1 : n_sweeps;
@@ -1059,8 +1054,9 @@ int launch_sweep(vmc_ensemble *e, int n_sweeps, int flags, int block_size, hipSt
         }
         if (exact) {
             timed = e->timer.begin(stream, ev);
-            hipLaunchKernelGGL((k_measure_parts<double, false>), dim3(grid), dim3(e->walker_threads), lds64, stream,
-                               d, st64, static_cast<double *>(nullptr), block_size);
+            if (!measure64(d, st64, grid, block_size, nullptr, stream))
+                hipLaunchKernelGGL((k_measure_parts<double, false>), dim3(grid), dim3(e->walker_threads), lds64,
+                                   stream, d, st64, static_cast<double *>(nullptr), block_size);
             if (timed) e->timer.end(stream, ev, kTimeMeasure);
         }
     }
@@ -1374,22 +1370,22 @@ int launch_parts(vmc_ensemble *e, double *d_parts, hipStream_t s) {
     const int fam = sweep_family(e);
     if (fam == kFamRegister)
         done = rb == 4 ? rr_parts_f32(d, e->st, grid, d_parts, s) : rr_parts_f64(d, e->st, grid, d_parts, s);
-    else if (fam == kFamDelayed)
-        done = rrw_measure64(d, e->st, grid, 1, d_parts, s);
-    else if (fam == kFamMultiwave)
-        done = rb == 4 ? rrw_parts_exact_f32(d, e->st, grid, d_parts, e->inv64, s, ReinvLaunch{rb})
-                       : rrw_parts_f64(d, e->st, grid, d_parts, s);
+    else if (rb == 8 && fam != kFamGeneric)
+        done = measure64(d, e->st, grid, 1, d_parts, s);
     if (!done && rb == 4) {
-        // Mixed precision, generic kernel: FP64 re-inversion of every walker
-        // into inv64 (the walkers' state untouched), then the FP64 local
-        // energy from it, as a measured sweep takes it.
+        // Mixed precision, multi-wavefront and generic kernels: FP64
+        // re-inversion of every walker into inv64 (the walkers' state
+        // untouched), then the FP64 local energy from it, as a measured sweep
+        // takes it.
         DevState st_refresh = e->st, st64 = e->st;
         st_refresh.inv64 = e->inv64;
         st_refresh.inv64_only = 1;
         st64.inv = e->inv64;
         reinv_generic_launch(d, st_refresh, grid, s, rb);
-        hipLaunchKernelGGL((k_measure_parts<double, false>), dim3(grid), dim3(static_cast<unsigned>(e->walker_threads)),
-                           lds_for(d, 8, false), s, d, st64, d_parts, 1);
+        if (!measure64(d, st64, grid, 1, d_parts, s))
+            hipLaunchKernelGGL((k_measure_parts<double, false>), dim3(grid),
+                               dim3(static_cast<unsigned>(e->walker_threads)), lds_for(d, 8, false), s, d, st64,
+                               d_parts, 1);
         done = true;
     }
     if (!done) {
@@ -1397,13 +1393,8 @@ int launch_parts(vmc_ensemble *e, double *d_parts, hipStream_t s) {
         const bool inv_lds = lds_in <= kMaxLdsBytes && e->inv_placement != 2;
         const size_t lds = inv_lds ? lds_in : lds_for(d, rb, false);
         const dim3 block(static_cast<unsigned>(e->walker_threads));
-        if (rb == 8) {
-            if (inv_lds) hipLaunchKernelGGL((k_measure_parts<double, true>), dim3(grid), block, lds, s, d, e->st, d_parts, 1);
-            else hipLaunchKernelGGL((k_measure_parts<double, false>), dim3(grid), block, lds, s, d, e->st, d_parts, 1);
-        } else {
-            if (inv_lds) hipLaunchKernelGGL((k_measure_parts<float, true>), dim3(grid), block, lds, s, d, e->st, d_parts, 1);
-            else hipLaunchKernelGGL((k_measure_parts<float, false>), dim3(grid), block, lds, s, d, e->st, d_parts, 1);
-        }
+        if (inv_lds) hipLaunchKernelGGL((k_measure_parts<double, true>), dim3(grid), block, lds, s, d, e->st, d_parts, 1);
+        else hipLaunchKernelGGL((k_measure_parts<double, false>), dim3(grid), block, lds, s, d, e->st, d_parts, 1);
     }
     VMC_HIP_TRY(hipGetLastError());
     return VMC_OK;
@@ -1759,6 +1750,9 @@ struct BatchGroup {
     BatchItem *items_refresh = nullptr, *items_m64 = nullptr;
     std::vector<Reinv> refresh_sets;
     size_t lds64 = 0;
+    // LDS and largest N of the members whose FP64 local energy is measure64's.
+    size_t energy_lds = 0;
+    int energy_n = 0;
 
     void release() {
         for (auto &r : reinv_sets)
@@ -1873,6 +1867,11 @@ int batch_build_groups(vmc_batch *b) {
             items[k].walker_end = static_cast<int>(total);
             items[k].inv_lds = 0;
             if (d.reinv_k > 0) g.reinv = true;
+            items[k].generic_energy = measure64_fits(d) ? 0 : 1;
+            if (!items[k].generic_energy) {
+                g.energy_lds = std::max(g.energy_lds, measure64_lds(d));
+                g.energy_n = std::max(g.energy_n, d.N);
+            }
             if (g.family == 0) {
                 const bool fits = lds_for(d, e->tables.real_bytes, true) <= kMaxLdsBytes;
                 const bool inv_lds = b->placement[static_cast<size_t>(i)] == 2 ? false : fits;
@@ -1890,7 +1889,7 @@ int batch_build_groups(vmc_batch *b) {
                 const vmc_ensemble *e = b->members[static_cast<size_t>(g.members[k])];
                 ir[k].st.inv64 = e->inv64;
                 i64[k].st.inv = e->inv64;
-                if (g.family == 0) g.lds64 = std::max(g.lds64, lds_for(items[k].s, 8, false));
+                if (g.family == 0 && items[k].generic_energy) g.lds64 = std::max(g.lds64, lds_for(items[k].s, 8, false));
             }
             if ((rc = dev_alloc(&g.items_refresh, ir.size())) || (rc = dev_alloc(&g.items_m64, i64.size()))) return rc;
             VMC_HIP_TRY(hipMemcpy(g.items_refresh, ir.data(), sizeof(BatchItem) * ir.size(), hipMemcpyHostToDevice));
@@ -1983,7 +1982,10 @@ int batch_group_step(vmc_batch *b, const BatchGroup &g, int flags, int block_siz
         for (const auto &r : exact ? g.refresh_sets : g.reinv_sets)
             reinv_batch_launch(r.shape, r.items, r.n_items, static_cast<unsigned>(r.total), stream,
                                static_cast<int>(sizeof(Real)));
-        if (exact)
+        if (exact && g.energy_n > 0)
+            measure64_batch(g.energy_n, g.energy_lds, g.items_m64, n, static_cast<unsigned>(g.total), block_size,
+                            stream);
+        if (exact && g.lds64 > 0)
             hipLaunchKernelGGL(k_measure_batch64, dim3(static_cast<unsigned>(g.total)), dim3(b->threads), g.lds64,
                                stream, g.items_m64, n, block_size);
     } else if (g.family == 1) {
@@ -1993,9 +1995,9 @@ int batch_group_step(vmc_batch *b, const BatchGroup &g, int flags, int block_siz
                                      g.reinv, stream);
     } else {
         ok = f32 ? rrw_batch_step_f32(g.shape, g.items, n, static_cast<unsigned>(g.total), b->ctr, flags,
-                                      block_size, g.reinv, stream, g.items_refresh, g.items_m64)
+                                      block_size, g.reinv, stream, g.items_refresh, g.items_m64, g.energy_lds)
                  : rrw_batch_step_f64(g.shape, g.items, n, static_cast<unsigned>(g.total), b->ctr, flags,
-                                      block_size, g.reinv, stream, nullptr, nullptr);
+                                      block_size, g.reinv, stream, nullptr, nullptr, g.energy_lds);
     }
     if (!ok) return fail(VMC_ERR_INVALID, "no register-resident instantiation for a batch group");
     return VMC_OK;

@@ -107,14 +107,18 @@ bool rrw_launch_f32(const DevSys &d, const DevState &st, unsigned grid, int n_sw
 bool rrw_launch_f64(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
                     unsigned long long s0, int flags, int bs, hipStream_t stream, KernelTimer &timer,
                     const ReinvLaunch &reinv, double *inv64);
-// The FP64 multi-wavefront local energy from FP64 inverses (st64.inv): into
-// the statistics, or with `parts` into parts[w][kPartCount].
-bool rrw_measure64(const DevSys &d, const DevState &st64, unsigned grid, int bs, double *parts,
-                   hipStream_t stream);
-// Mixed-precision parts: FP64 re-inversion of every walker into inv64, then
-// rrw_measure64.
-bool rrw_parts_exact_f32(const DevSys &d, const DevState &st, unsigned grid, double *parts, double *inv64,
-                         hipStream_t stream, const ReinvLaunch &reinv);
+// The FP64 local energy from FP64 inverses (st64.inv), any number of electrons
+// (vmc_measure.hip): into the statistics, or with `parts` into
+// parts[w][kPartCount].  False where it does not fit its LDS (thousands of
+// electrons, or a reciprocal sum reaching past the 30th multiple).
+constexpr size_t kMeasure64LdsLimit = 160 * 1024;
+size_t measure64_lds(const DevSys &d);
+bool measure64_fits(const DevSys &d);
+bool measure64(const DevSys &d, const DevState &st64, unsigned grid, int bs, double *parts, hipStream_t stream);
+// A batch group's walkers (items of generic_energy = 0): max_n and lds, the
+// largest number of electrons and LDS of those systems.
+void measure64_batch(int max_n, size_t lds, const BatchItem *items_m64, int n_items, unsigned grid, int bs,
+                     hipStream_t stream);
 
 // One sweep of a batch group of register-resident systems of one size
 // (`shape` = any member's tables, `grid` = the group's walkers): the sweep,
@@ -127,16 +131,14 @@ bool rr_batch_step_f64(const DevSys &shape, const BatchItem *items, int n_items,
                        const unsigned long long *sweep_ctr, int flags, int bs, bool reinv, hipStream_t stream);
 // items_refresh / items_m64 (mixed precision): the group's items with
 // st.inv64 set and with st.inv = inv64; a measured sweep then re-inverts
-// every walker into inv64 and measures in FP64 (rrw_measure64_batch).
+// every walker into inv64 and measures in FP64.  energy_lds: the group's
+// largest measure64_lds.
 bool rrw_batch_step_f32(const DevSys &shape, const BatchItem *items, int n_items, unsigned grid,
                         const unsigned long long *sweep_ctr, int flags, int bs, bool reinv, hipStream_t stream,
-                        const BatchItem *items_refresh, const BatchItem *items_m64);
+                        const BatchItem *items_refresh, const BatchItem *items_m64, size_t energy_lds);
 bool rrw_batch_step_f64(const DevSys &shape, const BatchItem *items, int n_items, unsigned grid,
                         const unsigned long long *sweep_ctr, int flags, int bs, bool reinv, hipStream_t stream,
-                        const BatchItem *items_refresh, const BatchItem *items_m64);
-bool rrw_measure64_batch(const DevSys &shape, const BatchItem *items_m64, int n_items, unsigned grid, int bs,
-                         hipStream_t stream);
-
+                        const BatchItem *items_refresh, const BatchItem *items_m64, size_t energy_lds);
 // One sweep of the register kernels with the caller's moves, each recorded
 // (then the re-inversion, as after a sweep); and the per-walker parts of the
 // local energy by the measurement kernel, statistics untouched.  False when
@@ -151,8 +153,6 @@ bool rrw_given_f32(const DevSys &d, const DevState &st, unsigned grid, const Swe
                    hipStream_t stream, const ReinvLaunch &reinv);
 bool rrw_given_f64(const DevSys &d, const DevState &st, unsigned grid, const SweepGiven &given,
                    hipStream_t stream, const ReinvLaunch &reinv);
-bool rrw_parts_f32(const DevSys &d, const DevState &st, unsigned grid, double *parts, hipStream_t stream);
-bool rrw_parts_f64(const DevSys &d, const DevState &st, unsigned grid, double *parts, hipStream_t stream);
 
 // FP64 sweeps with delayed Woodbury updates of HBM-resident inverses, a block
 // of moves at a time (vmc_sweep_du.hip).  du_supported: what a caller may ask

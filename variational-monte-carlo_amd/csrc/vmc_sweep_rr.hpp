@@ -203,8 +203,6 @@ __device__ __forceinline__ Real jastrow_pair(Real r, Real a, Real b) {
 
 }  // namespace rr
 
-// Maximum G vectors per lane of the register-resident measurement.
-constexpr int kRRMaxGPerLane = 12;
 // Electrons whose axis-power tables are staged in LDS at once.
 constexpr int kRRChunk = 8;
 // Highest power of an axis phasor the structure factor needs (|m| <= 7).
@@ -230,13 +228,11 @@ struct RRShared {
 };
 
 // Structure factor S(G) = sum_j e^{i G.r_j} (energy_tracking.cpp:72-91) by
-// threads that own G vectors (thread t owns G t + NT k).  Electrons go
-// through in chunks of kRRChunk: 3 kRRChunk threads stage the chunk's axis
-// phasor powers X^0..X^7, Y^-7..Y^7 and Z^-7..Z^7 (one axis of one electron
-// each) in LDS as [entry][electron] (complex, padded pitch), and every thread
-// adds X^mx Y^my Z^mz of its G vectors: three conflict-free LDS reads whose
-// electron index is the reads' immediate offset, one complex product and four
-// fused accumulations.
+// threads that own column segments of G vectors.  Electrons go through in
+// chunks of kRRChunk: 3 kRRChunk threads stage the chunk's axis phasor powers
+// X^0..X^7, Y^-7..Y^7 and Z^-7..Z^7 (one axis of one electron each) in LDS as
+// [entry][electron] (complex, padded pitch; the electron index is the reads'
+// immediate offset).
 namespace sf {
 
 constexpr int kEntries = (kRRMaxPow + 1) + 2 * (2 * kRRMaxPow + 1);
@@ -276,98 +272,6 @@ __device__ __forceinline__ void stage_axis(Pair<Real> *tab, int i, int ax, bool 
         if (ax != 0) t[(centre - m) * kPitch] = {p.re, -p.im};
         p = rr::cmul(p, a);
     }
-}
-
-// term_k += X Y Z of the staged electron at pointer offset i of the entries.
-template <typename Real, int GPT>
-__device__ __forceinline__ void add_one(const Pair<Real> *tab, int i, int k, const int (&ox)[GPT],
-                                        const int (&oy)[GPT], const int (&oz)[GPT], Real (&re)[GPT],
-                                        Real (&im)[GPT]) {
-    const Pair<Real> X = tab[ox[k] + i], Y = tab[oy[k] + i], Z = tab[oz[k] + i];
-    const Real xr = X.re * Y.re - X.im * Y.im, xi = X.re * Y.im + X.im * Y.re;
-    re[k] = fma(xr, Z.re, re[k]);
-    re[k] = fma(-xi, Z.im, re[k]);
-    im[k] = fma(xr, Z.im, im[k]);
-    im[k] = fma(xi, Z.re, im[k]);
-}
-
-// Adds the kRRChunk staged electrons to the sums of the thread's G vectors
-// (ox, oy, oz: table offsets of their entries), two electrons at a time (the
-// reads in flight stay within the register budget).  Up to 5 G vectors per
-// thread the electron index is the reads' immediate offset; above, the
-// electron pairs are a loop, taken once per group of 5 G vectors.
-template <typename Real, int GPT>
-__device__ __forceinline__ void add(const Pair<Real> *tab, const int (&ox)[GPT], const int (&oy)[GPT],
-                                    const int (&oz)[GPT], Real (&re)[GPT], Real (&im)[GPT]) {
-    constexpr int kG = 5;
-    if constexpr (GPT <= kG) {
-#pragma unroll
-        for (int i = 0; i < kRRChunk; ++i) {
-#pragma unroll
-            for (int k = 0; k < GPT; ++k) add_one(tab, i, k, ox, oy, oz, re, im);
-            if (i % 2 == 1) {
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int k0 = 0; k0 < GPT; k0 += kG) {
-#pragma unroll 1
-            for (int i = 0; i < kRRChunk; i += 2) {
-#pragma unroll
-                for (int k = k0; k < (k0 + kG < GPT ? k0 + kG : GPT); ++k) {
-                    add_one(tab, i, k, ox, oy, oz, re, im);
-                    add_one(tab, i + 1, k, ox, oy, oz, re, im);
-                }
-            }
-        }
-    }
-}
-
-// sum over the thread's G vectors of w_G |S_G|^2 (to be reduced over the
-// threads).  pos_of(ax, e): coordinate ax of electron e (LDS).  tab: LDS of
-// table_reals<Real>(); every thread of the workgroup takes part.
-template <typename Real, int N, int GPT, int NT, typename PosOf>
-__device__ double energy_g(const DevSys &s, Pair<Real> *tab, int tid, PosOf pos_of) {
-    constexpr int P = kPitch;
-    int ox[GPT], oy[GPT], oz[GPT];
-    Real re[GPT], im[GPT];
-    // The G table reads stay here (not hoisted to the kernel's start, where
-    // their values would be live through the rest of the measurement).
-    asm volatile("" : "+v"(tid));
-#pragma unroll
-    for (int k = 0; k < GPT; ++k) {
-        const int g = tid + NT * k;
-        // Absent G vectors read the entries of G = 0 and get no weight.
-        const int4 G = g < s.ng ? s.gvec[g] : make_int4(0, 0, 0, 0);
-        ox[k] = G.x * P;
-        oy[k] = (kY0 + G.y) * P;
-        oz[k] = (kZ0 + G.z) * P;
-        re[k] = (Real)0;
-        im[k] = (Real)0;
-    }
-    // The last chunk's empty slots hold zeros, so every chunk is a full one.
-    constexpr int kChunks = (N + kRRChunk - 1) / kRRChunk;
-#pragma unroll 1
-    for (int c = 0; c < kChunks; ++c) {
-        __syncthreads();
-        // Thread 3 i + ax stages axis ax of slot i.
-        if (tid < 3 * kRRChunk) {
-            const int i = tid / 3, ax = tid - 3 * i, e = c * kRRChunk + i;
-            stage_axis(tab, i, ax, e < N, e < N ? pos_of(ax, e) : 0.0, s.inv_L);
-        }
-        __syncthreads();
-        add<Real, GPT>(tab, ox, oy, oz, re, im);
-    }
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < GPT; ++k) {
-        const int g = tid + NT * k;
-        if (g < s.ng) acc += s.gw[g] * ((double)re[k] * (double)re[k] + (double)im[k] * (double)im[k]);
-    }
-    __syncthreads();
-    return acc;
 }
 
 // sum_G w_G |S_G|^2 by column segments (DevSys::sfseg; thread t takes
@@ -437,17 +341,6 @@ __device__ double energy_cols(const DevSys &s, Pair<Real> *tab, int tid, PosOf p
     }
     __syncthreads();
     return acc;
-}
-
-// As energy_g with GPT slots per thread, and with fewer when the G set of the
-// Ewald sum with alpha = 5/L (at most 5 per wavefront lane) fits them.
-template <typename Real, int N, int GPT, int NT, typename PosOf>
-__device__ double energy(const DevSys &s, Pair<Real> *tab, int tid, PosOf pos_of) {
-    constexpr int kSmall = (5 * kWave + NT - 1) / NT;
-    if constexpr (kSmall < GPT) {
-        if (s.ng <= kSmall * NT) return energy_g<Real, N, kSmall, NT>(s, tab, tid, pos_of);
-    }
-    return energy_g<Real, N, GPT, NT>(s, tab, tid, pos_of);
 }
 
 }  // namespace sf

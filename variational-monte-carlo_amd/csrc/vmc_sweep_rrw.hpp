@@ -1,5 +1,5 @@
-// vmc_sweep_rrw.hpp -- register-resident sweep and local energy for spins of
-// 33 to 192 electrons: one to three wavefronts per spin.
+// vmc_sweep_rrw.hpp -- register-resident sweep for spins of 33 to 192
+// electrons: one to three wavefronts per spin.
 //
 // The workgroup of a walker holds WPS wavefronts per determinant; thread
 // (wave v, lane l) owns row r = (v mod WPS) * 64 + l of spin h = v / WPS:
@@ -32,15 +32,12 @@ struct RRWShared {
     double pos[3][N];
     alignas(16) double prop[4][N];  // this sweep's proposals (x, y, z) and accept uniforms
     Real pph[6][N];      // axis phasors of the proposals
-    Real tab[kRRChunk * 3 * (kRRMaxPow + 1) * 2];
     // Rows padded to 16 bytes, so that a row picked at run time still moves
     // with 16-byte LDS reads.
     static constexpr int kRowPad = (NMAX + 3) / 4 * 4;
     alignas(16) Real phi[2][kRowPad];   // orbital rows of the pending moves (by spin)
     alignas(16) Real row[2][kRowPad];   // inverse row of the (up) mover (by move parity)
     alignas(16) Real row2[2][kRowPad];  // inverse row of the down mover of a paired move
-    double red[NWAVE];   // per-wave partial sums
-    double red4[NWAVE][4];
     double jred[2][NWAVE];   // per-wave new Jastrow pair sums (by move parity)
     double jred2[2][NWAVE];  // the same for the down proposal of a paired move
     double mv[2][8];     // (up) mover: R, U, x, y, z (by move parity)
@@ -107,20 +104,6 @@ struct RRW {
             e = h ? NU + r : r;
         }
     };
-
-    // Workgroup sum of one value per thread (fixed order: every thread gets
-    // the same double).
-    __device__ static double block_total(double x, double *red) {
-        const double wsum = rr::wave_total(x);
-        const int v = threadIdx.x >> 6;
-        if ((threadIdx.x & (kWave - 1)) == 0) red[v] = wsum;
-        __syncthreads();
-        double t = 0.0;
-#pragma unroll
-        for (int i = 0; i < NWAVE; ++i) t += red[i];
-        __syncthreads();
-        return t;
-    }
 
     __device__ static void load(const DevSys &s, const DevState &st, int w, Sh &sh, const Thread &T,
                                 Real (&inv)[NMAX], double &x, double &y, double &z) {
@@ -608,207 +591,6 @@ __device__ __forceinline__ void sweep_rrw_body(const DevSys &s, const DevState &
     if (threadIdx.x < kStatCount) st.stats[(size_t)w * kStatCount + threadIdx.x] = sh.stat[threadIdx.x];
 }
 
-// Local energy after a sweep (energy_tracking.cpp:253-382 with the Jastrow
-// and Slater derivatives of jastrow_pade.cpp:57-138, slater_plane_wave.cpp:
-// 425-499): per thread its electron's pair terms and Slater terms; the
-// structure factor from per-electron axis-power tables staged in LDS, the
-// workgroup's threads owning G vectors.
-// With `parts` the walker's kinetic, V_real, V_recip, E_L, log|det| and J go
-// there ([w][kPartCount]) and the statistics are left alone.
-template <typename Real, int NU, int ND, int WPS>
-__device__ __forceinline__ void measure_rrw_body(const DevSys &s, const DevState &st, int w,
-                                                 int block_size, double *parts = nullptr) {
-    using K = RRW<Real, NU, ND, WPS>;
-    constexpr int N = K::N;
-    constexpr int NMAX = K::NMAX;
-    constexpr int NT = K::NT;
-    __shared__ typename K::Sh sh;
-    const RRConst<Real> c(s);
-    const typename K::Thread T;
-    // Above 96 per spin the inverse row is read where the Slater loop needs
-    // it (cached global loads) instead of being held in registers.
-    constexpr bool kRowsInMemory = NMAX > 96;
-    Real inv[kRowsInMemory ? 1 : NMAX];
-    double x, y, z;
-    if constexpr (kRowsInMemory)
-        K::load_pos(s, st, w, sh, T, x, y, z);
-    else
-        K::load(s, st, w, sh, T, inv, x, y, z);
-    const Real *row = reinterpret_cast<const Real *>(st.inv) + (size_t)w * s.ninv + (T.h ? NU * NU : 0) +
-                      (T.has_e ? T.r * T.nh : 0);
-    const auto inv_at = [&](int m) -> Real {
-        if constexpr (kRowsInMemory) return row[m];
-        else return inv[m];
-    };
-    __syncthreads();
-    // Pair terms: Jastrow gradient / Laplacian and real-space Ewald, each
-    // unordered pair once.  In step k (1 <= k <= N/2) electron e pairs with
-    // (e + k) mod N and keeps its side; the partner's side (gradient negated,
-    // same Laplacian term) goes through LDS -- the sweep's proposal arrays,
-    // unused here -- kXch steps at a time between two barriers.  For even N
-    // the last step's pairs are met from both ends: each keeps its own side
-    // and their energy counts half.  Working-precision sums per chunk, FP64
-    // across chunks.
-    constexpr int kSteps = N / 2;
-    constexpr bool kEven = N % 2 == 0;
-    constexpr int kXch = (int)((sizeof(sh.prop) + sizeof(sh.pph)) / (4 * N * sizeof(Real)));
-    static_assert(kXch >= 1, "exchange buffer");
-    static_assert(offsetof(typename K::Sh, pph) == offsetof(typename K::Sh, prop) + sizeof(sh.prop),
-                  "prop and pph are contiguous");
-    Real *xch = reinterpret_cast<Real *>(&sh.prop[0][0]);  // [kXch][4][N]
-    double gx = 0, gy = 0, gz = 0, lap = 0, vreal = 0;
-    {
-        const Real m2b = (Real)-2 * c.b;
-        for (int k0 = 1; k0 <= kSteps; k0 += kXch) {
-            Real gx_c = 0, gy_c = 0, gz_c = 0, l_c = 0, v_c = 0;
-#pragma unroll
-            for (int kk = 0; kk < kXch; ++kk) {
-                const int k = k0 + kk;
-                if (k > kSteps || !T.has_e) break;
-                const bool last_even = kEven && k == kSteps;
-                int j = T.e + k;
-                j = j >= N ? j - N : j;
-                const Real dx = c.mi_r(x, sh.pos[0][j]);
-                const Real dy = c.mi_r(y, sh.pos[1][j]);
-                const Real dz = c.mi_r(z, sh.pos[2][j]);
-                Real r, inv_r, den;
-                c.pair_geom(dx * dx + dy * dy + dz * dz, r, inv_r, den);
-                const Real a = ((ND > 0 && j >= NU) ? 1 : 0) == T.h ? c.a_same : c.a_anti;
-                const Real v = c.ewald_ri(r, inv_r);
-                v_c += last_even ? (Real)0.5 * v : v;
-                Real pgx = 0, pgy = 0, pgz = 0, pl = 0;
-                if (r >= (Real)1e-12) {
-                    const Real d1 = a * den * den;
-                    const Real gf = d1 * inv_r;
-                    const Real l = d1 * (m2b * den + (Real)2 * inv_r);
-                    gx_c += gf * dx;
-                    gy_c += gf * dy;
-                    gz_c += gf * dz;
-                    l_c += l;
-                    pgx = -gf * dx;
-                    pgy = -gf * dy;
-                    pgz = -gf * dz;
-                    pl = l;
-                }
-                if (!last_even) {
-                    Real *slot = xch + (size_t)kk * 4 * N;
-                    slot[j] = pgx;
-                    slot[N + j] = pgy;
-                    slot[2 * N + j] = pgz;
-                    slot[3 * N + j] = pl;
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int kk = 0; kk < kXch; ++kk) {
-                const int k = k0 + kk;
-                if (k > kSteps || !T.has_e) break;
-                if (kEven && k == kSteps) break;
-                const Real *slot = xch + (size_t)kk * 4 * N;
-                gx_c += slot[T.e];
-                gy_c += slot[N + T.e];
-                gz_c += slot[2 * N + T.e];
-                l_c += slot[3 * N + T.e];
-            }
-            __syncthreads();
-            gx += (double)gx_c;
-            gy += (double)gy_c;
-            gz += (double)gz_c;
-            lap += (double)l_c;
-            vreal += (double)v_c;
-        }
-    }
-    // Slater gradient and Laplacian of ln|D_h| at the thread's electron.
-    double sx = 0, sy = 0, sz = 0, sl = 0;
-    if (T.has_e) {
-        rr::Cx<Real> a[3];
-        a[0] = rr::axis_phasor<Real>(x, s.inv_L);
-        a[1] = rr::axis_phasor<Real>(y, s.inv_L);
-        a[2] = rr::axis_phasor<Real>(z, s.inv_L);
-        const Real ku = (Real)s.kunit;
-#pragma unroll
-        for (int m = 0; m < NMAX; ++m) {
-            if (K::orb[m].t == 1) continue;
-            const rr::Cx<Real> ph = K::phasor(K::orb[m].x, K::orb[m].y, K::orb[m].z, a);
-            const Real k2 = ku * ku * (Real)(K::orb[m].x * K::orb[m].x + K::orb[m].y * K::orb[m].y + K::orb[m].z * K::orb[m].z);
-            const Real wc = inv_at(m);
-            Real gsc = -wc * ph.im;
-            Real lpc = -wc * ph.re;
-            if (m + 1 < NMAX && K::orb[m + 1].t == 1) {
-                const Real ws = inv_at(m + 1);
-                gsc += ws * ph.re;
-                lpc -= ws * ph.im;
-            }
-            sx += (double)(gsc * ku * (Real)K::orb[m].x);
-            sy += (double)(gsc * ku * (Real)K::orb[m].y);
-            sz += (double)(gsc * ku * (Real)K::orb[m].z);
-            sl += (double)(lpc * k2);
-        }
-    }
-    const double slap = sl - (sx * sx + sy * sy + sz * sz);
-    const double tx = sx + gx, ty = sy + gy, tz = sz + gz;
-    const double kin_t = T.has_e ? (slap + lap + tx * tx + ty * ty + tz * tz) : 0.0;
-    const double kinetic = -0.5 * K::block_total(kin_t, sh.red);
-    const double vr = K::block_total(T.has_e ? vreal : 0.0, sh.red);
-    // Structure factor S(G) = sum_j e^{i G.r_j}: threads own G vectors; the
-    // tables are staged in the run prop | pph | tab.
-    using Sh = typename K::Sh;
-    static_assert(offsetof(Sh, pph) == offsetof(Sh, prop) + sizeof(sh.prop) &&
-                      offsetof(Sh, tab) == offsetof(Sh, pph) + sizeof(sh.pph) &&
-                      sizeof(sh.prop) + sizeof(sh.pph) + sizeof(sh.tab) >= sizeof(Real) * sf::table_reals<Real>(),
-                  "structure-factor tables exceed the run prop | pph | tab");
-    // Column segments (a third of the LDS reads per G) keep only as many
-    // threads busy as there are segments (about 80 for |n|^2 <= 25): from
-    // 256 threads one G vector per thread (at most 768 G) keeps more of
-    // them busy, which measured faster there.
-    const auto pos_of = [](int ax, int e) { return sh.pos[ax][e]; };
-    auto *sf_tab = reinterpret_cast<sf::Pair<Real> *>(&sh.prop[0][0]);
-    double acc;
-    if constexpr (NT >= 256)
-        acc = sf::energy<Real, N, (12 * kWave + NT - 1) / NT, NT>(s, sf_tab, (int)threadIdx.x, pos_of);
-    else
-        acc = sf::energy_cols<Real, N, NT>(s, sf_tab, (int)threadIdx.x, pos_of);
-    const double vrecip = __dmul_rn(s.pref, K::block_total(acc, sh.red));  // (uncontracted, as in every kernel)
-    if (parts) {
-        const double J = 0.5 * K::block_total(K::jastrow_row(c, sh, T, x, y, z), sh.red);
-        if (threadIdx.x == 0) {
-            double *q = parts + (size_t)w * kPartCount;
-            q[0] = kinetic;
-            q[1] = vr;
-            q[2] = vrecip;
-            q[3] = kinetic + vr + vrecip + s.e_const;
-            q[4] = st.logdet[2 * w + 0];
-            q[5] = ND > 0 ? st.logdet[2 * w + 1] : 0.0;
-            q[6] = J;
-        }
-        return;
-    }
-    if (threadIdx.x == 0) {
-        double *t = st.stats + (size_t)w * kStatCount;
-        const double en = kinetic + vr + vrecip + s.e_const;
-        const double pot = vr + vrecip + s.e_const;
-        t[0] += 1.0;
-        t[1] += en;
-        t[2] += en * en;
-        t[3] += kinetic;
-        t[4] += pot;
-        t[5] = en;
-        t[13] = kinetic;
-        t[14] = pot;
-        t[8] += en;
-        t[9] += 1.0;
-        if (t[9] >= (double)block_size) {
-            const double bm = t[8] / (double)block_size;
-            t[10] += 1.0;
-            const double delta = bm - t[11];
-            t[11] += delta / t[10];
-            t[12] += delta * (bm - t[11]);
-            t[8] = 0.0;
-            t[9] = 0.0;
-        }
-    }
-}
-
 // Waves per SIMD the sweep kernel is compiled for.  57 + 57 and 81 + 81 in
 // FP32 take four (at most 128 VGPRs, 16 and 32 B of spill per lane): eight
 // and four walkers per CU, so 2048 and 1024 walkers are resident at once.
@@ -827,31 +609,12 @@ __global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real,
     sweep_rrw_body<Real, NU, ND, WPS>(s, st, blockIdx.x, sweep0, flags);
 }
 
-template <typename Real, int NU, int ND, int WPS>
-constexpr int rrw_measure_waves() {
-    if constexpr (sizeof(Real) == 4 && ((NU == 33 && ND == 33) || (NU == 147 && ND == 147))) return 5;
-    return (sizeof(Real) == 4 && ((NU == 81 && ND == 81) || (NU == 123 && ND == 123))) ? 4 : 1;
-}
-
-template <typename Real, int NU, int ND, int WPS>
-__global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_measure_waves<Real, NU, ND, WPS>())) void k_measure_rrw(DevSys s, DevState st,
-                                                                            int block_size) {
-    measure_rrw_body<Real, NU, ND, WPS>(s, st, blockIdx.x, block_size);
-}
-
 // The sweep with the caller's moves, each recorded (parity checks of the
 // timed move code).
 template <typename Real, int NU, int ND, int WPS>
 __global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real, NU, ND, WPS>())) void k_sweep_rrw_given(
     DevSys s, DevState st, int flags, SweepGiven given) {
     sweep_rrw_body<Real, NU, ND, WPS, true>(s, st, blockIdx.x, 0, flags, given);
-}
-
-// The local energy's parts per walker, statistics untouched.
-template <typename Real, int NU, int ND, int WPS>
-__global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64) void k_measure_rrw_parts(DevSys s, DevState st,
-                                                                                  double *parts) {
-    measure_rrw_body<Real, NU, ND, WPS>(s, st, blockIdx.x, 1, parts);
 }
 
 // Batch forms over a group of systems of one size (as k_sweep_rr_b).
@@ -861,13 +624,6 @@ __global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real,
     int flags) {
     const BatchItem &it = items[batch_find(items, n_items, blockIdx.x)];
     sweep_rrw_body<Real, NU, ND, WPS>(it.s, it.st, blockIdx.x - it.walker_begin, *sweep_ctr, flags);
-}
-
-template <typename Real, int NU, int ND, int WPS>
-__global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_measure_waves<Real, NU, ND, WPS>())) void k_measure_rrw_b(
-    const BatchItem *__restrict__ items, int n_items, int block_size) {
-    const BatchItem &it = items[batch_find(items, n_items, blockIdx.x)];
-    measure_rrw_body<Real, NU, ND, WPS>(it.s, it.st, blockIdx.x - it.walker_begin, block_size);
 }
 
 }  // namespace vmc

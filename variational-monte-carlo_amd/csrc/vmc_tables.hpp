@@ -132,4 +132,40 @@ inline SfSegments sf_segments(const GTable &g) {
     return out;
 }
 
+// The same G vectors as a matrix: columns (mx, my), eight to a tile, by powers
+// a = |mz| of Z, eight to a tile, with the weights of +a and -a (0 where the
+// set holds none, in the padding too).
+struct SfMatrix {
+    int tiles = 0, nz8 = 1, reach = 0;
+    std::vector<std::array<int, 2>> col;  // [8 tiles]
+    std::vector<double> w;                // [8 tiles][8 nz8][2]
+};
+
+inline SfMatrix sf_matrix(const GTable &g) {
+    std::map<std::pair<int, int>, int> index;
+    int amax = 0;
+    SfMatrix out;
+    for (const auto &m : g.m) {
+        index.emplace(std::pair{m[0], m[1]}, 0);
+        amax = std::max(amax, std::abs(m[2]));
+        for (const int c : m) out.reach = std::max(out.reach, std::abs(c));
+    }
+    out.tiles = static_cast<int>((index.size() + 7) / 8);
+    out.nz8 = amax / 8 + 1;
+    int k = 0;
+    for (auto &[c, i] : index) {
+        i = k++;
+        out.col.push_back({c.first, c.second});
+    }
+    out.col.resize(static_cast<size_t>(8 * out.tiles), {0, 0});
+    const size_t na = static_cast<size_t>(8 * out.nz8);
+    out.w.assign(out.col.size() * na * 2, 0.0);
+    for (size_t i = 0; i < g.m.size(); ++i) {
+        const auto &m = g.m[i];
+        const size_t c = static_cast<size_t>(index[{m[0], m[1]}]);
+        out.w[(c * na + static_cast<size_t>(std::abs(m[2]))) * 2 + (m[2] < 0 ? 1 : 0)] = g.w[i];
+    }
+    return out;
+}
+
 }  // namespace vmc
