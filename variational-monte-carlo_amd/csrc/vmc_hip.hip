@@ -50,10 +50,12 @@ constexpr size_t kMaxLdsBytes = 64 * 1024;
 // retried while a determinant is singular, mirroring
 // Simulation::initialize_positions (simulation.cpp:43-76).  With draw == 0
 // the current positions are kept and only the FP64 inverses are rebuilt.
+// only_singular: just the walkers whose first draw init_fast found singular.
 template <typename Real>
-__global__ __launch_bounds__(kWave) void k_init(DevSys s, DevState st, int draw) {
+__global__ __launch_bounds__(kWave) void k_init(DevSys s, DevState st, int draw, int only_singular) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int w = blockIdx.x;
+    if (only_singular && !(st.flags[w] & kFlagSingular)) return;
     const int lane = threadIdx.x;
     const int N = s.N;
     Real *inv_hbm = reinterpret_cast<Real *>(st.inv) + (size_t)w * s.ninv;
@@ -829,12 +831,16 @@ struct vmc_ensemble {
 
 namespace {
 
+// Positions (draw: Philox; else aos, the caller's [W][N][3] on the device, or
+// null for the ones in place) and the FP64 inverses; walkers that init_fast
+// leaves singular, and determinants that it does not take, go through k_init.
 template <typename Real>
-int launch_init(vmc_ensemble *e, int draw, hipStream_t stream) {
+int launch_init(vmc_ensemble *e, int draw, const double *aos, hipStream_t stream) {
     const DevSys &d = e->tables.dev;
+    const bool fast = init_fast(d, e->st, draw, aos, static_cast<int>(sizeof(Real)), stream);
     const size_t lds = lds_for(d, sizeof(Real), false);
     hipLaunchKernelGGL((k_init<Real>), dim3(static_cast<unsigned>(e->W)), dim3(kWave), lds, stream,
-                       d, e->st, draw);
+                       d, e->st, draw, fast ? 1 : 0);
     VMC_HIP_TRY(hipGetLastError());
     return VMC_OK;
 }
@@ -1194,7 +1200,7 @@ static int finish_init(vmc_ensemble *e, hipStream_t stream) {
 int vmc_ensemble_init_positions(vmc_ensemble *e, void *stream) {
     if (!e) return fail(VMC_ERR_INVALID, "ensemble is NULL");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int rc = e->tables.real_bytes == 8 ? launch_init<double>(e, 1, s) : launch_init<float>(e, 1, s);
+    int rc = e->tables.real_bytes == 8 ? launch_init<double>(e, 1, nullptr, s) : launch_init<float>(e, 1, nullptr, s);
     if (rc) return rc;
     return finish_init(e, s);
 }
@@ -1204,17 +1210,26 @@ int vmc_ensemble_set_positions(vmc_ensemble *e, const double *pos, void *stream)
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int N = e->tables.dev.N;
     const size_t W = static_cast<size_t>(e->W);
-    std::vector<double> soa(W * 3 * N);
     const double L = e->tables.dev.L;
-    for (size_t w = 0; w < W; ++w)
-        for (int i = 0; i < N; ++i)
-            for (int c = 0; c < 3; ++c) {
-                const double x = pos[(w * N + i) * 3 + c];
-                if (!(x >= 0.0 && x < L)) return fail(VMC_ERR_INVALID, "position outside [0, L)");
-                soa[(w * 3 + c) * N + i] = x;
-            }
-    VMC_HIP_TRY(hipMemcpyAsync(e->st.pos, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice, s));
-    int rc = e->tables.real_bytes == 8 ? launch_init<double>(e, 0, s) : launch_init<float>(e, 0, s);
+    for (size_t i = 0; i < W * 3 * N; ++i)
+        if (!(pos[i] >= 0.0 && pos[i] < L)) return fail(VMC_ERR_INVALID, "position outside [0, L)");
+    // As they are into the Gauss-Jordan workspace, whence the device takes
+    // them into its layout (init_fast); for the determinants it does not take,
+    // and workspaces too small, they are laid out here.
+    const size_t nmax2 = static_cast<size_t>(e->tables.dev.nmax) * e->tables.dev.nmax;
+    std::vector<double> soa;
+    const double *aos = nullptr;
+    if (e->tables.dev.nmax <= kInitFastMax && nmax2 >= static_cast<size_t>(3 * N)) {
+        VMC_HIP_TRY(hipMemcpyAsync(e->st.scratch, pos, sizeof(double) * W * 3 * N, hipMemcpyHostToDevice, s));
+        aos = e->st.scratch;
+    } else {
+        soa.resize(W * 3 * N);
+        for (size_t w = 0; w < W; ++w)
+            for (int i = 0; i < N; ++i)
+                for (int c = 0; c < 3; ++c) soa[(w * 3 + c) * N + i] = pos[(w * N + i) * 3 + c];
+        VMC_HIP_TRY(hipMemcpyAsync(e->st.pos, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice, s));
+    }
+    int rc = e->tables.real_bytes == 8 ? launch_init<double>(e, 0, aos, s) : launch_init<float>(e, 0, aos, s);
     if (rc) return rc;
     return finish_init(e, s);
 }
