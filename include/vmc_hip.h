@@ -247,9 +247,9 @@ int vmc_ensemble_set_kernel(vmc_ensemble *e, int32_t kernel);
 /* The kernel the next sweep launch will use (VMC_KERNEL_GENERIC, _REGISTER
  * or _DELAYED). */
 int vmc_ensemble_get_kernel(const vmc_ensemble *e, int32_t *kernel);
-/* Register-kernel build variant: 0 = unbounded registers, 1 = at most 128
- * VGPRs (4 waves per SIMD, some spills).  No reference counterpart; an
- * autotuner knob. */
+/* Register-kernel build variant, 0 or 1: both are the same kernel now that
+ * every one fits 128 VGPRs (4 waves per SIMD) without spills.  No reference
+ * counterpart. */
 int vmc_ensemble_set_rr_variant(vmc_ensemble *e, int32_t variant);
 /* Walker groups of the register kernels' measured sweeps: the walkers are
  * split into `groups` contiguous ranges (1 to 8; default 1), each swept and

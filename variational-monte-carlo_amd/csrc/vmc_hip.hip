@@ -790,7 +790,6 @@ struct vmc_ensemble {
     double step0 = 0.0;
     bool positions_ready = false;
     int kernel = VMC_KERNEL_AUTO;
-    int rr_variant = 0;
     KernelTimer timer;
     int inv_placement = 0;  // generic kernel: 0 LDS when it fits, 1 LDS, 2 HBM
     int walker_threads = 64;  // generic kernel: threads (1, 2 or 4 wavefronts) per walker
@@ -978,8 +977,8 @@ int launch_sweep(vmc_ensemble *e, int n_sweeps, int flags, int block_size, hipSt
         const unsigned long long s0 = (unsigned long long)e->sweeps_done;
         const auto run = [&](const DevState &st, unsigned grid, hipStream_t s) {
             return sizeof(Real) == 4
-                       ? rr_launch_f32(d, st, grid, n_sweeps, s0, flags, block_size, e->rr_variant, s, e->timer)
-                       : rr_launch_f64(d, st, grid, n_sweeps, s0, flags, block_size, e->rr_variant, s, e->timer);
+                       ? rr_launch_f32(d, st, grid, n_sweeps, s0, flags, block_size, s, e->timer)
+                       : rr_launch_f64(d, st, grid, n_sweeps, s0, flags, block_size, s, e->timer);
         };
         const int G = walker_groups(e, flags);
         if (G <= 1) {
@@ -1521,8 +1520,7 @@ int vmc_ensemble_set_walker_groups(vmc_ensemble *e, int32_t groups) {
 int vmc_ensemble_set_rr_variant(vmc_ensemble *e, int32_t variant) {
     if (!e) return fail(VMC_ERR_INVALID, "ensemble is NULL");
     if (variant != 0 && variant != 1) return fail(VMC_ERR_INVALID, "unknown variant %d", variant);
-    e->rr_variant = variant;
-    return VMC_OK;
+    return VMC_OK;  // one kernel serves both
 }
 
 int vmc_ensemble_set_inverse_placement(vmc_ensemble *e, int32_t placement) {

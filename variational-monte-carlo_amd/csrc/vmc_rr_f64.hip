@@ -3,9 +3,9 @@
 
 namespace vmc {
 bool rr_launch_f64(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
-                   unsigned long long s0, int flags, int bs, int variant, hipStream_t stream,
+                   unsigned long long s0, int flags, int bs, hipStream_t stream,
                    KernelTimer &timer) {
-    return rr_launch<double>(d, st, grid, n_sweeps, s0, flags, bs, variant, stream, timer);
+    return rr_launch<double>(d, st, grid, n_sweeps, s0, flags, bs, stream, timer);
 }
 bool rr_batch_step_f64(const DevSys &shape, const BatchItem *items, int n_items, unsigned grid,
                        const unsigned long long *sweep_ctr, int flags, int bs, bool reinv, hipStream_t stream) {

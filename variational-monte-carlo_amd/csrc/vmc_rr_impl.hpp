@@ -15,7 +15,7 @@ namespace vmc {
 // walker's inverse itself: a measured sweep takes no separate re-inversion.
 template <typename Real, int NU, int ND, int GPL>
 void rr_launch_g(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
-                 unsigned long long s0, int flags, int bs, int variant, hipStream_t stream,
+                 unsigned long long s0, int flags, int bs, hipStream_t stream,
                  KernelTimer &timer) {
     constexpr bool kMixed = sizeof(Real) == 4;
     const bool measure = flags & VMC_SWEEP_MEASURE;
@@ -30,12 +30,8 @@ void rr_launch_g(const DevSys &d, const DevState &st, unsigned grid, int n_sweep
         const unsigned long long si = s0 + (unsigned long long)i;
         hipEvent_t ev = nullptr;
         bool timed = timer.begin(stream, ev);
-        if (variant == 1)
-            hipLaunchKernelGGL((k_sweep_rr_o4<Real, NU, ND, GPL>), dim3(grid), dim3(kWave), 0,
-                               stream, d, st, si, flags);
-        else
-            hipLaunchKernelGGL((k_sweep_rr<Real, NU, ND, GPL>), dim3(grid), dim3(kWave), 0, stream,
-                               d, st, si, flags);
+        hipLaunchKernelGGL((k_sweep_rr<Real, NU, ND, GPL>), dim3(grid), dim3(kWave), 0, stream,
+                           d, st, si, flags);
         if (timed) timer.end(stream, ev, kTimeSweep);
         if (reinv) {
             timed = timer.begin(stream, ev);
@@ -76,10 +72,10 @@ bool rr_dispatch(const DevSys &d, F &&f) {
 
 template <typename Real>
 bool rr_launch(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
-               unsigned long long s0, int flags, int bs, int variant, hipStream_t stream,
+               unsigned long long s0, int flags, int bs, hipStream_t stream,
                KernelTimer &timer) {
     return rr_dispatch<Real>(d, [&]<int NU, int ND, int GPL>() {
-        rr_launch_g<Real, NU, ND, GPL>(d, st, grid, n_sweeps, s0, flags, bs, variant, stream, timer);
+        rr_launch_g<Real, NU, ND, GPL>(d, st, grid, n_sweeps, s0, flags, bs, stream, timer);
     });
 }
 

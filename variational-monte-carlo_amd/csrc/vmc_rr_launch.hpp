@@ -173,12 +173,12 @@ bool du_launch(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
                const SweepGiven &given, hipStream_t stream);
 
 // Launches n_sweeps sweeps (and, with VMC_SWEEP_MEASURE, one measurement per
-// sweep).  variant 0: no occupancy bound; 1: at most 128 VGPRs.
+// sweep).
 bool rr_launch_f32(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
-                   unsigned long long s0, int flags, int bs, int variant, hipStream_t stream,
+                   unsigned long long s0, int flags, int bs, hipStream_t stream,
                    KernelTimer &timer);
 bool rr_launch_f64(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
-                   unsigned long long s0, int flags, int bs, int variant, hipStream_t stream,
+                   unsigned long long s0, int flags, int bs, hipStream_t stream,
                    KernelTimer &timer);
 
 }  // namespace vmc

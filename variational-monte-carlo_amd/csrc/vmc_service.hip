@@ -116,7 +116,6 @@ int vmc_autotune(const vmc_system *sys, int64_t n_walkers, double drift_tol, int
         if (rc) return rc;
         if (!vmc_ensemble_set_kernel(e, VMC_KERNEL_REGISTER)) {
             cands.push_back({VMC_KERNEL_REGISTER, 0, 0, 64});
-            cands.push_back({VMC_KERNEL_REGISTER, 1, 0, 64});
         }
         if (!vmc_ensemble_set_kernel(e, VMC_KERNEL_DELAYED)) cands.push_back({VMC_KERNEL_DELAYED, 0, 0, 64});
         const bool lds_ok = !vmc_ensemble_set_inverse_placement(e, 1);

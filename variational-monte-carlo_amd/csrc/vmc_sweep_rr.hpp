@@ -5,15 +5,19 @@
 // transposed inverse, lanes 32..63 those of spin down: lane (h, r) keeps
 // invT_h[r][0..n) in VGPRs together with electron r of spin h (position,
 // Jastrow row sum U, the sweep's proposal and its axis phasors).  Per move:
-//   - the proposal of electron p and its axis phasors e^{2 pi i u'} are read
-//     from lane p (v_readlane), every orbital of the row is a product of axis
-//     phasors (no transcendental on the move's critical path);
-//   - the orbital row is broadcast through 32 LDS words and every row lane
-//     forms s_k = sum_m phi_m invT[k][m]; the ratio is s_p (v_readlane);
-//   - the Jastrow new-pair sum is a DPP row reduction plus four readlanes, so
+//   - the proposals of the sweep and their axis phasors are made by all lanes
+//     at once beforehand and lie in LDS; lane m forms orbital m as a product
+//     of three staged phasors (no transcendental and no selection on the
+//     move's critical path);
+//   - every row lane forms s_k = sum_m phi_m invT[k][m] with phi_m broadcast
+//     from lane m by the FMA itself (DPP); the ratio is s_p (v_readlane);
+//   - the Jastrow new-pair sum is a DPP row reduction plus readlanes, so
 //     the accept decision is a scalar branch;
 //   - on accept, row p is broadcast through LDS and each row lane applies the
-//     Sherman-Morrison update to its own registers.
+//     Sherman-Morrison update to its own registers, both spins' in one pass.
+// What bounds it: VALU instructions (FP64 at 27 per spin: 375 per pair of
+// moves, 556 with the orbital row broadcast through LDS, phasors selected per
+// move and IEEE roots and divisions in the pair terms).
 // The per-sweep local energy uses the same registers plus an LDS mirror of the
 // positions.
 #pragma once
@@ -24,6 +28,14 @@
 
 #include <array>
 #include <cstddef>
+
+// The sweeps' broadcasting FP64 FMA (v_fmac_f64 with DPP) is a two-address
+// form, which the build turns off for the polynomials of the other kernels.
+#ifdef __HIP_DEVICE_COMPILE__
+#define VMC_FMAC64 __attribute__((target("fmacf64-inst")))
+#else
+#define VMC_FMAC64
+#endif
 
 namespace vmc {
 namespace rr {
@@ -122,6 +134,78 @@ __device__ __forceinline__ T wave_total(T v) {
     return (readlane(v, 0) + readlane(v, 16)) + (readlane(v, 32) + readlane(v, 48));
 }
 
+// a = the values of row 0 (rows 0, 1) or row 2 (rows 2, 3), b those of row 1 or
+// 3: both of a half's rows of 16 in each of its rows.
+__device__ __forceinline__ void swap_rows16(float &a, float &b) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(p[0]);
+    b = __uint_as_float(p[1]);
+}
+__device__ __forceinline__ void swap_rows16(double &a, double &b) {
+    const unsigned long long u = __double_as_longlong(a), v = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)v, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(v >> 32), false, false);
+    a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
+    b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+
+// The whole-wave sums of a and b as wave-uniform values: lanes 0..31 add up a,
+// lanes 32..63 b (v_permlane32_swap), so one row reduction serves both.
+__device__ __forceinline__ void wave_totals(double a, double b, double &sa, double &sb) {
+    const unsigned long long u = __double_as_longlong(a), v = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)v, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(v >> 32), false, false);
+    const double t = row_sum(__longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]) +
+                             __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]));
+    sa = readlane(t, 0) + readlane(t, 16);
+    sb = readlane(t, 32) + readlane(t, 48);
+}
+
+// s0 += sum over even, s1 += sum over odd k in [0, n) (n <= 4) of
+// p(lane B + k of the lane's row of 16) v[k], one FMA each with the broadcast in it.
+// One asm block: a DPP read needs two wait states after the VALU write of its
+// source, which the compiler's hazard pass does not see here.
+#define VMC_FMAC_ROW(ty, acc, v, b) \
+    "v_fmac_" ty "_dpp %" acc ", %2, %" v " row_newbcast:%" b " row_mask:0xf bank_mask:0xf\n\t"
+template <int n, int B, typename Real>
+__device__ __forceinline__ void fmac_row16(Real &s0, Real &s1, Real p, const Real *v) {
+#define VMC_FMAC_ROWS(ty)                                                                                           \
+    if constexpr (n == 1)                                                                                           \
+        asm("s_nop 1\n\t" VMC_FMAC_ROW(ty, "0", "3", "4") : "+v"(s0), "+v"(s1) : "v"(p), "v"(v[0]), "n"(B));          \
+    else if constexpr (n == 2)                                                                                      \
+        asm("s_nop 1\n\t" VMC_FMAC_ROW(ty, "0", "3", "5") VMC_FMAC_ROW(ty, "1", "4", "6")                           \
+            : "+v"(s0), "+v"(s1)                                                                                    \
+            : "v"(p), "v"(v[0]), "v"(v[1]), "n"(B), "n"(B + 1));                                                    \
+    else if constexpr (n == 3)                                                                                      \
+        asm("s_nop 1\n\t" VMC_FMAC_ROW(ty, "0", "3", "6") VMC_FMAC_ROW(ty, "1", "4", "7")                           \
+                VMC_FMAC_ROW(ty, "0", "5", "8")                                                                     \
+            : "+v"(s0), "+v"(s1)                                                                                    \
+            : "v"(p), "v"(v[0]), "v"(v[1]), "v"(v[2]), "n"(B), "n"(B + 1), "n"(B + 2));                             \
+    else                                                                                                            \
+        asm("s_nop 1\n\t" VMC_FMAC_ROW(ty, "0", "3", "7") VMC_FMAC_ROW(ty, "1", "4", "8")                           \
+                VMC_FMAC_ROW(ty, "0", "5", "9") VMC_FMAC_ROW(ty, "1", "6", "10")                                    \
+            : "+v"(s0), "+v"(s1)                                                                                    \
+            : "v"(p), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "n"(B), "n"(B + 1), "n"(B + 2), "n"(B + 3))
+    if constexpr (sizeof(Real) == 8) {
+        VMC_FMAC_ROWS("f64");
+    } else {
+        VMC_FMAC_ROWS("f32");
+    }
+#undef VMC_FMAC_ROWS
+}
+#undef VMC_FMAC_ROW
+
+// The same over the elements [M0, min(N, M0 + 16)) of v.
+template <int N, int M0, typename Real, int B = 0>
+__device__ __forceinline__ void dot_row16(Real &s0, Real &s1, Real p, const Real (&v)[N]) {
+    constexpr int left = (N - M0 < 16 ? N - M0 : 16) - B;
+    if constexpr (left > 0) {
+        constexpr int n = left < 4 ? left : 4;
+        fmac_row16<n, B>(s0, s1, p, &v[M0 + B]);
+        dot_row16<N, M0, Real, B + n>(s0, s1, p, v);
+    }
+}
+
 template <typename Real>
 struct Cx {
     Real re, im;
@@ -207,25 +291,6 @@ __device__ __forceinline__ Real jastrow_pair(Real r, Real a, Real b) {
 constexpr int kRRChunk = 8;
 // Highest power of an axis phasor the structure factor needs (|m| <= 7).
 constexpr int kRRMaxPow = 7;
-
-template <typename Real, int NU, int ND>
-struct RRShared {
-    double pos[3][kWave];          // positions by lane (pair loops of the measurement)
-    alignas(16) double prop[4][kWave];  // this sweep's proposal x, y, z and accept uniform
-    Real pph[6][kWave];            // axis phasors of the proposal (re, im per axis)
-    Real tab[kRRChunk * 3 * (kRRMaxPow + 1) * 2];  // with prop and pph: staging (below)
-    double stat[kStatCount];
-    double misc[4];                // sigma, log|det| up, log|det| down
-    Real phi[2][32];               // orbital rows of the pending moves (by spin)
-    Real row[32];                  // inverse row of the moved electron
-    double gjcol[32];
-    int perm[32];
-    // The run prop | pph | tab as one staging area (inverse blocks, the
-    // structure-factor tables of the measurement).
-    static constexpr size_t kStageBytes =
-        sizeof(double) * 4 * kWave + sizeof(Real) * 6 * kWave + sizeof(Real) * kRRChunk * 3 * (kRRMaxPow + 1) * 2;
-    __device__ void *stage() { return &prop[0][0]; }
-};
 
 // Structure factor S(G) = sum_j e^{i G.r_j} (energy_tracking.cpp:72-91) by
 // threads that own column segments of G vectors.  Electrons go through in
@@ -345,20 +410,42 @@ __device__ double energy_cols(const DevSys &s, Pair<Real> *tab, int tid, PosOf p
 
 }  // namespace sf
 
-// The LDS run prop | pph | tab of RRShared doubles as the stage through which
-// inverse blocks move between HBM and the lanes' registers, and holds the
-// structure-factor tables of the measurement.
+// LDS of the measurement: positions, and one staging area for the inverse
+// blocks and then the structure-factor tables.
 template <typename Real, int NU, int ND>
-__device__ __forceinline__ Real *rr_stage(RRShared<Real, NU, ND> &sh) {
-    using Sh = RRShared<Real, NU, ND>;
-    static_assert(offsetof(Sh, pph) == offsetof(Sh, prop) + sizeof(sh.prop) &&
-                      offsetof(Sh, tab) == offsetof(Sh, pph) + sizeof(sh.pph),
-                  "stage run must be contiguous");
-    constexpr int NMAX = NU > ND ? NU : ND;
-    static_assert(sizeof(sh.prop) + sizeof(sh.pph) + sizeof(sh.tab) >= sizeof(Real) * NMAX * NMAX,
-                  "stage too small for one inverse block");
-    return reinterpret_cast<Real *>(&sh.prop[0][0]);
-}
+struct RRShared {
+    static constexpr int NMAX = NU > ND ? NU : ND;
+    double pos[3][kWave];  // positions by lane
+    static constexpr int kStageReals =
+        NMAX * NMAX > sf::table_reals<Real>() ? NMAX * NMAX : sf::table_reals<Real>();
+    alignas(16) Real buf[kStageReals];
+    static constexpr size_t kStageBytes = sizeof(Real) * kStageReals;
+    __device__ Real *stage() { return buf; }
+};
+
+// Axis-phasor entries of one electron's proposal: X, -iX (the cosine and the
+// sine orbitals' real parts), Y, Y*, Z, Z*.
+constexpr int kRRPow = 6;
+
+// LDS of the sweep.  The inverse blocks pass through the run from prop on,
+// before the proposals are staged and after the last move; the positions are
+// there for the Jastrow row sums only.
+template <typename Real, int NU, int ND>
+struct RRSweepShared {
+    static constexpr int NMAX = NU > ND ? NU : ND;
+    static constexpr int kPropReals = 4 * kWave * (int)(sizeof(double) / sizeof(Real));
+    static constexpr int kPowPairs = (NU + ND) * kRRPow + 2;  // and the constants 1 and -i
+    static constexpr int kPad = NMAX * NMAX - kPropReals - 2 * kPowPairs;
+    union {
+        double prop[kWave][4];  // by lane: this sweep's proposal x, y, z and accept uniform
+        double pos[3][kWave];
+    };
+    alignas(16) sf::Pair<Real> pow[kPowPairs + (kPad > 0 ? (kPad + 1) / 2 : 0)];
+    alignas(16) Real row[2][32];  // inverse rows of the moved electrons (by spin)
+    double stat[kStatCount];
+    double misc[4];               // sigma, log|det| up, log|det| down
+    __device__ Real *stage() { return reinterpret_cast<Real *>(&prop[0][0]); }
+};
 
 // Inverse blocks of both spins between HBM ([NU x NU][ND x ND], row k =
 // invT[k][.]) and the lanes' registers (lane (h, r) holds row r of spin h):
@@ -531,7 +618,6 @@ struct RRLane {
     Real inv[NMAX];   // row r of invT of spin h
     double x, y, z;   // electron position
     double U;         // Jastrow row sum
-    int orb;          // orbital r: (nx+4) | (ny+4) << 4 | (nz+4) << 8 | type << 12
 };
 
 __device__ __forceinline__ int orb_nx(int o) { return (o & 15) - 4; }
@@ -539,7 +625,18 @@ __device__ __forceinline__ int orb_ny(int o) { return ((o >> 4) & 15) - 4; }
 __device__ __forceinline__ int orb_nz(int o) { return ((o >> 8) & 15) - 4; }
 __device__ __forceinline__ int orb_t(int o) { return o >> 12; }
 
-__device__ __attribute__((noinline)) double rr_exp_f64(double x);
+// e^x for |x| < 100 within an ulp or two: x = k ln 2 + f and the Taylor series of
+// e^f in Horner form.  The accept test's rare exact branch: a loop without
+// constants of its own, so that nothing is kept in registers for it across the
+// moves (a call would keep the wave's state out of the caller-saved half).
+__device__ __forceinline__ double rr_exp_f64(double x) {
+    const double k = rint(x * 1.4426950408889634);
+    const double f = fma(-k, 2.3190468138462996e-17, fma(-k, 0.69314718055994531, x));
+    double e = 1.0;
+#pragma unroll 1
+    for (int n = 18; n > 0; --n) e = fma(f * e, rcp_nr((double)n), 1.0);
+    return ldexp(e, (int)k);
+}
 
 template <typename Real, int NU, int ND, int GPL>
 struct RRKernel {
@@ -547,7 +644,7 @@ struct RRKernel {
     static constexpr int NMAX = NU > ND ? NU : ND;
     static constexpr auto orb = rr::shell_orbitals<NMAX>();
     static constexpr int kMaxPow = rr::max_component<NMAX>();
-    using Sh = RRShared<Real, NU, ND>;
+    using Sh = RRSweepShared<Real, NU, ND>;
     static_assert(NU <= 32 && ND <= 32, "register-resident path holds at most 32 rows per spin");
     static_assert(ND == 0 || ND == NU, "register-resident path: polarised or equal spins");
 
@@ -762,52 +859,121 @@ struct RRKernel {
         return wave_uniform(acc);
     }
 
-    // Pade pair value of the lane's electron with the point (xq, yq, zq).
-    __device__ static Real pair_with(const RRConst<Real> &c, const RRLane<Real, NMAX> &L, double xq, double yq,
+    // Pade pair value a r / (1 + b r) at separation d.  In FP64 as
+    // a / (1/r + b): one inverse square root and one reciprocal (rsqrt_nr and
+    // rcp_nr, 17 operations) instead of an IEEE root and division (50).
+    __device__ static Real pade(const RRConst<Real> &c, Real dx, Real dy, Real dz, Real a) {
+        if constexpr (sizeof(Real) == 8) {
+            const double r2 = fmax(fma(dx, dx, fma(dy, dy, dz * dz)), 1e-200);
+            return a * rcp_nr(rsqrt_nr(r2) + c.b);
+        } else {
+            const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
+            return a * rn * wrcp<Real>((Real)1 + c.b * rn);
+        }
+    }
+    __device__ static Real pair_with(const RRConst<Real> &c, double x, double y, double z, double xq, double yq,
                                      double zq, Real a) {
-        const Real dx = c.mi_r(xq, L.x);
-        const Real dy = c.mi_r(yq, L.y);
-        const Real dz = c.mi_r(zq, L.z);
-        const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-        return a * rn * wrcp<Real>((Real)1 + c.b * rn);
+        return pade(c, c.mi_r(xq, x), c.mi_r(yq, y), c.mi_r(zq, z), a);
     }
 
-    // Sherman-Morrison for an accepted move of electron (hm, i) with ratio R
-    // (row s_k of every lane of spin hm), then the Jastrow row sums: every
-    // other lane adds its new pair term un minus its old one, recomputed from
-    // the mover's old position.  Lane lm takes the proposal (xn, yn, zn) and
-    // the row sum jn.
-    __device__ static void apply_move(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, int lane,
-                                      bool has_e, int h, int r, int hm, int i, double R, Real sk, Real un,
-                                      double jn, double xn, double yn, double zn) {
-        constexpr int NP = NU;
-        const int lm = hm * 32 + i;
-        if (lane == lm) {
-#pragma unroll
-            for (int m = 0; m < NP; ++m) sh.row[m] = L.inv[m];
+    // Where a lane's orbital finds its axis phasors in Sh::pow: entry i step + first
+    // for move i (constants have step 0).
+    struct PhasorAt {
+        int first[3], step[3];
+        int sine;
+    };
+    __device__ static void phasor_at(int lane, int h, int r, PhasorAt &at) {
+        static_assert(kMaxPow <= 1, "axis phasors are staged as first powers");
+        constexpr int kOne = N * kRRPow;
+        at.sine = 0;
+        for (int k = 0; k < 3; ++k) {
+            at.first[k] = kOne;
+            at.step[k] = 0;
         }
-        __syncthreads();
-        {
-            const Real inv_ratio = wrcp<Real>((Real)R);
-            Real f = (r == i) ? (Real)1 - inv_ratio : sk * inv_ratio;
-            f = (h == hm && r < NP) ? f : (Real)0;
 #pragma unroll
-            for (int m = 0; m < NP; ++m) L.inv[m] -= sh.row[m] * f;
+        for (int m = 0; m < NMAX; ++m) {
+            if (r != m) continue;
+            const int n[3] = {orb[m].x, orb[m].y, orb[m].z};
+            const int sine = orb[m].t;
+            at.sine = sine;
+            for (int k = 0; k < 3; ++k) {
+                // FP64 takes sin orbitals from the phasor -iX, FP32 as the imaginary part.
+                const int alt = k == 0 ? (sizeof(Real) == 8 ? sine : 0) : (n[k] < 0 ? 1 : 0);
+                if (n[k] != 0) {
+                    at.first[k] = (h && ND > 0 ? NU * kRRPow : 0) + 2 * k + alt;
+                    at.step[k] = kRRPow;
+                } else if (k == 0) {
+                    at.first[k] = kOne + alt;
+                }
+            }
         }
+    }
+    // The lane's orbital at its spin's proposal i.
+    __device__ static Real orbital(const Sh &sh, const PhasorAt &at, int i) {
+        const sf::Pair<Real> X = sh.pow[at.first[0] + i * at.step[0]];
+        const sf::Pair<Real> Y = sh.pow[at.first[1] + i * at.step[1]];
+        const sf::Pair<Real> Z = sh.pow[at.first[2] + i * at.step[2]];
+        const rr::Cx<Real> P = rr::cmul(rr::Cx<Real>{X.re, X.im}, rr::Cx<Real>{Y.re, Y.im});
+        if constexpr (sizeof(Real) == 8) {
+            return P.re * Z.re - P.im * Z.im;
+        } else {
+            const rr::Cx<Real> ph = rr::cmul(P, rr::Cx<Real>{Z.re, Z.im});
+            return at.sine ? ph.im : ph.re;
+        }
+    }
+
+    // s_k = sum_m phi_m invT[k][m] for the lane's row, phi_m on lane m of the
+    // lane's half: each row of 16 lanes takes the 16 (and the other 16)
+    // values of its half by v_permlane16_swap and broadcasts them one by one
+    // within the FMA (DPP row_newbcast), even and odd m in two sums.
+    __device__ static Real dot_phi(Real phi, const Real (&inv)[NMAX]) {
+        Real lo = phi, hi = phi;
+        if constexpr (NMAX > 16) rr::swap_rows16(lo, hi);
+        Real s0 = (Real)0, s1 = (Real)0;
+        rr::dot_row16<NMAX, 0>(s0, s1, lo, inv);
+        if constexpr (NMAX > 16) rr::dot_row16<NMAX, 16>(s0, s1, hi, inv);
+        return s0 + s1;
+    }
+
+    // Jastrow row sums after an accepted move of lane lm: every other lane
+    // adds its new pair term un minus its old one, recomputed from the mover's
+    // old position; lane lm takes its proposal and the row sum jn.
+    __device__ static void accept_jastrow(const RRConst<Real> &c, const Sh &sh, RRLane<Real, NMAX> &L, int lane,
+                                          bool has_e, int lm, Real a, Real un, double jn) {
         const double xo = rr::readlane(L.x, lm), yo = rr::readlane(L.y, lm), zo = rr::readlane(L.z, lm);
-        if (has_e && lane != lm) {
-            const Real ao = (h == hm) ? c.a_same : c.a_anti;
-            L.U += (double)un - (double)pair_with(c, L, xo, yo, zo, ao);
-        }
+        const double du = (double)un - (double)pair_with(c, L.x, L.y, L.z, xo, yo, zo, a);
+        if (has_e && lane != lm) L.U += du;
         if (lane == lm) {
             L.U = jn;
-            L.x = xn;
-            L.y = yn;
-            L.z = zn;
-            sh.pos[0][lane] = xn;
-            sh.pos[1][lane] = yn;
-            sh.pos[2][lane] = zn;
+            L.x = sh.prop[lane][0];
+            L.y = sh.prop[lane][1];
+            L.z = sh.prop[lane][2];
         }
+    }
+
+    // Sherman-Morrison (simulation.cpp:133-145, slater_plane_wave.cpp:
+    // 367-423) as one FMA per element and lane: rows k != i of a determinant
+    // whose move was accepted lose (s_k / R) row_i; row i itself (row_i is
+    // its own registers) loses (1 - 1/R) of itself, i.e. becomes row_i / R;
+    // every other lane subtracts 0 x (a finite row).  Both determinants at
+    // once: each half of the wave reads its own row i.
+    __device__ static void update_rows(Sh &sh, RRLane<Real, NMAX> &L, int h, int r, int i, bool accepted, double R,
+                                       Real sk) {
+        constexpr int kHalves = ND > 0 ? 2 : 1;
+        const int hr = kHalves == 2 ? h : 0;
+        __syncthreads();  // the last move's rows have been read
+        if (r == i && h < kHalves) {
+#pragma unroll
+            for (int m = 0; m < NU; ++m) sh.row[hr][m] = L.inv[m];
+        }
+        __syncthreads();
+        Real inv_ratio;
+        if constexpr (sizeof(Real) == 8) inv_ratio = rcp_nr(accepted ? R : 1.0);
+        else inv_ratio = wrcp<Real>((Real)R);
+        Real f = (r == i) ? (Real)1 - inv_ratio : sk * inv_ratio;
+        f = (accepted && r < NU) ? f : (Real)0;
+#pragma unroll
+        for (int m = 0; m < NU; ++m) L.inv[m] -= sh.row[hr][m] * f;
     }
 
     // The moves of up electron i and then down electron i (the sweep order
@@ -816,71 +982,49 @@ struct RRKernel {
     // ratios of both proposals at once, and every lane forms its pair terms
     // with both.  The down move's Jastrow change uses the up electron where
     // the up move left it: its pair term with the down proposal is formed for
-    // both outcomes.  Same decisions and updates as two calls of move.
-    // Returns the number of accepted moves.
-    __device__ static int move_pair(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, int lane,
-                                    bool has_e, int h, int r, int i, LogDetTrack &ldt, double *rec) {
+    // both outcomes (the one with the up proposal by the up electron's own
+    // lane).  Same decisions and updates as two calls of move.  Returns the
+    // number of accepted moves.
+    __device__ static int move_pair(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, const PhasorAt &at,
+                                    int lane, bool has_e, int h, int r, int i, LogDetTrack &ldt, double *rec) {
         static_assert(ND == NU, "paired moves need equal spins");
-        constexpr int NP = NU;
         const int lu = i, ld = 32 + i;
-        const double xu = sh.prop[0][lu], yu = sh.prop[1][lu], zu = sh.prop[2][lu];
-        const double xd = sh.prop[0][ld], yd = sh.prop[1][ld], zd = sh.prop[2][ld];
-        // Orbital rows: lane (h, j) evaluates orbital j at its spin's proposal.
-        {
-            const int lp = h ? ld : lu;
-            rr::Cx<Real> a[3], a2[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                a[k].re = sh.pph[2 * k][lp];
-                a[k].im = sh.pph[2 * k + 1][lp];
-            }
-            squares(a, a2);
-            if (r < NP) {
-                const rr::Cx<Real> ph = rr::orbital_phasor<Real>(orb_nx(L.orb), orb_ny(L.orb), orb_nz(L.orb), a, a2);
-                sh.phi[h][r] = orb_t(L.orb) ? ph.im : ph.re;
-            }
+        const Real phi = orbital(sh, at, i);
+        const double *qu = sh.prop[lu], *qd = sh.prop[ld];
+        const Real a_u = h == 0 ? c.a_same : c.a_anti, a_d = h == 1 ? c.a_same : c.a_anti;
+        const bool mover = lane == lu;
+        Real un_u = pair_with(c, mover ? qd[0] : L.x, mover ? qd[1] : L.y, mover ? qd[2] : L.z, qu[0], qu[1], qu[2],
+                              mover ? c.a_anti : a_u);
+        Real un_d = pair_with(c, L.x, L.y, L.z, qd[0], qd[1], qd[2], a_d);
+        const Real ud_new = rr::readlane(un_u, lu), ud_old = rr::readlane(un_d, lu);
+        un_u = has_e && lane != lu ? un_u : (Real)0;
+        un_d = has_e && lane != ld ? un_d : (Real)0;
+        double jn_u, jn_d0;  // new row sums of the movers; down with the up electron at its old position
+        if constexpr (sizeof(Real) == 8) {
+            rr::wave_totals(un_u, un_d, jn_u, jn_d0);
+        } else {
+            jn_u = (double)rr::wave_total(un_u);
+            jn_d0 = (double)rr::wave_total(un_d);
         }
-        // Jastrow: new pair terms against both proposals; the down proposal's
-        // pair with the up proposal (taken when the up move is accepted).
-        Real un_u = (Real)0, un_d = (Real)0;
-        if (has_e && lane != lu) un_u = pair_with(c, L, xu, yu, zu, h == 0 ? c.a_same : c.a_anti);
-        if (has_e && lane != ld) un_d = pair_with(c, L, xd, yd, zd, h == 1 ? c.a_same : c.a_anti);
-        Real ud_new;
-        {
-            const Real dx = c.mi_r(xd, xu), dy = c.mi_r(yd, yu), dz = c.mi_r(zd, zu);
-            const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-            ud_new = c.a_anti * rn * wrcp<Real>((Real)1 + c.b * rn);
-        }
-        __syncthreads();
-        // s_k = sum_m phi_m invT[k][m] with the lane's spin's orbital row.
-        Real sk0 = (Real)0, sk1 = (Real)0;
-#pragma unroll
-        for (int m = 0; m < NP; m += 2) {
-            sk0 += sh.phi[h][m] * L.inv[m];
-            if (m + 1 < NP) sk1 += sh.phi[h][m + 1] * L.inv[m + 1];
-        }
-        const Real sk = sk0 + sk1;
+        const Real sk = dot_phi(phi, L.inv);
         const double Ru = (double)rr::readlane(sk, lu), Rd = (double)rr::readlane(sk, ld);
-        const double jn_u = (double)rr::wave_total(un_u);
-        const double jn_d0 = (double)rr::wave_total(un_d);    // up electron at its old position
-        const Real ud_old = rr::readlane(un_d, lu);
         // Up move.
         const double dj_u = jn_u - rr::readlane(L.U, lu);
-        const int acc_u = accept_test(Ru, dj_u, sh.prop[3][lu]);
+        const int acc_u = accept_test(Ru, dj_u, qu[3]);
         if (acc_u) {
-            apply_move(c, sh, L, lane, has_e, h, r, 0, i, Ru, sk, un_u, jn_u, xu, yu, zu);
+            accept_jastrow(c, sh, L, lane, has_e, lu, a_u, un_u, jn_u);
             if (lane == lu) un_d = ud_new;
             ldt.add(0, Ru);
         }
         // Down move, after the up move's outcome.
         const double jn_d = acc_u ? jn_d0 + ((double)ud_new - (double)ud_old) : jn_d0;
         const double dj_d = jn_d - rr::readlane(L.U, ld);
-        const int acc_d = accept_test(Rd, dj_d, sh.prop[3][ld]);
+        const int acc_d = accept_test(Rd, dj_d, qd[3]);
         if (acc_d) {
-            __syncthreads();  // the up move's reads of the broadcast row are done
-            apply_move(c, sh, L, lane, has_e, h, r, 1, i, Rd, sk, un_d, jn_d, xd, yd, zd);
+            accept_jastrow(c, sh, L, lane, has_e, ld, a_d, un_d, jn_d);
             ldt.add(1, Rd);
         }
+        if (acc_u | acc_d) update_rows(sh, L, h, r, i, (h ? acc_d : acc_u) != 0, h ? Rd : Ru, sk);
         if (rec && lane == 0) {
             double *ru = rec + kTraceCount * i, *rd = rec + kTraceCount * (NU + i);
             ru[0] = Ru;
@@ -893,138 +1037,54 @@ struct RRKernel {
         return acc_u + acc_d;
     }
 
-    // One move of electron (HP, rp).  Returns 1 if accepted.
-    template <int HP>
-    __device__ static int move(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, int lane,
-                               bool has_e, int h, int r, int rp, LogDetTrack &ldt, double *rec) {
-        constexpr int NP = HP ? ND : NU;
-        const int lp = HP * 32 + rp;
-        const double xn = sh.prop[0][lp], yn = sh.prop[1][lp], zn = sh.prop[2][lp];
-        rr::Cx<Real> a[3], a2[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            a[k].re = sh.pph[2 * k][lp];
-            a[k].im = sh.pph[2 * k + 1][lp];
-        }
-        squares(a, a2);
-        // Orbital row of the proposal: lane (HP, j) evaluates orbital j.
-        if (h == HP && r < NP) {
-            const rr::Cx<Real> ph = rr::orbital_phasor<Real>(orb_nx(L.orb), orb_ny(L.orb), orb_nz(L.orb), a, a2);
-            sh.phi[HP][r] = orb_t(L.orb) ? ph.im : ph.re;
-        }
-        // Jastrow: new pair terms against every other electron.
-        const Real apair = (h == HP) ? c.a_same : c.a_anti;
-        Real un = (Real)0;
-        if (has_e && lane != lp) {
-            const Real dx = c.mi_r(xn, L.x);
-            const Real dy = c.mi_r(yn, L.y);
-            const Real dz = c.mi_r(zn, L.z);
-            const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-            un = apair * rn * wrcp<Real>((Real)1 + c.b * rn);
-        }
-        __syncthreads();
-        // s_k = sum_m phi_m invT[k][m] for every row k of spin HP (computed
-        // on every lane without branching; only spin HP's rows are used).
-        Real sk0 = (Real)0, sk1 = (Real)0;
-#pragma unroll
-        for (int m = 0; m < NP; m += 2) {
-            sk0 += sh.phi[HP][m] * L.inv[m];
-            if (m + 1 < NP) sk1 += sh.phi[HP][m + 1] * L.inv[m + 1];
-        }
-        const Real sk = sk0 + sk1;
-        const double R = (double)rr::readlane(sk, lp);
-        // New Jastrow row sum of the mover: summed in the working precision
-        // (its FP32 rounding only moves the accept threshold by ~1e-6).
+    // One move of electron i of the only determinant.  Returns 1 if accepted.
+    __device__ static int move(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, const PhasorAt &at, int lane,
+                               bool has_e, int h, int r, int i, LogDetTrack &ldt, double *rec) {
+        static_assert(ND == 0, "unpaired moves are the polarised system's");
+        const Real phi = orbital(sh, at, i);
+        const double *q = sh.prop[i];
+        Real un = pair_with(c, L.x, L.y, L.z, q[0], q[1], q[2], c.a_same);
+        un = has_e && lane != i ? un : (Real)0;
         const double jn = (double)rr::wave_total(un);
-        const double dj = jn - rr::readlane(L.U, lp);
-        const double ua = sh.prop[3][lp];
-        // Metropolis test u < R^2 exp(2 dJ) (simulation.cpp:125-131).  The
-        // hardware exp2 (relative error < 1e-6 here) decides unless u lies
-        // within 1e-5 of the threshold, where the exact FP64 exp decides, so
-        // the outcome equals the FP64 comparison.
-        const double r2 = R * R;
-        const float e32 = __builtin_amdgcn_exp2f((float)(2.0 * dj * 1.4426950408889634));
-        const double approx = r2 * (double)e32;
-        int acc;
-        if (!(approx == approx)) {
-            acc = 0;
-        } else if (fabs(ua - approx) > 1e-5 * approx || !(fabs(dj) < 40.0)) {
-            acc = ua < approx;
-        } else {
-            acc = ua < r2 * rr_exp_f64(2.0 * dj);
-        }
-        // Every input above is wave-uniform; say so, so the branches are scalar.
-        const int accepted = wave_uniform(acc);
+        const Real sk = dot_phi(phi, L.inv);
+        const double R = (double)rr::readlane(sk, i);
+        const double dj = jn - rr::readlane(L.U, i);
+        const int accepted = accept_test(R, dj, q[3]);
         if (rec && lane == 0) {
-            double *q = rec + kTraceCount * (HP ? NU + rp : rp);
-            q[0] = R;
-            q[1] = dj;
-            q[2] = (double)accepted;
-        }
-        // Sherman-Morrison (simulation.cpp:133-145, slater_plane_wave.cpp:
-        // 367-423) as one FMA per element and lane: rows k != p of spin HP
-        // lose (s_k / R) row_p; row p itself (row_p is its own registers)
-        // loses (1 - 1/R) of itself, i.e. becomes row_p / R; every other lane
-        // subtracts 0 x (a finite row).  A rejected move skips the update on
-        // a wave-uniform branch.
-        if (!accepted) return 0;
-        if (lane == lp) {
-#pragma unroll
-            for (int m = 0; m < NP; ++m) sh.row[m] = L.inv[m];
-        }
-        __syncthreads();
-        {
-            const Real inv_ratio = wrcp<Real>((Real)R);
-            Real f = (r == rp) ? (Real)1 - inv_ratio : sk * inv_ratio;
-            f = (accepted && h == HP && r < NP) ? f : (Real)0;
-#pragma unroll
-            for (int m = 0; m < NP; ++m) L.inv[m] -= sh.row[m] * f;
+            double *t = rec + kTraceCount * i;
+            t[0] = R;
+            t[1] = dj;
+            t[2] = (double)accepted;
         }
         if (!accepted) return 0;
-        ldt.add(HP, R);
-        const double xo = rr::readlane(L.x, lp), yo = rr::readlane(L.y, lp), zo = rr::readlane(L.z, lp);
-        if (has_e && lane != lp) {
-            const Real dx = c.mi_r(xo, L.x);
-            const Real dy = c.mi_r(yo, L.y);
-            const Real dz = c.mi_r(zo, L.z);
-            const Real ro = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-            L.U += (double)un - (double)(apair * ro * wrcp<Real>((Real)1 + c.b * ro));
-        }
-        if (lane == lp) {
-            L.U = jn;
-            L.x = xn;
-            L.y = yn;
-            L.z = zn;
-            sh.pos[0][lane] = xn;
-            sh.pos[1][lane] = yn;
-            sh.pos[2][lane] = zn;
-        }
+        ldt.add(0, R);
+        accept_jastrow(c, sh, L, lane, has_e, i, c.a_same, un, jn);
+        update_rows(sh, L, h, r, i, h == 0, R, sk);
         return 1;
     }
 };
 
-// The proposal q (in [0, L)), its axis phasors and the accept uniform ua
-// into the lane's LDS slots.
-template <typename Real>
-__device__ __forceinline__ void rr_stage_proposal(const DevSys &s, const double (&q)[3], double ua, int lane,
-                                                  double *prop, Real *pph) {
+// The proposal q (in [0, L)), the accept uniform ua and the proposal's axis
+// phasors into the LDS slots of the lane's electron e.
+template <typename Real, typename Sh>
+__device__ __forceinline__ void rr_stage_proposal(const DevSys &s, const double (&q)[3], double ua, int lane, int e,
+                                                  Sh &sh) {
+    sf::Pair<Real> *t = sh.pow + e * kRRPow;
     for (int k = 0; k < 3; ++k) {
-        prop[k * kWave + lane] = q[k];
+        sh.prop[lane][k] = q[k];
         const rr::Cx<Real> ph = rr::axis_phasor<Real>(q[k], s.inv_L);
-        pph[(2 * k) * kWave + lane] = ph.re;
-        pph[(2 * k + 1) * kWave + lane] = ph.im;
+        t[2 * k] = {ph.re, ph.im};
+        t[2 * k + 1] = k == 0 ? sf::Pair<Real>{ph.im, -ph.re} : sf::Pair<Real>{ph.re, -ph.im};
     }
-    prop[3 * kWave + lane] = ua;
+    sh.prop[lane][3] = ua;
 }
 
 // Philox draws (tags MOVE and ACCP, counter {electron, walker, sweep}),
 // Box-Muller or uniform-cube displacement, wrap into [0, L) and the axis
 // phasors of the proposal, written to the lane's LDS slots.
-template <typename Real>
-__device__ __forceinline__ void rr_proposal(const DevSys &s, double sigma, double x0,
-                                                      double y0, double z0, int e, int w,
-                                                      uint32_t sweep, int lane, double *prop,
-                                                      Real *pph) {
+template <typename Real, typename Sh>
+__device__ __forceinline__ void rr_proposal(const DevSys &s, double sigma, double x0, double y0, double z0, int e,
+                                            int w, uint32_t sweep, int lane, Sh &sh) {
     const uint4 rm = philox4x32_10(make_uint4((uint32_t)e, (uint32_t)w, sweep, kTagMove), s.key0, s.key1);
     const uint4 ra = philox4x32_10(make_uint4((uint32_t)e, (uint32_t)w, sweep, kTagAccept), s.key0, s.key1);
     double dx, dy, dz;
@@ -1045,10 +1105,8 @@ __device__ __forceinline__ void rr_proposal(const DevSys &s, double sigma, doubl
     const double x = x0 + sigma * dx, y = y0 + sigma * dy, z = z0 + sigma * dz;
     const double q[3] = {x - s.L * floor(x * s.inv_L), y - s.L * floor(y * s.inv_L),
                          z - s.L * floor(z * s.inv_L)};
-    rr_stage_proposal<Real>(s, q, u01(ra.x), lane, prop, pph);
+    rr_stage_proposal<Real>(s, q, u01(ra.x), lane, e, sh);
 }
-
-__device__ __attribute__((noinline)) double rr_exp_f64(double x) { return exp(x); }
 
 // kGiven: the moves come from the caller (SweepGiven) instead of Philox and
 // each move's ratio, Jastrow change and decision are recorded.
@@ -1059,7 +1117,7 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
     using K = RRKernel<Real, NU, ND, GPL>;
     constexpr int NMAX = K::NMAX;
     constexpr int N = NU + ND;
-    __shared__ RRShared<Real, NU, ND> sh;
+    __shared__ typename K::Sh sh;
     const RRConst<Real> cst(s);
     const int lane = threadIdx.x;
     const int h = lane >> 5, r = lane & 31;
@@ -1070,7 +1128,7 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
     RRLane<Real, NMAX> L;
     const Real *inv_hbm = reinterpret_cast<const Real *>(st.inv) + (size_t)w * s.ninv;
     const double *gp = st.pos + (size_t)w * 3 * N;
-    rr_inverse_in<Real, NU, ND, NMAX>(inv_hbm, rr_stage(sh), L.inv, lane, h, r);
+    rr_inverse_in<Real, NU, ND, NMAX>(inv_hbm, sh.stage(), L.inv, lane, h, r);
     L.x = has_e ? gp[e] : 0.0;
     L.y = has_e ? gp[N + e] : 0.0;
     L.z = has_e ? gp[2 * N + e] : 0.0;
@@ -1083,11 +1141,8 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
         sh.misc[1] = st.logdet[2 * w + 0];
         sh.misc[2] = st.logdet[2 * w + 1];
     }
-    L.orb = 0;
-#pragma unroll
-    for (int m = 0; m < NMAX; ++m)
-        if (r == m)
-            L.orb = (K::orb[m].x + 4) | ((K::orb[m].y + 4) << 4) | ((K::orb[m].z + 4) << 8) | (K::orb[m].t << 12);
+    typename K::PhasorAt at;
+    K::phasor_at(lane, h, r, at);
     __syncthreads();
     int since = st.since[w];
     if (s.reinv_k > 0 && since >= s.reinv_k) since = 0;  // re-inverted after the last sweep
@@ -1104,16 +1159,20 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
     // move that reads it.  One sweep per launch keeps this straight-line code
     // out of the move loop, so its transcendental constants die before it.
     double *rec = nullptr;
+    __syncthreads();  // the row sums have read the positions that the proposals replace
     if constexpr (kGiven) {
         if (has_e) {
             const size_t q = (size_t)w * N + e;
             const double p3[3] = {given.prop[3 * q], given.prop[3 * q + 1], given.prop[3 * q + 2]};
-            rr_stage_proposal<Real>(s, p3, given.u[q], lane, &sh.prop[0][0], &sh.pph[0][0]);
+            rr_stage_proposal<Real>(s, p3, given.u[q], lane, e, sh);
         }
         rec = given.trace + (size_t)w * N * kTraceCount;
     } else {
-        if (has_e) rr_proposal<Real>(s, sh.misc[0], L.x, L.y, L.z, e, st.w0 + w, sweep, lane, &sh.prop[0][0],
-                                      &sh.pph[0][0]);
+        if (has_e) rr_proposal<Real>(s, sh.misc[0], L.x, L.y, L.z, e, st.w0 + w, sweep, lane, sh);
+    }
+    if (lane == 0) {
+        sh.pow[N * kRRPow] = {(Real)1, (Real)0};
+        sh.pow[N * kRRPow + 1] = {(Real)0, (Real)-1};
     }
     __syncthreads();
     // Sweep order (sweep_visit): with two determinants (ND == NU) the spins
@@ -1123,10 +1182,10 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
     if constexpr (ND > 0) {
         static_assert(ND == NU, "two determinants of equal size");
 #pragma unroll 1
-        for (int p = 0; p < NU; ++p) acc += K::move_pair(cst, sh, L, lane, has_e, h, r, p, ldt, rec);
+        for (int p = 0; p < NU; ++p) acc += K::move_pair(cst, sh, L, at, lane, has_e, h, r, p, ldt, rec);
     } else {
 #pragma unroll 1
-        for (int p = 0; p < NU; ++p) acc += K::template move<0>(cst, sh, L, lane, has_e, h, r, p, ldt, rec);
+        for (int p = 0; p < NU; ++p) acc += K::move(cst, sh, L, at, lane, has_e, h, r, p, ldt, rec);
     }
     const int n_acc = acc;
     since += acc;
@@ -1138,7 +1197,7 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
         }
     }
     Real *inv_out = reinterpret_cast<Real *>(st.inv) + (size_t)w * s.ninv;
-    rr_inverse_out<Real, NU, ND, NMAX>(inv_out, rr_stage(sh), L.inv, lane, h, r);
+    rr_inverse_out<Real, NU, ND, NMAX>(inv_out, sh.stage(), L.inv, lane, h, r);
     if (has_e) {
         double *gq = st.pos + (size_t)w * 3 * N;
         gq[e] = L.x;
@@ -1165,35 +1224,28 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
     if (lane < kStatCount) st.stats[(size_t)w * kStatCount + lane] = sh.stat[lane];
 }
 
-// The sweep kernel, without and with a 4-waves-per-SIMD occupancy bound (the
-// bound caps VGPRs at 128 at the price of some spills; the autotuner picks).
-// Waves per SIMD the sweep is built for (its registers at that occupancy;
-// the paired FP32 move at 27 per spin needs 100 VGPRs, four waves, without
-// spilling).
+// Waves per SIMD the sweep is built for.  FP64 at 27 per spin takes 115 VGPRs
+// and 8.1 KB of LDS: all four walkers of a SIMD at 4096 walkers run at once.
+// (With three at a time and the fourth alone, at 168 VGPRs and 11 KB, the
+// sweep took 188 us instead of 121.)
 template <typename Real, int NU, int ND>
 constexpr int rr_sweep_waves() {
     constexpr bool kLarge = (NU > ND ? NU : ND) >= 19;
-    if constexpr (sizeof(Real) == 8) return kLarge ? 3 : 4;
+    if constexpr (sizeof(Real) == 8) return 4;
     if constexpr ((NU > ND ? NU : ND) >= 27) return 4;
     return kLarge ? 5 : 6;
 }
 
 template <typename Real, int NU, int ND, int GPL>
-__global__ __launch_bounds__(kWave, (rr_sweep_waves<Real, NU, ND>())) void k_sweep_rr(DevSys s, DevState st,
-                                                    unsigned long long sweep0, int flags) {
-    sweep_rr_body<Real, NU, ND, GPL>(s, st, blockIdx.x, sweep0, flags);
-}
-
-template <typename Real, int NU, int ND, int GPL>
-__global__ __launch_bounds__(kWave, 4) void k_sweep_rr_o4(DevSys s, DevState st,
-                                                          unsigned long long sweep0, int flags) {
+VMC_FMAC64 __global__ __launch_bounds__(kWave, (rr_sweep_waves<Real, NU, ND>())) void k_sweep_rr(
+    DevSys s, DevState st, unsigned long long sweep0, int flags) {
     sweep_rr_body<Real, NU, ND, GPL>(s, st, blockIdx.x, sweep0, flags);
 }
 
 // The same sweep with the caller's moves, recording each move (parity checks
 // of the timed move code).
 template <typename Real, int NU, int ND, int GPL>
-__global__ __launch_bounds__(kWave, (rr_sweep_waves<Real, NU, ND>())) void k_sweep_rr_given(
+VMC_FMAC64 __global__ __launch_bounds__(kWave, (rr_sweep_waves<Real, NU, ND>())) void k_sweep_rr_given(
     DevSys s, DevState st, int flags, SweepGiven given) {
     sweep_rr_body<Real, NU, ND, GPL, true>(s, st, blockIdx.x, 0, flags, given);
 }
@@ -1451,7 +1503,7 @@ __device__ __forceinline__ void measure_rr_body(const DevSys &s, const DevState 
     RRLane<Real, NMAX> L;
     const Real *inv_hbm = reinterpret_cast<const Real *>(st.inv) + (size_t)w * s.ninv;
     const double *gp = st.pos + (size_t)w * 3 * N;
-    rr_inverse_in<Real, NU, ND, NMAX>(inv_hbm, rr_stage(sh), L.inv, lane, h, r);
+    rr_inverse_in<Real, NU, ND, NMAX>(inv_hbm, sh.stage(), L.inv, lane, h, r);
     L.x = has_e ? gp[e] : 0.0;
     L.y = has_e ? gp[N + e] : 0.0;
     L.z = has_e ? gp[2 * N + e] : 0.0;
@@ -1770,7 +1822,7 @@ __global__ __launch_bounds__(kWave, ND > 0 ? 2 : 1) void k_measure_rr_mixed_b(co
 // sweep index comes from device memory (so a captured graph continues the
 // chains).  A system's chain is the same in a batch and alone.
 template <typename Real, int NU, int ND, int GPL>
-__global__ __launch_bounds__(kWave, (rr_sweep_waves<Real, NU, ND>())) void k_sweep_rr_b(
+VMC_FMAC64 __global__ __launch_bounds__(kWave, (rr_sweep_waves<Real, NU, ND>())) void k_sweep_rr_b(
     const BatchItem *__restrict__ items, int n_items,
                                                       const unsigned long long *__restrict__ sweep_ctr,
                                                       int flags) {
