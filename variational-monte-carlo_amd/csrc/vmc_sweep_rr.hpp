@@ -876,43 +876,32 @@ struct RRKernel {
         return pade(c, c.mi_r(xq, x), c.mi_r(yq, y), c.mi_r(zq, z), a);
     }
 
-    // Where a lane's orbital finds its axis phasors in Sh::pow: entry i step + first
-    // for move i (constants have step 0).
+    // Where a lane's orbital finds its axis phasors in Sh::pow: the entries for
+    // the next move, and how far on those of the move after it are (constants 0).
     struct PhasorAt {
-        int first[3], step[3];
+        int next[3], step[3];
         int sine;
     };
-    __device__ static void phasor_at(int lane, int h, int r, PhasorAt &at) {
+    __device__ static void phasor_at(const DevSys &s, int h, int r, PhasorAt &at) {
         static_assert(kMaxPow <= 1, "axis phasors are staged as first powers");
         constexpr int kOne = N * kRRPow;
-        at.sine = 0;
-        for (int k = 0; k < 3; ++k) {
-            at.first[k] = kOne;
-            at.step[k] = 0;
-        }
-#pragma unroll
-        for (int m = 0; m < NMAX; ++m) {
-            if (r != m) continue;
-            const int n[3] = {orb[m].x, orb[m].y, orb[m].z};
-            const int sine = orb[m].t;
-            at.sine = sine;
-            for (int k = 0; k < 3; ++k) {
-                // FP64 takes sin orbitals from the phasor -iX, FP32 as the imaginary part.
-                const int alt = k == 0 ? (sizeof(Real) == 8 ? sine : 0) : (n[k] < 0 ? 1 : 0);
-                if (n[k] != 0) {
-                    at.first[k] = (h && ND > 0 ? NU * kRRPow : 0) + 2 * k + alt;
-                    at.step[k] = kRRPow;
-                } else if (k == 0) {
-                    at.first[k] = kOne + alt;
-                }
-            }
-        }
+        const int4 o = s.orb[r < NU ? r : 0];
+        const int base = h && ND > 0 ? NU * kRRPow : 0;
+        at.sine = o.w;
+        // FP64 takes sine orbitals from the phasor -iX, FP32 as the imaginary part.
+        const int alt = sizeof(Real) == 8 ? o.w : 0;
+        at.next[0] = (o.x ? base : kOne) + alt;
+        at.next[1] = o.y ? base + (o.y < 0 ? 3 : 2) : kOne;
+        at.next[2] = o.z ? base + (o.z < 0 ? 5 : 4) : kOne;
+        at.step[0] = o.x ? kRRPow : 0;
+        at.step[1] = o.y ? kRRPow : 0;
+        at.step[2] = o.z ? kRRPow : 0;
     }
-    // The lane's orbital at its spin's proposal i.
-    __device__ static Real orbital(const Sh &sh, const PhasorAt &at, int i) {
-        const sf::Pair<Real> X = sh.pow[at.first[0] + i * at.step[0]];
-        const sf::Pair<Real> Y = sh.pow[at.first[1] + i * at.step[1]];
-        const sf::Pair<Real> Z = sh.pow[at.first[2] + i * at.step[2]];
+    // The lane's orbital at its spin's next proposal.
+    __device__ static Real orbital(const Sh &sh, PhasorAt &at) {
+        const sf::Pair<Real> X = sh.pow[at.next[0]], Y = sh.pow[at.next[1]], Z = sh.pow[at.next[2]];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) at.next[k] += at.step[k];
         const rr::Cx<Real> P = rr::cmul(rr::Cx<Real>{X.re, X.im}, rr::Cx<Real>{Y.re, Y.im});
         if constexpr (sizeof(Real) == 8) {
             return P.re * Z.re - P.im * Z.im;
@@ -985,11 +974,11 @@ struct RRKernel {
     // both outcomes (the one with the up proposal by the up electron's own
     // lane).  Same decisions and updates as two calls of move.  Returns the
     // number of accepted moves.
-    __device__ static int move_pair(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, const PhasorAt &at,
+    __device__ static int move_pair(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, PhasorAt &at,
                                     int lane, bool has_e, int h, int r, int i, LogDetTrack &ldt, double *rec) {
         static_assert(ND == NU, "paired moves need equal spins");
         const int lu = i, ld = 32 + i;
-        const Real phi = orbital(sh, at, i);
+        const Real phi = orbital(sh, at);
         const double *qu = sh.prop[lu], *qd = sh.prop[ld];
         const Real a_u = h == 0 ? c.a_same : c.a_anti, a_d = h == 1 ? c.a_same : c.a_anti;
         const bool mover = lane == lu;
@@ -1038,10 +1027,10 @@ struct RRKernel {
     }
 
     // One move of electron i of the only determinant.  Returns 1 if accepted.
-    __device__ static int move(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, const PhasorAt &at, int lane,
+    __device__ static int move(const RRConst<Real> &c, Sh &sh, RRLane<Real, NMAX> &L, PhasorAt &at, int lane,
                                bool has_e, int h, int r, int i, LogDetTrack &ldt, double *rec) {
         static_assert(ND == 0, "unpaired moves are the polarised system's");
-        const Real phi = orbital(sh, at, i);
+        const Real phi = orbital(sh, at);
         const double *q = sh.prop[i];
         Real un = pair_with(c, L.x, L.y, L.z, q[0], q[1], q[2], c.a_same);
         un = has_e && lane != i ? un : (Real)0;
@@ -1142,7 +1131,7 @@ __device__ __forceinline__ void sweep_rr_body(const DevSys &s, const DevState &s
         sh.misc[2] = st.logdet[2 * w + 1];
     }
     typename K::PhasorAt at;
-    K::phasor_at(lane, h, r, at);
+    K::phasor_at(s, h, r, at);
     __syncthreads();
     int since = st.since[w];
     if (s.reinv_k > 0 && since >= s.reinv_k) since = 0;  // re-inverted after the last sweep
