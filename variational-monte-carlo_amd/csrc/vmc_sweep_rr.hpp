@@ -206,6 +206,29 @@ __device__ __forceinline__ void dot_row16(Real &s0, Real &s1, Real p, const Real
     }
 }
 
+// g[k] = the values of v's lanes 16 k .. 16 k + 15 in every row of 16 lanes.
+__device__ __forceinline__ void swap_halves(float &a, float &b) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(p[0]);
+    b = __uint_as_float(p[1]);
+}
+__device__ __forceinline__ void swap_halves(double &a, double &b) {
+    const unsigned long long u = __double_as_longlong(a), v = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)v, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(v >> 32), false, false);
+    a = __longlong_as_double(((unsigned long long)hi[0] << 32) | lo[0]);
+    b = __longlong_as_double(((unsigned long long)hi[1] << 32) | lo[1]);
+}
+template <typename Real>
+__device__ __forceinline__ void spread_rows16(Real v, Real (&g)[4]) {
+    g[0] = g[1] = v;
+    swap_rows16(g[0], g[1]);  // rows 0 0 2 2 and 1 1 3 3
+    g[2] = g[0];
+    g[3] = g[1];
+    swap_halves(g[0], g[2]);
+    swap_halves(g[1], g[3]);
+}
+
 template <typename Real>
 struct Cx {
     Real re, im;
@@ -556,6 +579,54 @@ struct RRConst {
     }
 };
 
+// e^x for |x| < 100 within an ulp or two: x = k ln 2 + f and the Taylor series of
+// e^f in Horner form.  The accept test's rare exact branch: a loop without
+// constants of its own, so that nothing is kept in registers for it across the
+// moves (a call would keep the wave's state out of the caller-saved half).
+__device__ __forceinline__ double rr_exp_f64(double x) {
+    const double k = rint(x * 1.4426950408889634);
+    const double f = fma(-k, 2.3190468138462996e-17, fma(-k, 0.69314718055994531, x));
+    double e = 1.0;
+#pragma unroll 1
+    for (int n = 18; n > 0; --n) e = fma(f * e, rcp_nr((double)n), 1.0);
+    return ldexp(e, (int)k);
+}
+
+// Pade pair value a r / (1 + b r) of two points, as the moves form it.  In FP64
+// as a / (1/r + b): one inverse square root and one reciprocal (rsqrt_nr and
+// rcp_nr, 17 operations) instead of an IEEE root and division (50).
+template <typename Real>
+__device__ __forceinline__ Real pair_with(const RRConst<Real> &c, double x, double y, double z, double xq, double yq,
+                                          double zq, Real a) {
+    const Real dx = c.mi_r(xq, x), dy = c.mi_r(yq, y), dz = c.mi_r(zq, z);
+    if constexpr (sizeof(Real) == 8) {
+        const double r2 = fmax(fma(dx, dx, fma(dy, dy, dz * dz)), 1e-200);
+        return a * rcp_nr(rsqrt_nr(r2) + c.b);
+    } else {
+        const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
+        return a * rn * wrcp<Real>((Real)1 + c.b * rn);
+    }
+}
+
+// Metropolis test u < R^2 exp(2 dJ) (simulation.cpp:125-131).  The hardware
+// exp2 (relative error < 1e-6 here) decides unless u lies within 1e-5 of the
+// threshold, where the FP64 exponential decides, so the outcome equals the
+// FP64 comparison.  Inputs are wave-uniform; so is the result.
+__device__ __forceinline__ int accept_test(double R, double dj, double ua) {
+    const double r2 = R * R;
+    const float e32 = __builtin_amdgcn_exp2f((float)(2.0 * dj * 1.4426950408889634));
+    const double approx = r2 * (double)e32;
+    int acc;
+    if (!(approx == approx)) {
+        acc = 0;
+    } else if (fabs(ua - approx) > 1e-5 * approx || !(fabs(dj) < 40.0)) {
+        acc = ua < approx;
+    } else {
+        acc = ua < r2 * rr_exp_f64(2.0 * dj);
+    }
+    return wave_uniform(acc);
+}
+
 // In-LDS FP64 Gauss-Jordan inversion of the n x n matrix A (A = D^T on entry,
 // invT on exit) by the whole wave; returns log|det| or -inf below the
 // reference's pivot tolerance 1e-12 (matrix.hpp:35-39).
@@ -619,24 +690,6 @@ struct RRLane {
     double x, y, z;   // electron position
     double U;         // Jastrow row sum
 };
-
-__device__ __forceinline__ int orb_nx(int o) { return (o & 15) - 4; }
-__device__ __forceinline__ int orb_ny(int o) { return ((o >> 4) & 15) - 4; }
-__device__ __forceinline__ int orb_nz(int o) { return ((o >> 8) & 15) - 4; }
-__device__ __forceinline__ int orb_t(int o) { return o >> 12; }
-
-// e^x for |x| < 100 within an ulp or two: x = k ln 2 + f and the Taylor series of
-// e^f in Horner form.  The accept test's rare exact branch: a loop without
-// constants of its own, so that nothing is kept in registers for it across the
-// moves (a call would keep the wave's state out of the caller-saved half).
-__device__ __forceinline__ double rr_exp_f64(double x) {
-    const double k = rint(x * 1.4426950408889634);
-    const double f = fma(-k, 2.3190468138462996e-17, fma(-k, 0.69314718055994531, x));
-    double e = 1.0;
-#pragma unroll 1
-    for (int n = 18; n > 0; --n) e = fma(f * e, rcp_nr((double)n), 1.0);
-    return ldexp(e, (int)k);
-}
 
 template <typename Real, int NU, int ND, int GPL>
 struct RRKernel {
@@ -838,42 +891,6 @@ struct RRKernel {
         // Electron e sits in lane e (up) or 32 + e - NU (down).
         const auto pos_of = [&sh](int ax, int e) { return sh.pos[ax][e < NU ? e : 32 + e - NU]; };
         return rr::wave_total(sf::energy_cols<Real, N, kWave>(s, tab, lane, pos_of));
-    }
-
-    // Metropolis test u < R^2 exp(2 dJ) (simulation.cpp:125-131).  The
-    // hardware exp2 (relative error < 1e-6 here) decides unless u lies within
-    // 1e-5 of the threshold, where the exact FP64 exp decides, so the outcome
-    // equals the FP64 comparison.  Inputs are wave-uniform; so is the result.
-    __device__ static int accept_test(double R, double dj, double ua) {
-        const double r2 = R * R;
-        const float e32 = __builtin_amdgcn_exp2f((float)(2.0 * dj * 1.4426950408889634));
-        const double approx = r2 * (double)e32;
-        int acc;
-        if (!(approx == approx)) {
-            acc = 0;
-        } else if (fabs(ua - approx) > 1e-5 * approx || !(fabs(dj) < 40.0)) {
-            acc = ua < approx;
-        } else {
-            acc = ua < r2 * rr_exp_f64(2.0 * dj);
-        }
-        return wave_uniform(acc);
-    }
-
-    // Pade pair value a r / (1 + b r) at separation d.  In FP64 as
-    // a / (1/r + b): one inverse square root and one reciprocal (rsqrt_nr and
-    // rcp_nr, 17 operations) instead of an IEEE root and division (50).
-    __device__ static Real pade(const RRConst<Real> &c, Real dx, Real dy, Real dz, Real a) {
-        if constexpr (sizeof(Real) == 8) {
-            const double r2 = fmax(fma(dx, dx, fma(dy, dy, dz * dz)), 1e-200);
-            return a * rcp_nr(rsqrt_nr(r2) + c.b);
-        } else {
-            const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-            return a * rn * wrcp<Real>((Real)1 + c.b * rn);
-        }
-    }
-    __device__ static Real pair_with(const RRConst<Real> &c, double x, double y, double z, double xq, double yq,
-                                     double zq, Real a) {
-        return pade(c, c.mi_r(xq, x), c.mi_r(yq, y), c.mi_r(zq, z), a);
     }
 
     // Where a lane's orbital finds its axis phasors in Sh::pow: the entries for

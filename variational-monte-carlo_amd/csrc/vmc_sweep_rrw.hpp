@@ -5,16 +5,23 @@
 // (wave v, lane l) owns row r = (v mod WPS) * 64 + l of spin h = v / WPS:
 // that electron's position, its Jastrow row sum U and its row of the spin's
 // transposed inverse in registers.  A move of electron p (spin hp) is three
-// phases, A and B separated by a workgroup barrier only when a spin spans
-// several wavefronts, B and C always:
+// phases with one workgroup barrier, between B and C:
 //   A  every thread forms its new pair term against the proposal (DPP wave
-//      sum -> LDS); the rows of spin hp form the orbital row of the proposal;
-//   B  spin hp's rows form s_k = sum_m phi_m invT[k][m]; the mover publishes
+//      sum -> LDS);
+//   B  spin hp's rows form s_k = sum_m phi_m invT[k][m]: each of its
+//      wavefronts forms the orbital row for itself from the staged powers of the
+//      axis phasors and broadcasts it within the FMA (DPP); the mover publishes
 //      R = s_p, its U, old position and inverse row;
 //   C  every thread takes the same accept decision from the same LDS values;
 //      on accept spin hp's rows apply Sherman-Morrison (one FMA per element,
 //      the other spin's wavefronts skip it on a wave-uniform branch) and every
 //      thread updates its U.
+// What bounds it: the move's chain and VALU instructions (506 instead of 589
+// in the FP32 loop at 57 per spin).  With the orbital row through LDS, a
+// second barrier where a spin spans wavefronts, powers selected per move and, in FP64,
+// IEEE roots and divisions: FP64 sweeps 202 -> 163 us at 57 per spin and 113 ->
+// 87 at 33 (tens of walkers), FP32 285 -> 273 at 57 (2048 walkers) and, 1000
+// walkers and more in a batch, 1878 -> 1657 at 81 per spin and 821 -> 744 at 33.
 // Same chain as the one-wavefront kernel (the reference's
 // src/simulation/simulation.cpp:80-156 with per-sweep electron order and
 // Philox draws), same HBM layout, so ensembles switch kernels freely.
@@ -24,24 +31,29 @@
 
 namespace vmc {
 
+__device__ __forceinline__ float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 template <typename Real, int NU, int ND, int WPS>
 struct RRWShared {
     static constexpr int N = NU + ND;
     static constexpr int NMAX = NU > ND ? NU : ND;
     static constexpr int NWAVE = (ND > 0 ? 2 : 1) * WPS;
-    double pos[3][N];
-    alignas(16) double prop[4][N];  // this sweep's proposals (x, y, z) and accept uniforms
-    Real pph[6][N];      // axis phasors of the proposals
+    static constexpr int kMaxC = rr::max_component<NMAX>();
+    // Axis-phasor entries of one electron's proposal: 1, X .. X^kMaxC, Y .., Z ..
+    static constexpr int kPow = 1 + 3 * kMaxC;
+    double pos[3][N];               // at the start of the sweep
+    alignas(16) double prop[N][4];  // this sweep's proposals x, y, z and accept uniforms
+    alignas(16) sf::Pair<Real> pow[N][kPow];
     // Rows padded to 16 bytes, so that a row picked at run time still moves
     // with 16-byte LDS reads.
     static constexpr int kRowPad = (NMAX + 3) / 4 * 4;
-    alignas(16) Real phi[2][kRowPad];   // orbital rows of the pending moves (by spin)
     alignas(16) Real row[2][kRowPad];   // inverse row of the (up) mover (by move parity)
     alignas(16) Real row2[2][kRowPad];  // inverse row of the down mover of a paired move
     double jred[2][NWAVE];   // per-wave new Jastrow pair sums (by move parity)
     double jred2[2][NWAVE];  // the same for the down proposal of a paired move
-    double mv[2][8];     // (up) mover: R, U, x, y, z (by move parity)
-    double mv2[2][8];    // down mover of a paired move
+    alignas(16) double mv[2][8];   // (up) mover: R, U, x, y, z (by move parity)
+    alignas(16) double mv2[2][8];  // down mover of a paired move
     double stat[kStatCount];
     double misc[4];      // sigma, log|det| up, log|det| down
 };
@@ -52,12 +64,11 @@ struct RRW {
     static constexpr int NMAX = NU > ND ? NU : ND;
     static constexpr int NWAVE = (ND > 0 ? 2 : 1) * WPS;
     static constexpr int NT = NWAVE * kWave;
-    static constexpr auto orb = rr::shell_orbitals<NMAX>();
     using Sh = RRWShared<Real, NU, ND, WPS>;
     static_assert(ND == 0 || ND == NU, "polarised or equal spins");
     static_assert(NMAX <= WPS * kWave, "rows per spin exceed the spin's wavefronts");
-    static constexpr int kMaxC = rr::max_component<NMAX>();
-    static constexpr bool kOneBarrier = WPS == 1 && NMAX >= 57;
+    static constexpr int kMaxC = Sh::kMaxC;
+    static constexpr int kGroups = (NMAX + kWave - 1) / kWave;  // orbitals of a lane
     // Sizes whose sweep moves an up and a down electron per pass (move_pair):
     // measured faster there; at 81 and 123 per spin in FP32 (and 33, 57 in
     // FP64) the paired pass's registers cost more than it saves.
@@ -65,29 +76,48 @@ struct RRW {
                                                                   : NMAX == 81);
     static_assert(kMaxC <= 3, "orbital phasors use powers up to 3");
 
-    // e^{2 pi i n.u} from the axis phasors a and their powers.
-    __device__ static rr::Cx<Real> phasor(int nx, int ny, int nz, const rr::Cx<Real> a[3]) {
-        rr::Cx<Real> a2[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) a2[k] = rr::cmul(a[k], a[k]);
-        if constexpr (kMaxC <= 2) {
-            return rr::orbital_phasor<Real>(nx, ny, nz, a, a2);
-        } else {
-            rr::Cx<Real> a3[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) a3[k] = rr::cmul(a2[k], a[k]);
-            return rr::orbital_phasor3<Real>(nx, ny, nz, a, a2, a3);
-        }
+    // Orbital m: its entries in Sh::pow (x | y << 4 | z << 8), the signs of its
+    // y and z components (bits 31 and 30) and its type (bit 12).
+    __device__ static int packed_orbital(const DevSys &s, int m) {
+        const int4 o = s.orb[m < NU ? m : 0];
+        const int ay = o.y < 0 ? -o.y : o.y, az = o.z < 0 ? -o.z : o.z;
+        const int x = o.x, y = ay ? kMaxC + ay : 0, z = az ? 2 * kMaxC + az : 0;
+        return x | (y << 4) | (z << 8) | (o.w << 12) | (o.y < 0 ? (int)0x80000000 : 0) | (o.z < 0 ? 0x40000000 : 0);
     }
-
-    // Orbital r of the compile-time table, packed (nx+4) | (ny+4)<<4 |
-    // (nz+4)<<8 | type<<12 (selected once per kernel).
-    __device__ static int packed_orbital(int r) {
-        int o = 0;
-#pragma unroll
-        for (int m = 0; m < NMAX; ++m)
-            if (r == m) o = (orb[m].x + 4) | ((orb[m].y + 4) << 4) | ((orb[m].z + 4) << 8) | (orb[m].t << 12);
-        return o;
+    __device__ static float flip(float v, int sign) { return __int_as_float(__float_as_int(v) ^ (sign & (int)0x80000000)); }
+    __device__ static double flip(double v, int sign) {
+        return __longlong_as_double(__double_as_longlong(v) ^ ((long long)(sign & (int)0x80000000) << 32));
+    }
+    // Packed orbital ob at proposal p.
+    __device__ static Real orbital(const Sh &sh, int ob, int p) {
+        const sf::Pair<Real> *t = sh.pow[p];
+        const sf::Pair<Real> X = t[ob & 15], Y = t[(ob >> 4) & 15], Z = t[(ob >> 8) & 15];
+        // (which products are rounded and which fused is part of the FP32
+        // chain, so it is written out)
+        const Real yi = flip(Y.im, ob), zi = flip(Z.im, ob << 1);
+        const Real re = fma_r(X.re, Y.re, -(X.im * yi));
+        const Real im = kMaxC <= 2 ? fma_r(X.im, Y.re, X.re * yi) : fma_r(X.re, yi, X.im * Y.re);
+        return ob & 0x1000 ? fma_r(im, Z.re, re * zi) : fma_r(re, Z.re, -(im * zi));
+    }
+    // s_k = sum_m phi_m(proposal p) invT[k][m] for the thread's row k: every
+    // wavefront forms the whole orbital row, lane l orbitals l, 64 + l, ...,
+    // and the FMA itself broadcasts them from its row of 16 lanes; even and
+    // odd m in two sums.
+    __device__ static Real ratio_row(const Sh &sh, const int (&ob)[kGroups], int p, const Real (&inv)[NMAX]) {
+        Real s0 = (Real)0, s1 = (Real)0;
+        const auto group = [&]<int g>() {
+            constexpr int m0 = g * kWave;
+            Real v[4];
+            rr::spread_rows16(orbital(sh, ob[g], p), v);
+            rr::dot_row16<NMAX, m0>(s0, s1, v[0], inv);
+            if constexpr (NMAX > m0 + 16) rr::dot_row16<NMAX, m0 + 16>(s0, s1, v[1], inv);
+            if constexpr (NMAX > m0 + 32) rr::dot_row16<NMAX, m0 + 32>(s0, s1, v[2], inv);
+            if constexpr (NMAX > m0 + 48) rr::dot_row16<NMAX, m0 + 48>(s0, s1, v[3], inv);
+        };
+        group.template operator()<0>();
+        if constexpr (kGroups > 1) group.template operator()<1>();
+        if constexpr (kGroups > 2) group.template operator()<2>();
+        return s0 + s1;
     }
 
     struct Thread {
@@ -145,30 +175,6 @@ struct RRW {
         return U;
     }
 
-    // Pade pair value of the point (xn, yn, zn) with (x, y, z), as the moves
-    // form it.
-    __device__ static Real pair_at(const RRConst<Real> &c, double xn, double yn, double zn, double x, double y,
-                                   double z, Real a) {
-        const Real dx = c.mi_r(xn, x);
-        const Real dy = c.mi_r(yn, y);
-        const Real dz = c.mi_r(zn, z);
-        const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-        return a * rn * wrcp<Real>((Real)1 + c.b * rn);
-    }
-
-    // Metropolis test (simulation.cpp:125-131), exact FP64 exponential within
-    // 1e-5 of the threshold; wave-uniform inputs and result.
-    __device__ static int accept_test(double R, double dj, double ua) {
-        const double r2 = R * R;
-        const float e32 = __builtin_amdgcn_exp2f((float)(2.0 * dj * 1.4426950408889634));
-        const double approx = r2 * (double)e32;
-        int acc;
-        if (!(approx == approx)) acc = 0;
-        else if (fabs(ua - approx) > 1e-5 * approx || !(fabs(dj) < 40.0)) acc = ua < approx;
-        else acc = ua < r2 * rr_exp_f64(2.0 * dj);
-        return wave_uniform(acc);
-    }
-
     // The moves of up electron i and then down electron i (the sweep order
     // of equal spins) in one pass: each spin's wavefronts form their orbital
     // row and ratios at their spin's proposal, and every thread forms its pair
@@ -177,53 +183,33 @@ struct RRW {
     // the down electron, formed as the threads form them).  Same decisions
     // and updates as two calls of move.  Returns the accepted moves.
     __device__ static int move_pair(const RRConst<Real> &c, Sh &sh, const Thread &T, Real (&inv)[NMAX],
-                                    double &x, double &y, double &z, double &U, int ob, int i, int par,
+                                    double &x, double &y, double &z, double &U, const int (&ob)[kGroups], int i, int par,
                                     LogDetTrack &ldt, double *rec) {
         static_assert(ND == NU, "paired moves need equal spins");
         const int pu = i, pd = NU + i;
-        const double xu = sh.prop[0][pu], yu = sh.prop[1][pu], zu = sh.prop[2][pu];
-        const double xd = sh.prop[0][pd], yd = sh.prop[1][pd], zd = sh.prop[2][pd];
+        const double xu = sh.prop[pu][0], yu = sh.prop[pu][1], zu = sh.prop[pu][2];
+        const double xd = sh.prop[pd][0], yd = sh.prop[pd][1], zd = sh.prop[pd][2];
         // Phase A.
-        if (T.has_e) {
-            const int pp = T.h ? pd : pu;
-            rr::Cx<Real> a[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                a[k].re = sh.pph[2 * k][pp];
-                a[k].im = sh.pph[2 * k + 1][pp];
-            }
-            const rr::Cx<Real> q = phasor(orb_nx(ob), orb_ny(ob), orb_nz(ob), a);
-            sh.phi[T.h][T.r] = orb_t(ob) ? q.im : q.re;
-        }
         Real un_u = (Real)0, un_d = (Real)0;
-        if (T.has_e && T.e != pu) un_u = pair_at(c, xu, yu, zu, x, y, z, T.h == 0 ? c.a_same : c.a_anti);
-        if (T.has_e && T.e != pd) un_d = pair_at(c, xd, yd, zd, x, y, z, T.h == 1 ? c.a_same : c.a_anti);
-        {
+        if (T.has_e && T.e != pu) un_u = pair_with(c, x, y, z, xu, yu, zu, T.h == 0 ? c.a_same : c.a_anti);
+        if (T.has_e && T.e != pd) un_d = pair_with(c, x, y, z, xd, yd, zd, T.h == 1 ? c.a_same : c.a_anti);
+        if constexpr (sizeof(Real) == 8) {
+            double wu, wd;
+            rr::wave_totals(un_u, un_d, wu, wd);
+            if (T.lane == 0) {
+                sh.jred[par][T.v] = wu;
+                sh.jred2[par][T.v] = wd;
+            }
+        } else {
             const Real wu = rr::wave_total(un_u), wd = rr::wave_total(un_d);
             if (T.lane == 0) {
                 sh.jred[par][T.v] = (double)wu;
                 sh.jred2[par][T.v] = (double)wd;
             }
         }
-        if constexpr (kOneBarrier) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        } else {
-            __syncthreads();
-        }
         // Phase B: every thread's s_k with its spin's orbital row; the two
         // movers publish their values and rows.
-        Real sk;
-        {
-            Real s0 = 0, s1 = 0;
-#pragma unroll
-            for (int m = 0; m < NMAX; m += 2) {
-                s0 += sh.phi[T.h][m] * inv[m];
-                if (m + 1 < NMAX) s1 += sh.phi[T.h][m + 1] * inv[m + 1];
-            }
-            sk = s0 + s1;
-        }
+        const Real sk = ratio_row(sh, ob, T.h ? pd : pu, inv);
         if (T.r == i) {
             double *mvp = T.h ? sh.mv2[par] : sh.mv[par];
             Real *rowp = T.h ? sh.row2[par] : sh.row[par];
@@ -235,27 +221,18 @@ struct RRW {
 #pragma unroll
             for (int m = 0; m < NMAX; ++m) rowp[m] = inv[m];
         }
-        double jn_u = 0.0, jn_d = 0.0;
-        if constexpr (!kOneBarrier) {
-#pragma unroll
-            for (int v = 0; v < NWAVE; ++v) {
-                jn_u += sh.jred[par][v];
-                jn_d += sh.jred2[par][v];
-            }
-        }
         __syncthreads();
-        if constexpr (kOneBarrier) {
+        double jn_u = 0.0, jn_d = 0.0;
 #pragma unroll
-            for (int v = 0; v < NWAVE; ++v) {
-                jn_u += sh.jred[par][v];
-                jn_d += sh.jred2[par][v];
-            }
+        for (int v = 0; v < NWAVE; ++v) {
+            jn_u += sh.jred[par][v];
+            jn_d += sh.jred2[par][v];
         }
         // Phase C, up move.
         const double Ru = sh.mv[par][0];
         const double uxo = sh.mv[par][2], uyo = sh.mv[par][3], uzo = sh.mv[par][4];
         const double dj_u = jn_u - sh.mv[par][1];
-        const int acc_u = accept_test(Ru, dj_u, sh.prop[3][pu]);
+        const int acc_u = accept_test(Ru, dj_u, sh.prop[pu][3]);
         double Ud = sh.mv2[par][1];
         if (acc_u) {
             ldt.add(0, Ru);
@@ -267,30 +244,29 @@ struct RRW {
                 for (int m = 0; m < NMAX; ++m) inv[m] -= sh.row[par][m] * f;
             }
             if (T.has_e && T.e != pu)
-                U += (double)un_u - (double)pair_at(c, uxo, uyo, uzo, x, y, z, T.h == 0 ? c.a_same : c.a_anti);
+                U += (double)un_u - (double)pair_with(c, x, y, z, uxo, uyo, uzo, T.h == 0 ? c.a_same : c.a_anti);
             if (T.has_e && T.e == pu) {
                 U = jn_u;
                 x = xu;
                 y = yu;
                 z = zu;
-                sh.pos[0][pu] = xu;
-                sh.pos[1][pu] = yu;
-                sh.pos[2][pu] = zu;
             }
             // The down mover's row sum after this update, and the down
-            // proposal's pair with the up electron where it now is.
-            const double dxo = sh.mv2[par][2], dyo = sh.mv2[par][3], dzo = sh.mv2[par][4];
-            Ud += (double)pair_at(c, xu, yu, zu, dxo, dyo, dzo, c.a_anti) -
-                  (double)pair_at(c, uxo, uyo, uzo, dxo, dyo, dzo, c.a_anti);
-            const Real ud_new = pair_at(c, xd, yd, zd, xu, yu, zu, c.a_anti);
-            const Real ud_old = pair_at(c, xd, yd, zd, uxo, uyo, uzo, c.a_anti);
+            // proposal's pair with the up electron where it now is: the up
+            // electron's new and old place with the down mover and with the
+            // down proposal, one of the four pairs in each lane of four.
+            const double *up = T.lane & 1 ? &sh.mv[par][2] : &sh.prop[pu][0];
+            const double *dn = T.lane & 2 ? &sh.prop[pd][0] : &sh.mv2[par][2];
+            const Real four = pair_with(c, dn[0], dn[1], dn[2], up[0], up[1], up[2], c.a_anti);
+            Ud += (double)rr::readlane(four, 0) - (double)rr::readlane(four, 1);
+            const Real ud_new = rr::readlane(four, 2), ud_old = rr::readlane(four, 3);
             jn_d += (double)ud_new - (double)ud_old;
             if (T.has_e && T.e == pu) un_d = ud_new;
         }
         // Phase C, down move.
         const double Rd = sh.mv2[par][0];
         const double dj_d = jn_d - Ud;
-        const int acc_d = accept_test(Rd, dj_d, sh.prop[3][pd]);
+        const int acc_d = accept_test(Rd, dj_d, sh.prop[pd][3]);
         if (rec && threadIdx.x == 0) {
             double *ru = rec + kTraceCount * pu, *rd = rec + kTraceCount * pd;
             ru[0] = Ru;
@@ -311,15 +287,12 @@ struct RRW {
             }
             const double dxo = sh.mv2[par][2], dyo = sh.mv2[par][3], dzo = sh.mv2[par][4];
             if (T.has_e && T.e != pd)
-                U += (double)un_d - (double)pair_at(c, dxo, dyo, dzo, x, y, z, T.h == 1 ? c.a_same : c.a_anti);
+                U += (double)un_d - (double)pair_with(c, x, y, z, dxo, dyo, dzo, T.h == 1 ? c.a_same : c.a_anti);
             if (T.has_e && T.e == pd) {
                 U = jn_d;
                 x = xd;
                 y = yd;
                 z = zd;
-                sh.pos[0][pd] = xd;
-                sh.pos[1][pd] = yd;
-                sh.pos[2][pd] = zd;
             }
         }
         return acc_u + acc_d;
@@ -328,60 +301,28 @@ struct RRW {
     // One move of electron p, the sweep's move number par (mod 2) selecting
     // the LDS buffers phase C reads.  Returns 1 if accepted (uniform).
     __device__ static int move(const RRConst<Real> &c, Sh &sh, const Thread &T, Real (&inv)[NMAX],
-                               double &x, double &y, double &z, double &U, int ob, int p, int par,
+                               double &x, double &y, double &z, double &U, const int (&ob)[kGroups], int p, int par,
                                LogDetTrack &ldt, double *rec) {
         const int hp = (ND > 0 && p >= NU) ? 1 : 0;
         const int rp = hp ? p - NU : p;
-        const int NP = hp ? ND : NU;
         // Phase A.
-        const double xn = sh.prop[0][p], yn = sh.prop[1][p], zn = sh.prop[2][p];
-        if (T.h == hp && T.has_e) {
-            rr::Cx<Real> a[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                a[k].re = sh.pph[2 * k][p];
-                a[k].im = sh.pph[2 * k + 1][p];
-            }
-            const rr::Cx<Real> q = phasor(orb_nx(ob), orb_ny(ob), orb_nz(ob), a);
-            sh.phi[hp][T.r] = orb_t(ob) ? q.im : q.re;
-        }
+        const double xn = sh.prop[p][0], yn = sh.prop[p][1], zn = sh.prop[p][2];
+        const Real apair = T.h == hp ? c.a_same : c.a_anti;
         Real un = (Real)0;
-        if (T.has_e && T.e != p) {
-            const Real dx = c.mi_r(xn, x);
-            const Real dy = c.mi_r(yn, y);
-            const Real dz = c.mi_r(zn, z);
-            const Real rn = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-            const Real a = (T.h == hp) ? c.a_same : c.a_anti;
-            un = a * rn * wrcp<Real>((Real)1 + c.b * rn);
-        }
+        if (T.has_e && T.e != p) un = pair_with(c, x, y, z, xn, yn, zn, apair);
         {
             const Real ws = rr::wave_total(un);
             if (T.lane == 0) sh.jred[par][T.v] = (double)ws;
         }
-        // With one wavefront per spin the orbital row is written and read by
-        // the mover's wavefront alone, in issue order: phases A and B need no
-        // workgroup barrier between them (used from 57 per spin; at 33 the
-        // pair sums read after the one barrier cost more than the barrier).  The mover's values and the pair
-        // sums that phase C reads alternate between two buffers by move
+        // Each of the mover's wavefronts forms the orbital row for itself, so
+        // one workgroup barrier serves a move.  The mover's values and the
+        // pair sums that phase C reads alternate between two buffers by move
         // parity, so a wavefront already in the next move's phase A or B
         // cannot overwrite what a slower one still reads.
-        if constexpr (kOneBarrier) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        } else {
-            __syncthreads();
-        }
         // Phase B.
         Real sk = (Real)0;
         if (T.h == hp) {
-            Real s0 = 0, s1 = 0;
-#pragma unroll
-            for (int m = 0; m < NMAX; m += 2) {
-                s0 += sh.phi[hp][m] * inv[m];
-                if (m + 1 < NMAX) s1 += sh.phi[hp][m + 1] * inv[m + 1];
-            }
-            sk = s0 + s1;
+            sk = ratio_row(sh, ob, p, inv);
             if (T.r == rp) {
                 sh.mv[par][0] = (double)sk;
                 sh.mv[par][1] = U;
@@ -392,31 +333,16 @@ struct RRW {
                 for (int m = 0; m < NMAX; ++m) sh.row[par][m] = inv[m];
             }
         }
-        // The pair sums: complete since the first barrier when there is one
-        // (read before the second, off phase C's path), else after this one.
-        double jn = 0.0;
-        if constexpr (!kOneBarrier) {
-#pragma unroll
-            for (int i = 0; i < NWAVE; ++i) jn += sh.jred[par][i];
-        }
         __syncthreads();
-        if constexpr (kOneBarrier) {
+        double jn = 0.0;
 #pragma unroll
-            for (int i = 0; i < NWAVE; ++i) jn += sh.jred[par][i];
-        }
+        for (int i = 0; i < NWAVE; ++i) jn += sh.jred[par][i];
         // Phase C: the same decision in every thread (simulation.cpp:125-131),
         // exact FP64 exponential within 1e-5 of the threshold.
         const double R = sh.mv[par][0];
         const double dj = jn - sh.mv[par][1];
-        const double ua = sh.prop[3][p];
-        const double r2 = R * R;
-        const float e32 = __builtin_amdgcn_exp2f((float)(2.0 * dj * 1.4426950408889634));
-        const double approx = r2 * (double)e32;
-        int acc;
-        if (!(approx == approx)) acc = 0;
-        else if (fabs(ua - approx) > 1e-5 * approx || !(fabs(dj) < 40.0)) acc = ua < approx;
-        else acc = ua < r2 * rr_exp_f64(2.0 * dj);
-        acc = wave_uniform(acc);
+        const double ua = sh.prop[p][3];
+        const int acc = accept_test(R, dj, ua);
         if (rec && threadIdx.x == 0) {
             double *q = rec + kTraceCount * p;
             q[0] = R;
@@ -432,47 +358,43 @@ struct RRW {
 #pragma unroll
             for (int m = 0; m < NMAX; ++m) inv[m] -= sh.row[par][m] * f;
         }
-        if (T.has_e && T.e != p) {
-            const Real dx = c.mi_r(sh.mv[par][2], x);
-            const Real dy = c.mi_r(sh.mv[par][3], y);
-            const Real dz = c.mi_r(sh.mv[par][4], z);
-            const Real ro = wsqrt<Real>(dx * dx + dy * dy + dz * dz);
-            const Real a = (T.h == hp) ? c.a_same : c.a_anti;
-            U += (double)un - (double)(a * ro * wrcp<Real>((Real)1 + c.b * ro));
-        }
+        if (T.has_e && T.e != p)
+            U += (double)un - (double)pair_with(c, x, y, z, sh.mv[par][2], sh.mv[par][3], sh.mv[par][4], apair);
         if (T.has_e && T.e == p) {
             U = jn;
             x = xn;
             y = yn;
             z = zn;
-            sh.pos[0][p] = xn;
-            sh.pos[1][p] = yn;
-            sh.pos[2][p] = zn;
         }
-        (void)NP;
         return 1;
     }
 };
 
-// Proposal q (in [0, L)) of electron e, its axis phasors and accept uniform
-// ua into the electron's slots.
-template <typename Real>
-__device__ __forceinline__ void rrw_stage_proposal(const DevSys &s, const double (&q)[3], double ua, int e, int N,
-                                                   double *prop, Real *pph) {
+// Proposal q (in [0, L)) of electron e, its axis phasors' powers and accept
+// uniform ua into the electron's slots.
+template <typename Real, typename Sh>
+__device__ __forceinline__ void rrw_stage_proposal(const DevSys &s, const double (&q)[3], double ua, int e, Sh &sh) {
+    sf::Pair<Real> *t = sh.pow[e];
+    t[0] = {(Real)1, (Real)0};
     for (int k = 0; k < 3; ++k) {
-        prop[k * N + e] = q[k];
-        const rr::Cx<Real> ph = rr::axis_phasor<Real>(q[k], s.inv_L);
-        pph[(2 * k) * N + e] = ph.re;
-        pph[(2 * k + 1) * N + e] = ph.im;
+        sh.prop[e][k] = q[k];
+        const rr::Cx<Real> a = rr::axis_phasor<Real>(q[k], s.inv_L);
+        t[1 + k * Sh::kMaxC] = {a.re, a.im};
+        if constexpr (Sh::kMaxC >= 2) {
+            const Real c = a.re * a.im;
+            const rr::Cx<Real> a2{fma_r(a.re, a.re, -(a.im * a.im)), c + c};
+            t[2 + k * Sh::kMaxC] = {a2.re, a2.im};
+            if constexpr (Sh::kMaxC >= 3)
+                t[3 + k * Sh::kMaxC] = {fma_r(a.re, a2.re, -(a.im * a2.im)), fma_r(a.re, a2.im, a.im * a2.re)};
+        }
     }
-    prop[3 * N + e] = ua;
+    sh.prop[e][3] = ua;
 }
 
 // Philox draws of one electron for this sweep into its proposal slots.
-template <typename Real>
-__device__ __forceinline__ void rrw_proposal(const DevSys &s, double sigma, double x0, double y0,
-                                             double z0, int e, int w, uint32_t sweep, int N,
-                                             double *prop, Real *pph) {
+template <typename Real, typename Sh>
+__device__ __forceinline__ void rrw_proposal(const DevSys &s, double sigma, double x0, double y0, double z0, int e,
+                                             int w, uint32_t sweep, Sh &sh) {
     const uint4 rm = philox4x32_10(make_uint4((uint32_t)e, (uint32_t)w, sweep, kTagMove), s.key0, s.key1);
     const uint4 ra = philox4x32_10(make_uint4((uint32_t)e, (uint32_t)w, sweep, kTagAccept), s.key0, s.key1);
     double dx, dy, dz;
@@ -493,7 +415,7 @@ __device__ __forceinline__ void rrw_proposal(const DevSys &s, double sigma, doub
     const double x = x0 + sigma * dx, y = y0 + sigma * dy, z = z0 + sigma * dz;
     const double q[3] = {x - s.L * floor(x * s.inv_L), y - s.L * floor(y * s.inv_L),
                          z - s.L * floor(z * s.inv_L)};
-    rrw_stage_proposal<Real>(s, q, u01(ra.x), e, N, prop, pph);
+    rrw_stage_proposal<Real>(s, q, u01(ra.x), e, sh);
 }
 
 // kGiven: the moves come from the caller (SweepGiven) instead of Philox and
@@ -524,18 +446,20 @@ __device__ __forceinline__ void sweep_rrw_body(const DevSys &s, const DevState &
         U = K::jastrow_row(cst, sh, T, x, y, z);
     else
         U = T.has_e ? st.jrow[(size_t)w * N + T.e] : 0.0;
-    const int ob = K::packed_orbital(T.r);
+    int ob[K::kGroups];
+#pragma unroll
+    for (int g = 0; g < K::kGroups; ++g) ob[g] = K::packed_orbital(s, g * kWave + T.lane);
     double *rec = nullptr;
     if constexpr (kGiven) {
         if (T.has_e) {
             const size_t q = (size_t)w * N + T.e;
             const double p3[3] = {given.prop[3 * q], given.prop[3 * q + 1], given.prop[3 * q + 2]};
-            rrw_stage_proposal<Real>(s, p3, given.u[q], T.e, N, &sh.prop[0][0], &sh.pph[0][0]);
+            rrw_stage_proposal<Real>(s, p3, given.u[q], T.e, sh);
         }
         rec = given.trace + (size_t)w * N * kTraceCount;
     } else {
         if (T.has_e)
-            rrw_proposal<Real>(s, sh.misc[0], x, y, z, T.e, w, (uint32_t)sweep0, N, &sh.prop[0][0], &sh.pph[0][0]);
+            rrw_proposal<Real>(s, sh.misc[0], x, y, z, T.e, w, (uint32_t)sweep0, sh);
     }
     __syncthreads();
     int acc = 0;
@@ -603,7 +527,7 @@ constexpr int rrw_sweep_waves() {
 }
 
 template <typename Real, int NU, int ND, int WPS>
-__global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real, NU, ND, WPS>())) void k_sweep_rrw(DevSys s, DevState st,
+VMC_FMAC64 __global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real, NU, ND, WPS>())) void k_sweep_rrw(DevSys s, DevState st,
                                                                           unsigned long long sweep0,
                                                                           int flags) {
     sweep_rrw_body<Real, NU, ND, WPS>(s, st, blockIdx.x, sweep0, flags);
@@ -612,14 +536,14 @@ __global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real,
 // The sweep with the caller's moves, each recorded (parity checks of the
 // timed move code).
 template <typename Real, int NU, int ND, int WPS>
-__global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real, NU, ND, WPS>())) void k_sweep_rrw_given(
+VMC_FMAC64 __global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real, NU, ND, WPS>())) void k_sweep_rrw_given(
     DevSys s, DevState st, int flags, SweepGiven given) {
     sweep_rrw_body<Real, NU, ND, WPS, true>(s, st, blockIdx.x, 0, flags, given);
 }
 
 // Batch forms over a group of systems of one size (as k_sweep_rr_b).
 template <typename Real, int NU, int ND, int WPS>
-__global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real, NU, ND, WPS>())) void k_sweep_rrw_b(
+VMC_FMAC64 __global__ __launch_bounds__((ND > 0 ? 2 : 1) * WPS * 64, (rrw_sweep_waves<Real, NU, ND, WPS>())) void k_sweep_rrw_b(
     const BatchItem *__restrict__ items, int n_items, const unsigned long long *__restrict__ sweep_ctr,
     int flags) {
     const BatchItem &it = items[batch_find(items, n_items, blockIdx.x)];
