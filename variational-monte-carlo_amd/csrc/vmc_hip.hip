@@ -836,7 +836,7 @@ namespace {
 template <typename Real>
 int launch_init(vmc_ensemble *e, int draw, const double *aos, hipStream_t stream) {
     const DevSys &d = e->tables.dev;
-    const bool fast = init_fast(d, e->st, draw, aos, static_cast<int>(sizeof(Real)), stream);
+    const bool fast = sizeof(Real) == 8 && init_fast(d, e->st, draw, aos, stream);
     const size_t lds = lds_for(d, sizeof(Real), false);
     hipLaunchKernelGGL((k_init<Real>), dim3(static_cast<unsigned>(e->W)), dim3(kWave), lds, stream,
                        d, e->st, draw, fast ? 1 : 0);
@@ -1218,7 +1218,7 @@ int vmc_ensemble_set_positions(vmc_ensemble *e, const double *pos, void *stream)
     const size_t nmax2 = static_cast<size_t>(e->tables.dev.nmax) * e->tables.dev.nmax;
     std::vector<double> soa;
     const double *aos = nullptr;
-    if (e->tables.dev.nmax <= kInitFastMax && nmax2 >= static_cast<size_t>(3 * N)) {
+    if (e->tables.real_bytes == 8 && e->tables.dev.nmax <= kInitFastMax && nmax2 >= static_cast<size_t>(3 * N)) {
         VMC_HIP_TRY(hipMemcpyAsync(e->st.scratch, pos, sizeof(double) * W * 3 * N, hipMemcpyHostToDevice, s));
         aos = e->st.scratch;
     } else {

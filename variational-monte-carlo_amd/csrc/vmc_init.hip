@@ -16,6 +16,9 @@
 // per spin, 554 us for 1000 at 81, 2.2 ms for 1024 at 147; one wavefront per
 // walker with the matrix in memory took 435 us at 33 and 42.6 ms at 147.  Above
 // 160 a lane's row no longer fits its registers.
+// FP64 inverses only: the elimination rounds in another order than k_init's, which
+// moves about one FP32 element in a million by its last place, and an FP32 chain
+// turns that into another accept decision now and then.
 #include "../../include/vmc_hip.h"
 #include "vmc_device.hpp"
 #include "vmc_rr_launch.hpp"
@@ -88,7 +91,7 @@ __device__ __forceinline__ double in_quad(double v) {
 }
 
 // C: columns of a lane, n <= 4 C rows and columns, 16 C threads.
-template <typename Real, int C>
+template <int C>
 __global__ __launch_bounds__(16 * C < 64 ? 64 : 16 * C) void k_invert(DevSys s, DevState st) {
     constexpr int NT = 16 * C < 64 ? 64 : 16 * C;
     constexpr int NW = NT / kWave;
@@ -202,21 +205,20 @@ __global__ __launch_bounds__(16 * C < 64 ? 64 : 16 * C) void k_invert(DevSys s, 
         if (t == 0) atomicOr(st.flags + w, kFlagSingular);
         return;
     }
-    Real *inv = reinterpret_cast<Real *>(st.inv) + (size_t)w * s.ninv + s.inv_off[d] + (size_t)mine * n;
+    double *inv = static_cast<double *>(st.inv) + (size_t)w * s.ninv + s.inv_off[d] + (size_t)mine * n;
 #pragma unroll
     for (int j = 0; j < C; ++j) {
         const int col = 4 * (j + groups < C ? j + groups : j + groups - C) + q;
-        if (row < n && col < n) inv[order[col]] = (Real)T[j];
+        if (row < n && col < n) inv[order[col]] = T[j];
     }
     if (t == 0) st.logdet[2 * w + d] = log(ldm) + (double)lde * 0.69314718055994531;
 }
 
-template <typename Real>
 bool invert_launch(const DevSys &d, const DevState &st, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>(st.W) * static_cast<unsigned>(d.ndet));
     const size_t lds = sizeof(double2) * 3 * static_cast<size_t>(d.kmax + 1) * static_cast<size_t>(d.nmax);
     const auto run = [&]<int C>() {
-        hipLaunchKernelGGL((k_invert<Real, C>), grid, dim3(16 * C < 64 ? 64 : 16 * C), lds, stream, d, st);
+        hipLaunchKernelGGL((k_invert<C>), grid, dim3(16 * C < 64 ? 64 : 16 * C), lds, stream, d, st);
         return true;
     };
     const int n = d.nmax;
@@ -233,12 +235,12 @@ bool invert_launch(const DevSys &d, const DevState &st, hipStream_t stream) {
 
 }  // namespace
 
-bool init_fast(const DevSys &d, const DevState &st, int draw, const double *aos, int real_bytes, hipStream_t stream) {
+bool init_fast(const DevSys &d, const DevState &st, int draw, const double *aos, hipStream_t stream) {
     if (d.nmax > kInitFastMax) return false;
     const size_t total = static_cast<size_t>(st.W) * static_cast<size_t>(d.N);
     const unsigned grid = static_cast<unsigned>(total / 256 + 1 < 4096 ? total / 256 + 1 : 4096);
     hipLaunchKernelGGL(k_place, dim3(grid), dim3(256), 0, stream, d, st, draw, aos);
-    return real_bytes == 8 ? invert_launch<double>(d, st, stream) : invert_launch<float>(d, st, stream);
+    return invert_launch(d, st, stream);
 }
 
 }  // namespace vmc

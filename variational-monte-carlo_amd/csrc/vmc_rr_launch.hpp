@@ -69,12 +69,12 @@ inline bool rrw_supported_sizes(int ndet, int n_up, int n_dn, int ng, int real_b
     return n_ok && ng <= 12 * kWave;
 }
 
-// Start positions and their FP64 inverses for determinants of up to
+// Start positions and their inverses, FP64 ensembles with determinants of up to
 // kInitFastMax electrons (vmc_init.hip): with draw Philox draws of attempt 0,
 // else aos (device, [W][N][3]), else the positions in place.  Walkers with a
 // singular determinant get kFlagSingular and no inverse.  False for larger ones.
 constexpr int kInitFastMax = 160;
-bool init_fast(const DevSys &d, const DevState &st, int draw, const double *aos, int real_bytes, hipStream_t stream);
+bool init_fast(const DevSys &d, const DevState &st, int draw, const double *aos, hipStream_t stream);
 
 // Newton-Schulz re-inversion on the matrix cores for FP32 inverses of
 // determinants up to kNSMaxOrder electrons (vmc_reinv_ns.hip); above 80 it
