@@ -3,7 +3,8 @@
 Sizes sit at the edges of its register tiles (2, 4, 8, ... 40 columns a lane:
 up to 8, 16, 32, 48, 64, 96, 128 and 160 electrons of a spin), one past each,
 columns that do not fill a group of four, unequal spins and one determinant;
-161 is the first that the kernel in memory takes.  With kappa = n |D^-1|_1
+161 is the first that the kernel in memory takes, which serves mixed
+precision at every size.  With kappa = n |D^-1|_1
 (|D| <= 1, so |D|_inf <= n) Gauss-Jordan with partial pivoting is within a
 small multiple of n eps kappa of the inverse and of log|det D|: both are held
 to 4 n eps kappa against the FP64 oracle, which has such an error itself, plus
