@@ -46,6 +46,37 @@ def test_blocks_follow_the_oracle_twin(vmc, oracle, n_up, n_dn):
     ens.close()
 
 
+# A smaller determinant beside the one that chose the instantiation: its rows
+# end inside a column tile that the larger one's fill, in each instantiation,
+# on either side, down to one electron.
+SMALLER = [(33, 8), (8, 33), (57, 19), (19, 57), (64, 31), (81, 57), (57, 81), (97, 33), (129, 1), (147, 123)]
+
+
+@pytest.mark.parametrize("n_up,n_dn", SMALLER, ids=[f"{a}+{b}" for a, b in SMALLER])
+def test_the_smaller_determinants_rows_keep_to_themselves(vmc, oracle, n_up, n_dn):
+    """The chain of the blocks above with one determinant much smaller, and
+    both inverses afterwards those of the final positions, within 1e-9 of
+    their largest element (the bound of a chain of delayed updates)."""
+    test_blocks_follow_the_oracle_twin(vmc, oracle, n_up, n_dn)
+    N = n_up + n_dn
+    L = vmc.box_length_from_rs(2.0, N)
+    s = vmc.System(n_up, n_dn, L, 0.25, 0.5, 1.0, 5.0 / L, 25, 0.5 * L, vmc.ERFC_EXACT, vmc.MOVE_GAUSSIAN,
+                   vmc.PREC_FP64, 0)
+    W = 5
+    ens = vmc.Ensemble(s, W, 900 + N, step0=0.8)
+    ens.init_positions()
+    ens.sweep(2, adapt=False)
+    inv, pos = ens.inverse(), ens.positions()
+    ens.close()
+    osys = oracle_system(oracle, s)
+    for w in range(W):
+        wk = oracle.Walker(osys, pos[w])
+        for d, (at, n) in enumerate(((0, n_up), (n_up * n_up, n_dn))):
+            ref = wk.inverse(d)
+            got = inv[w, at:at + n * n].reshape(n, n)
+            assert np.abs(got - ref).max() <= 1e-9 * np.abs(ref).max(), (w, d)
+
+
 def test_several_sweeps_in_one_launch_are_those_of_single_launches(vmc):
     """Unmeasured sweeps share a launch: the same chain, bit for bit, as one
     launch per sweep, step adaptation included."""

@@ -62,7 +62,7 @@ constexpr int kDuMaxAcc = 16;  // accepted moves per determinant between flushes
 constexpr int kDuGrowth = 4 * 256;
 
 // Dynamic LDS of a walker, in doubles from its start.  TH > 0: rows of up to
-// 16 TH columns (n > 16 (TH - 2)), so every offset but those of the arrays
+// 16 TH columns, so every offset but those of the arrays
 // over electrons and orbitals is a constant.
 template <int NB, int TH, bool kTwo, int NW>
 struct DuLds {
@@ -266,9 +266,13 @@ __device__ __forceinline__ void du_flush(const DuLds<NB, TH, kTwo, NW> &l, doubl
     const int r = lane & 15, g = lane >> 4;
     const int T = TH > 0 ? TH : (n + 15) / 16, TF = n / 16;  // column tiles, whole ones
     const int R = (n + 15) / 16;                               // row tiles
+    // Tiles that lie within the row's n columns: with equal spins n is the n
+    // that chose TH, so the first TH - 2 are known to; the smaller of two
+    // unequal determinants may have any number fewer.
+    const auto whole = [&](int jt) { return (kTwo && jt < TH - 2) || jt < TF; };
     const auto load = [&](const double *row, int jt) {
         du_v4d c = {0.0, 0.0, 0.0, 0.0};
-        if (jt < TH - 2 || jt < TF) {
+        if (whole(jt)) {
             const du_v4u u = *reinterpret_cast<const du_v4u *>(row + 16 * jt);
             c = u;
         } else {
@@ -317,7 +321,7 @@ __device__ __forceinline__ void du_flush(const DuLds<NB, TH, kTwo, NW> &l, doubl
         du_v4d z = {0.0, 0.0, 0.0, 0.0}, y = {0.0, 0.0, 0.0, 0.0};
         const auto store = [&](int jt, const du_v4d &c) {
             if (k >= n) return;
-            if (jt < TH - 2 || jt < TF) {
+            if (whole(jt)) {
                 *reinterpret_cast<du_v4u *>(row + 16 * jt) = c;
             } else {
 #pragma unroll
