@@ -417,11 +417,13 @@ __global__ __launch_bounds__(kMsMaxThreads, 4) void k_measure64(DevSys s, DevSta
 }
 
 // A batch group, its systems of one size or of several: one workgroup per
-// walker of the group.
+// walker of the group.  The walkers of a system that does not fit are
+// k_measure_batch64's: the launch's LDS and threads are those of the others.
 __global__ __launch_bounds__(kMsMaxThreads, 4) void k_measure64_b(const BatchItem *__restrict__ items, int n_items,
                                                                   int block_size) {
     extern __shared__ __align__(16) double sm[];
     const BatchItem &it = items[batch_find(items, n_items, blockIdx.x)];
+    if (it.generic_energy) return;
     ms_walker<false>(it.s, it.st, blockIdx.x - it.walker_begin, nullptr, block_size, sm);
 }
 

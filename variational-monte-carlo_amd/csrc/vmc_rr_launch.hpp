@@ -116,14 +116,16 @@ bool rrw_launch_f64(const DevSys &d, const DevState &st, unsigned grid, int n_sw
                     const ReinvLaunch &reinv, double *inv64);
 // The FP64 local energy from FP64 inverses (st64.inv), any number of electrons
 // (vmc_measure.hip): into the statistics, or with `parts` into
-// parts[w][kPartCount].  False where it does not fit its LDS (thousands of
-// electrons, or a reciprocal sum reaching past the 30th multiple).
+// parts[w][kPartCount].  False where it does not fit its LDS (more than 2033
+// electrons at a reach of 8; a reciprocal sum reaching past the 48th multiple
+// at 54 electrons, the 39th at 485).
 constexpr size_t kMeasure64LdsLimit = 160 * 1024;
 size_t measure64_lds(const DevSys &d);
 bool measure64_fits(const DevSys &d);
 bool measure64(const DevSys &d, const DevState &st64, unsigned grid, int bs, double *parts, hipStream_t stream);
-// A batch group's walkers (items of generic_energy = 0): max_n and lds, the
-// largest number of electrons and LDS of those systems.
+// A batch group's walkers (of its items of generic_energy = 0; it passes over
+// the others): max_n and lds, the largest number of electrons and LDS of those
+// systems.
 void measure64_batch(int max_n, size_t lds, const BatchItem *items_m64, int n_items, unsigned grid, int bs,
                      hipStream_t stream);
 
