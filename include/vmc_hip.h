@@ -234,14 +234,14 @@ int vmc_ensemble_get_inverse(vmc_ensemble *e, double *inv, void *stream);
 /* Choose the sweep kernel: VMC_KERNEL_GENERIC keeps the inverses in LDS (or
  * HBM) for any N; VMC_KERNEL_REGISTER keeps each inverse row in a lane's
  * registers (7, 19, 27, 33, 57 or 81 electrons per spin, FP32 also 123 and
- * 147; equal spins or polarised); VMC_KERNEL_DELAYED (FP64, at most 160
- * electrons per spin) keeps the inverse in HBM and applies accepted moves
- * as delayed Woodbury updates on the matrix cores, a block of moves at a time.
- * VMC_KERNEL_AUTO (default) takes the register kernel whenever it applies,
- * else, in FP64, the delayed-update kernel (any spins, up to about 500
- * electrons per spin), else the generic kernel.  No reference counterpart: the reference has a
- * single CPU code path (its rank-1 update, slater_plane_wave.cpp:367-423);
- * this is the autotuner's knob.  VMC_ERR_INVALID if the system does not fit
+ * 147; equal spins or polarised); VMC_KERNEL_DELAYED (FP64, any
+ * spins, up to about 500 electrons per spin, 512 polarised) keeps the inverse in HBM
+ * and applies accepted moves as delayed Woodbury updates on the matrix cores,
+ * a block of moves at a time.  VMC_KERNEL_AUTO (default) takes the register
+ * kernel whenever it applies, else, in FP64, the delayed-update kernel
+ * wherever it fits, else the generic kernel.  No reference counterpart: the
+ * reference has a single CPU code path (its rank-1 update,
+ * slater_plane_wave.cpp:367-423); this is the autotuner's knob.  VMC_ERR_INVALID if the system does not fit
  * the requested kernel. */
 int vmc_ensemble_set_kernel(vmc_ensemble *e, int32_t kernel);
 /* The kernel the next sweep launch will use (VMC_KERNEL_GENERIC, _REGISTER
@@ -384,7 +384,7 @@ int vmc_ensemble_footprint(const vmc_system *sys, int64_t n_walkers, int64_t *by
 
 /* --------------------------------------------------------------- autotuner
  * Picks, for one system and walker count, the kernel family (register
- * resident or generic), its build variant, the wavefronts per walker and the
+ * resident, delayed-update or generic), the wavefronts per walker and the
  * inverse placement (LDS or HBM) of the generic kernel and -- in mixed
  * precision -- the longest FP64 re-inversion interval K
  * in {256, 64, 16} whose measured inverse drift stays below drift_tol, by

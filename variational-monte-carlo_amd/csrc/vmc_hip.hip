@@ -1503,8 +1503,8 @@ int vmc_ensemble_set_kernel(vmc_ensemble *e, int32_t kernel) {
         return fail(VMC_ERR_INVALID, "unknown kernel %d", kernel);
     if (kernel == VMC_KERNEL_REGISTER && !rr_supported(e->tables.dev) && !rrw_supported(e->tables.dev, e->tables.real_bytes))
         return fail(VMC_ERR_INVALID, "register kernel needs 7, 19, 27, 33, 57 or 81 electrons per spin (FP32 also 123, 147)");
-    if (kernel == VMC_KERNEL_DELAYED && (e->tables.real_bytes != 8 || !du_supported(e->tables.dev)))
-        return fail(VMC_ERR_INVALID, "delayed-update kernel needs an FP64 system of at most 160 electrons per spin");
+    if (kernel == VMC_KERNEL_DELAYED && (e->tables.real_bytes != 8 || !du_fits(e->tables.dev)))
+        return fail(VMC_ERR_INVALID, "delayed-update kernel needs an FP64 system whose block of moves fits LDS (about 500 electrons per spin)");
     e->kernel = kernel;
     return VMC_OK;
 }

@@ -164,12 +164,10 @@ bool rrw_given_f64(const DevSys &d, const DevState &st, unsigned grid, const Swe
                    hipStream_t stream, const ReinvLaunch &reinv);
 
 // FP64 sweeps with delayed Woodbury updates of HBM-resident inverses, a block
-// of moves at a time (vmc_sweep_du.hip).  du_supported: what a caller may ask
-// for by name (at most 160 electrons per spin, equal spins or polarised).
-// du_fits: whether a walker's block fits the 160 KB of LDS (any spins; 485
-// polarised electrons do).  du_launch runs n_sweeps sweeps (no measurement)
+// of moves at a time (vmc_sweep_du.hip).  du_fits: whether a walker's block
+// fits the 160 KB of LDS (equal spins: as many as an ensemble can have; one
+// determinant: up to 512 electrons).  du_launch runs n_sweeps sweeps (no measurement)
 // with the Philox draws, or with `given` set one sweep of the caller's moves.
-bool du_supported(const DevSys &d);
 bool du_fits(const DevSys &d);
 bool du_launch(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps, unsigned long long s0, int flags,
                const SweepGiven &given, hipStream_t stream);

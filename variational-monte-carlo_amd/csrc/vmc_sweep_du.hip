@@ -811,10 +811,6 @@ size_t du_lds(const DevSys &d) {
 
 }  // namespace
 
-bool du_supported(const DevSys &d) {
-    return d.nmax <= 160 && (d.ndet == 1 || d.n_dn == d.n_up) && d.N <= 2 * 160;
-}
-
 bool du_fits(const DevSys &d) { return du_lds(d) <= kDuLdsLimit; }
 
 bool du_launch(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps, unsigned long long s0, int flags,
