@@ -1019,7 +1019,7 @@ int launch_sweep(vmc_ensemble *e, int n_sweeps, int flags, int block_size, hipSt
                                              e->inv64)
                             : rrw_launch_f64(d, e->st, grid, n_sweeps, s0, flags, block_size, stream, e->timer, rl,
                                              nullptr);
-        if (!ok) return fail(VMC_ERR_INVALID, "no register-resident instantiation for this system");
+        if (!ok) return fail(VMC_ERR_INVALID, "no register-resident kernels for this system");
         VMC_HIP_TRY(hipGetLastError());
         return VMC_OK;
     }
@@ -1995,9 +1995,10 @@ int batch_group_step(vmc_batch *b, const BatchGroup &g, int flags, int block_siz
         for (const auto &r : exact ? g.refresh_sets : g.reinv_sets)
             reinv_batch_launch(r.shape, r.items, r.n_items, static_cast<unsigned>(r.total), stream,
                                static_cast<int>(sizeof(Real)));
-        if (exact && g.energy_n > 0)
-            measure64_batch(g.energy_n, g.energy_lds, g.items_m64, n, static_cast<unsigned>(g.total), block_size,
-                            stream);
+        if (exact && g.energy_n > 0 &&
+            !measure64_batch(g.energy_n, g.energy_lds, g.items_m64, n, static_cast<unsigned>(g.total), block_size,
+                             stream))
+            return fail(VMC_ERR_DEVICE, "the local energy's LDS was refused");
         if (exact && g.lds64 > 0)
             hipLaunchKernelGGL(k_measure_batch64, dim3(static_cast<unsigned>(g.total)), dim3(b->threads), g.lds64,
                                stream, g.items_m64, n, block_size);
@@ -2012,7 +2013,7 @@ int batch_group_step(vmc_batch *b, const BatchGroup &g, int flags, int block_siz
                  : rrw_batch_step_f64(g.shape, g.items, n, static_cast<unsigned>(g.total), b->ctr, flags,
                                       block_size, g.reinv, stream, nullptr, nullptr, g.energy_lds);
     }
-    if (!ok) return fail(VMC_ERR_INVALID, "no register-resident instantiation for a batch group");
+    if (!ok) return fail(VMC_ERR_INVALID, "no register-resident kernels for a batch group");
     return VMC_OK;
 }
 

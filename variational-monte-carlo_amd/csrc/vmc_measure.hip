@@ -457,11 +457,12 @@ bool measure64(const DevSys &d, const DevState &st64, unsigned grid, int bs, dou
     return true;
 }
 
-void measure64_batch(int max_n, size_t lds, const BatchItem *items_m64, int n_items, unsigned grid, int bs,
+bool measure64_batch(int max_n, size_t lds, const BatchItem *items_m64, int n_items, unsigned grid, int bs,
                      hipStream_t stream) {
-    (void)ms_allow(reinterpret_cast<const void *>(k_measure64_b), lds);
+    if (!ms_allow(reinterpret_cast<const void *>(k_measure64_b), lds)) return false;
     hipLaunchKernelGGL(k_measure64_b, dim3(grid), dim3(static_cast<unsigned>(ms_threads(max_n))), lds, stream,
                        items_m64, n_items, bs);
+    return true;
 }
 
 }  // namespace vmc

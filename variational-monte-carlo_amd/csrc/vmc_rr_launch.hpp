@@ -126,7 +126,7 @@ bool measure64(const DevSys &d, const DevState &st64, unsigned grid, int bs, dou
 // A batch group's walkers (of its items of generic_energy = 0; it passes over
 // the others): max_n and lds, the largest number of electrons and LDS of those
 // systems.
-void measure64_batch(int max_n, size_t lds, const BatchItem *items_m64, int n_items, unsigned grid, int bs,
+bool measure64_batch(int max_n, size_t lds, const BatchItem *items_m64, int n_items, unsigned grid, int bs,
                      hipStream_t stream);
 
 // One sweep of a batch group of register-resident systems of one size
