@@ -1,6 +1,7 @@
 """GPU parity of the FP64 local energy from inverses in memory (vmc_measure.hip).
 
-Sizes sit where its split changes: two, four and eight wavefronts (up to 40,
+Sizes sit where it begins (below six electrons the generic local energy is
+taken) and where its split changes: two, four and eight wavefronts (up to 40,
 384 and more electrons), one and several slices of an electron's partners,
 electrons in one pass and in two, chunks of 64 electrons whose last one is
 short, rows of one to three column steps, unequal spins and one determinant;
@@ -18,7 +19,8 @@ from helpers import oracle_system
 pytestmark = pytest.mark.gpu
 
 # n_up, n_dn, alpha L, nmax2, cutoff / L (0: none), erfc
-CASES = [(1, 0, 5.0, 25, 0.5, 1), (2, 1, 5.0, 25, 0.5, 1), (8, 1, 5.0, 1, 0.5, 1), (17, 23, 5.0, 25, 0.5, 1),
+CASES = [(1, 0, 5.0, 25, 0.5, 1), (2, 1, 5.0, 25, 0.5, 1), (3, 2, 5.0, 25, 0.5, 1),
+         (3, 3, 5.0, 25, 0.5, 1), (6, 0, 5.0, 25, 0.5, 1), (8, 1, 5.0, 1, 0.5, 1), (17, 23, 5.0, 25, 0.5, 1),
          (21, 20, 5.0, 25, 0.5, 1), (33, 33, 5.0, 25, 0.5, 1), (33, 33, 0.0, 0, 0.0, 0), (34, 31, 8.0, 121, 0.5, 1),
          (64, 64, 5.0, 64, 0.0, 1), (65, 64, 5.0, 49, 0.49, 1), (81, 81, 5.0, 25, 0.5, 1), (150, 0, 5.0, 25, 0.5, 1),
          (147, 147, 5.0, 25, 0.5, 1), (193, 192, 5.0, 9, 0.5, 1)]

@@ -1,5 +1,5 @@
-// vmc_measure.hip -- the FP64 local energy from FP64 inverses in memory, any
-// number of electrons (energy_tracking.cpp:253-382 with the Jastrow and Slater
+// vmc_measure.hip -- the FP64 local energy from FP64 inverses in memory, six
+// electrons and more (energy_tracking.cpp:253-382 with the Jastrow and Slater
 // derivatives of jastrow_pade.cpp:57-138, slater_plane_wave.cpp:425-499).
 //
 // One workgroup per walker, 2 to 8 wavefronts by the number of electrons alone
@@ -433,9 +433,14 @@ size_t measure64_lds(const DevSys &d) {
     return sizeof(double) * (size_t)MsLds(d.N, d.n[0], d.ndet == 2 ? d.n[1] : 0, d.pmax).total;
 }
 
-// (a system past the limit, by its number of electrons or the reach of its
-// reciprocal sum, keeps the generic local energy)
-bool measure64_fits(const DevSys &d) { return measure64_lds(d) <= kMeasure64LdsLimit; }
+// A system past the LDS limit, by its number of electrons or the reach of its
+// reciprocal sum, keeps the generic local energy; so do the smallest, for which
+// two wavefronts per walker and a staging pass cost more than they share out
+// (one call, generic -> here: 1 + 0 electrons, 16384 walkers 157 -> 327 us, 2 + 2
+// 201 -> 249, 3 + 2 217 -> 238, 3 + 3 232 -> 240, 6 + 0 240 -> 239, 5 + 5 301 ->
+// 236; 2 + 1, one walker 34 -> 38, 6 + 0 40 -> 37).
+constexpr int kMsMinN = 6;
+bool measure64_fits(const DevSys &d) { return d.N >= kMsMinN && measure64_lds(d) <= kMeasure64LdsLimit; }
 
 // Dynamic LDS above 64 KB has to be asked for, kernel by kernel.
 static bool ms_allow(const void *kernel, size_t lds) {

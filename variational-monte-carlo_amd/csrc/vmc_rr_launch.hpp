@@ -114,9 +114,9 @@ bool rrw_launch_f32(const DevSys &d, const DevState &st, unsigned grid, int n_sw
 bool rrw_launch_f64(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
                     unsigned long long s0, int flags, int bs, hipStream_t stream, KernelTimer &timer,
                     const ReinvLaunch &reinv, double *inv64);
-// The FP64 local energy from FP64 inverses (st64.inv), any number of electrons
+// The FP64 local energy from FP64 inverses (st64.inv), six electrons and more
 // (vmc_measure.hip): into the statistics, or with `parts` into
-// parts[w][kPartCount].  False where it does not fit its LDS (more than 2033
+// parts[w][kPartCount].  False for fewer and where it does not fit its LDS (more than 2033
 // electrons at a reach of 8; a reciprocal sum reaching past the 48th multiple
 // at 54 electrons, the 39th at 485).
 constexpr size_t kMeasure64LdsLimit = 160 * 1024;
