@@ -28,6 +28,7 @@ def test_blocks_follow_the_oracle_twin(vmc, oracle, n_up, n_dn):
                    vmc.PREC_FP64, 0)
     W, seed, step = 2, 700 + N, 0.8
     ens = vmc.Ensemble(s, W, seed, step0=step)
+    ens.set_kernel(vmc.KERNEL_DELAYED)
     assert ens.kernel() == vmc.KERNEL_DELAYED
     ens.init_positions()
     osys = oracle_system(oracle, s)
@@ -64,6 +65,7 @@ def test_the_smaller_determinants_rows_keep_to_themselves(vmc, oracle, n_up, n_d
                    vmc.PREC_FP64, 0)
     W = 5
     ens = vmc.Ensemble(s, W, 900 + N, step0=0.8)
+    ens.set_kernel(vmc.KERNEL_DELAYED)
     ens.init_positions()
     ens.sweep(2, adapt=False)
     inv, pos = ens.inverse(), ens.positions()
@@ -86,6 +88,7 @@ def test_several_sweeps_in_one_launch_are_those_of_single_launches(vmc):
     out = []
     for calls, n in ((1, 5), (5, 1)):
         e = vmc.Ensemble(s, 67, 9, step0=0.7)
+        e.set_kernel(vmc.KERNEL_DELAYED)
         e.init_positions()
         for _ in range(calls):
             e.sweep(n, adapt=True)

@@ -33,6 +33,39 @@ def test_the_reported_kernel_can_be_set(vmc, n_up, n_dn):
         e.close()
 
 
+# Electrons up and down, walkers, and whether AUTO takes the delayed-update kernel:
+# both sides of the lines that its rule has.
+LINES = [(3, 3, 8, False), (4, 4, 8, True), (4, 4, 513, False), (5, 5, 513, True), (5, 5, 1281, False),
+         (8, 8, 1281, True), (16, 16, 1281, True), (17, 17, 1280, True), (17, 17, 1281, False),
+         (24, 24, 1281, True), (6, 0, 8, False), (8, 0, 1280, True), (8, 0, 1281, False), (12, 0, 1281, True),
+         (5, 2, 8, False), (8, 1, 512, True), (8, 1, 513, False), (12, 4, 1280, True), (19, 7, 1281, False),
+         (33, 8, 1281, True)]
+
+
+@pytest.mark.parametrize("n_up,n_dn,W,delayed", LINES, ids=[f"{a}+{b}_{w}" for a, b, w, _ in LINES])
+def test_auto_takes_the_faster_kernel_and_both_follow_one_chain(vmc, n_up, n_dn, W, delayed):
+    """The rule's lines; and on either side the chain is that of the other
+    kernel: the same number of accepted moves, and positions to the rounding of
+    the FP64 proposal (1e-12 L)."""
+    s = gas(vmc, n_up, n_dn)
+    N, L = s.N, s.box_length
+    auto = vmc.Ensemble(s, W, 77 + N, step0=0.5)
+    assert auto.kernel() == (vmc.KERNEL_DELAYED if delayed else vmc.KERNEL_GENERIC)
+    other = vmc.Ensemble(s, W, 77 + N, step0=0.5)
+    other.set_kernel(vmc.KERNEL_GENERIC if delayed else vmc.KERNEL_DELAYED)
+    out = []
+    for e in (auto, other):
+        e.init_positions()
+        e.sweep(2, measure=True)
+        out.append((e.positions(), e.stats()))
+        e.close()
+    (p, st), (q, su) = out
+    acc, nmeas = vmc.STAT["ACCEPTED"], vmc.STAT["NMEAS"]
+    np.testing.assert_array_equal(st[:, acc], su[:, acc])
+    assert np.all(st[:, nmeas] == 2) and np.all(su[:, nmeas] == 2)
+    np.testing.assert_allclose(p, q, rtol=0, atol=1e-12 * L)
+
+
 def test_the_delayed_kernel_is_refused_where_it_does_not_fit(vmc):
     e = vmc.Ensemble(gas(vmc, 513, 0), 1, 3)
     assert e.kernel() == vmc.KERNEL_GENERIC

@@ -849,12 +849,36 @@ bool rrw_supported(const DevSys &d, int real_bytes) {
     return rrw_supported_sizes(d.ndet, d.n_up, d.n_dn, d.ng, real_bytes);
 }
 
+// Where the delayed-update sweep beats the generic one, which keeps inverses
+// of these sizes in LDS.  A block of moves costs a fixed dozen phases, so it
+// takes more electrons to pay the more walkers share the chip: a walker is one
+// wavefront of the generic kernel and four or more of the block's, so beyond
+// 1024 walkers the blocks queue first.  One determinant or equal spins of up to
+// 32 electrons are one block a sweep (32 movers; 16 up to 16 per spin), unequal
+// spins two.  Time of
+// the generic sweep over the delayed one's, unmeasured / measured:
+//   up to 512 walkers   equal 3 + 3 1.24 / 0.93, 4 + 4 1.54 / 1.20; one determinant
+//                       6 1.46 / 0.99, 7 1.67 / 1.17; unequal 5 + 2 0.89 / 0.86, 8 + 1
+//                       1.11 / 1.08
+//   1280 walkers        4 + 4 0.93 / 0.95, 5 + 5 1.08 / 1.14, 23 + 23 1.53 / 1.66; 7 1.02 /
+//                       0.97, 8 1.13 / 1.07; 8 + 6 0.90 / 1.15, 12 + 4 1.06 / 1.31
+//   4096 walkers        6 + 6 0.91 / 0.98, 8 + 8 1.09 / 1.21, 16 + 16 1.87 / 1.88, 17 + 17
+//                       0.82 / 0.99, 20 + 20 0.92 / 1.08, 24 + 24 1.13 / 1.39; 10 1.01 /
+//                       0.96, 12 1.15 / 1.12; 19 + 7 0.91 / 1.09, 33 + 8 1.09 / 1.46
+//   16384 walkers       8 + 8 0.94 / 1.20, 12 1.00 / 1.10, 19 + 7 0.75 / 1.04, 25 + 5 0.87 /
+//                       1.16 (8192: 23 + 23 0.81 / 1.03, 24 + 24 0.93 / 1.17, 27 + 19 1.16 / 1.50)
+// and beyond, 40 + 40 at 4096 walkers 2.6 / 3.2 and 485 electrons at eight 31.
+bool du_pays(const DevSys &d, int64_t W) {
+    const bool one = d.ndet == 1, equal = !one && d.n_up == d.n_dn;
+    if (W > 1280) return equal ? d.N >= 16 && (d.N <= 32 || d.N >= 48) : d.N >= (one ? 12 : 40);
+    if (W > 512) return d.N >= (equal ? 10 : one ? 8 : 16);
+    return d.N >= (equal ? 8 : one ? 7 : 9);
+}
+
 // Sweep kernel family of an ensemble: the register-resident kernels where an
-// instantiation exists, in FP64 the delayed-update kernel wherever it fits
-// (against the generic kernel, per sweep: 19 + 7 electrons, 777 walkers, 0.46
-// -> 0.07 ms; 485 electrons, 8 walkers, 138 -> 3.5 ms), else the generic
-// kernel; or the family the caller forced (vmc_ensemble_set_kernel validated
-// it).
+// instantiation exists, in FP64 the delayed-update kernel where it fits and
+// pays, else the generic kernel; or the family the caller forced
+// (vmc_ensemble_set_kernel validated it).
 enum { kFamGeneric = 0, kFamRegister = 1, kFamMultiwave = 2, kFamDelayed = 3 };
 int sweep_family(const vmc_ensemble *e) {
     const DevSys &d = e->tables.dev;
@@ -863,7 +887,8 @@ int sweep_family(const vmc_ensemble *e) {
     if (e->kernel == VMC_KERNEL_DELAYED) return kFamDelayed;
     if (rr_supported(d)) return kFamRegister;
     if (rrw_supported(d, rb)) return kFamMultiwave;
-    if (e->kernel == VMC_KERNEL_AUTO && rb == 8 && du_fits(d)) return kFamDelayed;
+    if (e->kernel == VMC_KERNEL_AUTO && rb == 8 && du_fits(d) && du_pays(d, e->W))
+        return kFamDelayed;
     return kFamGeneric;
 }
 
