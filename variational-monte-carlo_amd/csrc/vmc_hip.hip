@@ -1235,8 +1235,10 @@ int vmc_ensemble_set_positions(vmc_ensemble *e, const double *pos, void *stream)
     const int N = e->tables.dev.N;
     const size_t W = static_cast<size_t>(e->W);
     const double L = e->tables.dev.L;
-    for (size_t i = 0; i < W * 3 * N; ++i)
-        if (!(pos[i] >= 0.0 && pos[i] < L)) return fail(VMC_ERR_INVALID, "position outside [0, L)");
+    // Checked without an early exit, which lets the pass be vectorised, and in
+    // the pass that lays them out where there is one: a scan of its own before
+    // it took as long again (mixed 13 + 13, 16384 walkers 1093 -> 1396 us a call).
+    bool inside = true;
     // As they are into the Gauss-Jordan workspace, whence the device takes
     // them into its layout (init_fast); for the determinants it does not take,
     // and workspaces too small, they are laid out here.
@@ -1244,13 +1246,20 @@ int vmc_ensemble_set_positions(vmc_ensemble *e, const double *pos, void *stream)
     std::vector<double> soa;
     const double *aos = nullptr;
     if (e->tables.real_bytes == 8 && e->tables.dev.nmax <= kInitFastMax && nmax2 >= static_cast<size_t>(3 * N)) {
+        for (size_t i = 0; i < W * 3 * N; ++i) inside &= pos[i] >= 0.0 && pos[i] < L;
+        if (!inside) return fail(VMC_ERR_INVALID, "position outside [0, L)");
         VMC_HIP_TRY(hipMemcpyAsync(e->st.scratch, pos, sizeof(double) * W * 3 * N, hipMemcpyHostToDevice, s));
         aos = e->st.scratch;
     } else {
         soa.resize(W * 3 * N);
         for (size_t w = 0; w < W; ++w)
             for (int i = 0; i < N; ++i)
-                for (int c = 0; c < 3; ++c) soa[(w * 3 + c) * N + i] = pos[(w * N + i) * 3 + c];
+                for (int c = 0; c < 3; ++c) {
+                    const double x = pos[(w * N + i) * 3 + c];
+                    inside &= x >= 0.0 && x < L;
+                    soa[(w * 3 + c) * N + i] = x;
+                }
+        if (!inside) return fail(VMC_ERR_INVALID, "position outside [0, L)");
         VMC_HIP_TRY(hipMemcpyAsync(e->st.pos, soa.data(), sizeof(double) * soa.size(), hipMemcpyHostToDevice, s));
     }
     int rc = e->tables.real_bytes == 8 ? launch_init<double>(e, 0, aos, s) : launch_init<float>(e, 0, aos, s);
