@@ -62,3 +62,32 @@ def test_two_electrons_at_one_place(vmc, oracle):
     assert abs(got["VREAL"][0] - wk.vreal()) <= 1e-10 * max(abs(wk.vreal()), 1e-3 * N)
     assert abs(got["JASTROW"][0] - wk.jastrow()) <= 1e-10 * max(abs(wk.jastrow()), 1e-3 * N)
     assert np.isfinite(got["KINETIC"][0])
+
+
+@pytest.mark.parametrize("n_up,n_dn", [(27, 27), (27, 0)], ids=["27+27", "27+0"])
+def test_mixed_energy_does_not_depend_on_the_number_of_walkers(vmc, n_up, n_dn):
+    """The mixed-precision local energy of 27 per spin takes the Slater rows in
+    one trip up to 2048 walkers and in two above: the same walkers give the
+    same bits in both, refreshed inverses and statistics included, alone and
+    in a batch."""
+    N = n_up + n_dn
+    L = vmc.box_length_from_rs(2.0, N)
+    s = vmc.System(n_up, n_dn, L, 0.25, 0.5, 1.0, 5.0 / L, 25, 0.5 * L, vmc.ERFC_EXACT, vmc.MOVE_GAUSSIAN,
+                   vmc.PREC_MIXED, 64)
+    out = []
+    for W in (2048, 2049):
+        e = vmc.Ensemble(s, W, 11, step0=0.4)
+        e.init_positions()
+        e.sweep(3, measure=True)
+        parts = e.measure()
+        out.append([a[:2048] for a in (e.positions(), e.inverse(), e.stats(), *parts.values())])
+        e.close()
+        b = vmc.Batch([s], [W], [11], step0=[0.4])
+        b.init_positions()
+        b.sweep(3, measure=True)
+        m = b.member(0)
+        out.append([a[:2048] for a in (m.positions(), m.inverse(), m.stats())])
+        b.close()
+    for other in out[1:]:
+        for x, y in zip(out[0], other):
+            np.testing.assert_array_equal(x, y)

@@ -8,6 +8,21 @@
 
 namespace vmc {
 
+// Calls f.template operator()<kTrips>() with the mixed-precision local energy's
+// form for `walkers` walkers in a launch (RRMixedShared; the same bits in both).
+// One trip while its LDS holds sixteen walkers on a CU (up to 19 per spin), and
+// at 27 up to 2048 walkers, eight to a CU.
+template <int NU, int ND, typename F>
+void rr_mixed_form(unsigned walkers, F &&f) {
+    constexpr unsigned kOneTrip = 2048;
+    if constexpr (sizeof(RRMixedShared<NU, ND, 1>) <= 10 * 1024) {
+        f.template operator()<1>();
+    } else {
+        if (walkers <= kOneTrip) f.template operator()<1>();
+        else f.template operator()<2>();
+    }
+}
+
 // One launch of the sweep kernel per sweep, each followed by the FP64
 // re-inversion of the walkers that reached K accepted moves (when K > 0) and,
 // with MEASURE, the local energy.  In mixed precision the local energy is
@@ -43,8 +58,10 @@ void rr_launch_g(const DevSys &d, const DevState &st, unsigned grid, int n_sweep
         if (measure) {
             timed = timer.begin(stream, ev);
             if constexpr (kMixed)
-                hipLaunchKernelGGL((k_measure_rr_mixed<NU, ND, GPL>), dim3(grid), dim3(kWave), 0, stream, d, st,
-                                   bs);
+                rr_mixed_form<NU, ND>(grid, [&]<int kTrips>() {
+                    hipLaunchKernelGGL((k_measure_rr_mixed<NU, ND, GPL, kTrips>), dim3(grid), dim3(kWave), 0, stream,
+                                       d, st, bs);
+                });
             else
                 hipLaunchKernelGGL((k_measure_rr<Real, NU, ND, GPL>), dim3(grid), dim3(kWave), 0,
                                    stream, d, st, bs);
@@ -102,8 +119,10 @@ template <typename Real>
 bool rr_parts(const DevSys &d, const DevState &st, unsigned grid, double *parts, hipStream_t stream) {
     return rr_dispatch<Real>(d, [&]<int NU, int ND, int GPL>() {
         if constexpr (sizeof(Real) == 4)
-            hipLaunchKernelGGL((k_measure_rr_mixed_parts<NU, ND, GPL>), dim3(grid), dim3(kWave), 0, stream, d, st,
-                               parts);
+            rr_mixed_form<NU, ND>(grid, [&]<int kTrips>() {
+                hipLaunchKernelGGL((k_measure_rr_mixed_parts<NU, ND, GPL, kTrips>), dim3(grid), dim3(kWave), 0,
+                                   stream, d, st, parts);
+            });
         else
             hipLaunchKernelGGL((k_measure_rr_parts<Real, NU, ND, GPL>), dim3(grid), dim3(kWave), 0, stream, d, st,
                                parts);
@@ -124,8 +143,10 @@ bool rr_batch_step(const DevSys &shape, const BatchItem *items, int n_items, uns
                                stream, items, n_items);
         if (measure) {
             if constexpr (kMixed)
-                hipLaunchKernelGGL((k_measure_rr_mixed_b<NU, ND, GPL>), dim3(grid), dim3(kWave), 0, stream,
-                                   items, n_items, bs);
+                rr_mixed_form<NU, ND>(grid, [&]<int kTrips>() {
+                    hipLaunchKernelGGL((k_measure_rr_mixed_b<NU, ND, GPL, kTrips>), dim3(grid), dim3(kWave), 0,
+                                       stream, items, n_items, bs);
+                });
             else
                 hipLaunchKernelGGL((k_measure_rr_b<Real, NU, ND, GPL>), dim3(grid), dim3(kWave), 0, stream,
                                    items, n_items, bs);

@@ -1550,18 +1550,21 @@ __device__ __forceinline__ void measure_rr_body(const DevSys &s, const DevState 
 // of the row).  A second step follows when n max|E|^2 exceeds 1e-10; a
 // residual of 0.5 or more (or a non-finite one) rebuilds the inverse by FP64
 // Gauss-Jordan instead (also refreshing log|det|).
-// LDS of the mixed-precision local energy: the D rows (FP64) and X rows (FP32) of half
-// the electrons of each spin at a time during the refinement; after it the
-// structure-factor tables and the positions.  10 KB at 27 per spin, so that
-// the four walkers of a SIMD at 4096 walkers run at once (whole rows and E's
-// columns took 20 KB, two walkers at a time: 124 us instead of 115 for 4096).
-template <int NU, int ND>
+// LDS of the mixed-precision local energy: the D rows (FP64) and X rows (FP32) of all
+// the electrons of each spin, or of half of them at a time, during the
+// refinement; after it the structure-factor tables and the positions.
+// At 27 per spin one trip takes 19 KB, two walkers to a SIMD, and two trips 10 KB,
+// four: per measured sweep one trip against two, 1 walker 78 / 87 us, 1024 92 / 105,
+// 2048 114 / 130, 2560 162 / 153, 4096 213 / 192, 8192 371 / 342 (two trips build the
+// D rows in two half-empty passes and spill).  At 19 per spin one trip takes 9 KB:
+// 62 / 67 at 1024, 117 / 122 at 4096 (147 with E's columns in LDS beside whole rows).
+template <int NU, int ND, int kTrips>
 struct RRMixedShared {
     static constexpr int NMAX = NU > ND ? NU : ND;
-    static constexpr int kHalf = (NMAX + 1) / 2;  // rows of a spin at a time
+    static constexpr int kRows = (NMAX + kTrips - 1) / kTrips;  // rows of a spin at a time
     static constexpr int P = (NMAX + 1) / 2 * 2;  // D row pitch in doubles (16-byte rows)
     static constexpr int PX = (NMAX + 3) / 4 * 4; // X row pitch in floats (16-byte rows)
-    static constexpr int kRefineDoubles = 2 * kHalf * P + kHalf * PX;
+    static constexpr int kRefineDoubles = 2 * kRows * P + kRows * PX;
     static constexpr int kRebuildDoubles = NMAX * NMAX;
     static constexpr int kTableDoubles = sf::table_reals<double>();
     union {
@@ -1575,9 +1578,9 @@ struct RRMixedShared {
     int perm[32];
     static constexpr size_t kStageBytes = sizeof(tab);
     __device__ void *stage() { return tab; }
-    __device__ double *d_row(int h, int i) { return buf + (h * kHalf + i) * P; }
+    __device__ double *d_row(int h, int i) { return buf + (h * kRows + i) * P; }
     __device__ float *x_row(int h, int i) {
-        return reinterpret_cast<float *>(buf + 2 * kHalf * P) + (h * kHalf + i) * PX;
+        return reinterpret_cast<float *>(buf + 2 * kRows * P) + (h * kRows + i) * PX;
     }
 };
 
@@ -1593,12 +1596,12 @@ constexpr double kRefineTarget = 1e-8;
 // inverse (the drift; +inf when it was rebuilt from scratch, -1 when a
 // determinant is singular).  ld[h] receives a rebuilt determinant's
 // log|det|.
-template <int NU, int ND, int GPL>
-__device__ double rr_refine(const DevSys &s, RRMixedShared<NU, ND> &sh, RRLane<double, (NU > ND ? NU : ND)> &L,
+template <int NU, int ND, int GPL, int kTrips>
+__device__ double rr_refine(const DevSys &s, RRMixedShared<NU, ND, kTrips> &sh, RRLane<double, (NU > ND ? NU : ND)> &L,
                             int lane, int h, int r, bool has_e, double (&ld)[2]) {
     using K = RRKernel<double, NU, ND, GPL>;
-    using Sh = RRMixedShared<NU, ND>;
-    constexpr int NMAX = K::NMAX, kHalf = Sh::kHalf;
+    using Sh = RRMixedShared<NU, ND, kTrips>;
+    constexpr int NMAX = K::NMAX, kRows = Sh::kRows;
     constexpr int NP = NU;  // equal spins or polarised: every row lane has NU rows
     const int nh = h ? ND : NU;
     constexpr auto orb = rr::shell_orbitals<NMAX>();
@@ -1635,8 +1638,8 @@ __device__ double rr_refine(const DevSys &s, RRMixedShared<NU, ND> &sh, RRLane<d
 #pragma unroll
         for (int j = 0; j < NMAX; ++j) c[j] = 0.0f;
 #pragma unroll 1
-        for (int i0 = 0; i0 < NMAX; i0 += kHalf) {
-            const int rows = NMAX - i0 < kHalf ? NMAX - i0 : kHalf;
+        for (int i0 = 0; i0 < NMAX; i0 += kRows) {
+            const int rows = NMAX - i0 < kRows ? NMAX - i0 : kRows;
             __syncthreads();  // the rows before have been read
             if (has_e && r >= i0 && r - i0 < rows) {
                 put_d_row(sh.d_row(h, r - i0), 1);
@@ -1713,13 +1716,13 @@ __device__ double rr_refine(const DevSys &s, RRMixedShared<NU, ND> &sh, RRLane<d
 // refined inverse, rounded to FP32, replaces the stored one (this is the
 // walker's periodic re-inversion: move count cleared, drift recorded) unless
 // only the parts are asked for.
-template <int NU, int ND, int GPL>
+template <int NU, int ND, int GPL, int kTrips>
 __device__ __forceinline__ void measure_rr_refined_body(const DevSys &s, const DevState &st, int w,
                                                         int block_size, double *parts = nullptr) {
     using K = RRKernel<double, NU, ND, GPL>;
     constexpr int NMAX = K::NMAX;
     constexpr int N = NU + ND;
-    __shared__ RRMixedShared<NU, ND> sh;
+    __shared__ RRMixedShared<NU, ND, kTrips> sh;
     const RRConst<double> cst(s);
     const int lane = threadIdx.x;
     const int h = lane >> 5, r = lane & 31;
@@ -1739,7 +1742,7 @@ __device__ __forceinline__ void measure_rr_refined_body(const DevSys &s, const D
     L.y = has_e ? gp[N + e] : 0.0;
     L.z = has_e ? gp[2 * N + e] : 0.0;
     double ld[2] = {st.logdet[2 * w + 0], st.logdet[2 * w + 1]};
-    const double drift = rr_refine<NU, ND, GPL>(s, sh, L, lane, h, r, has_e, ld);
+    const double drift = rr_refine<NU, ND, GPL, kTrips>(s, sh, L, lane, h, r, has_e, ld);
     if (!parts) {
         float xo[NMAX];
 #pragma unroll
@@ -1825,24 +1828,28 @@ __global__ __launch_bounds__(kWave) void k_measure_rr_parts(DevSys s, DevState s
 
 // Mixed precision: the FP64 local energy from the refined FP32 inverse
 // (which it also refreshes), its parts-only form, and the batch form.
-// 7 polarised electrons have the structure factor's values in registers.
-constexpr int rr_mixed_waves(int n_up, int n_dn) { return n_up + n_dn > kRRChunk ? 4 : 1; }
-
-template <int NU, int ND, int GPL>
-__global__ __launch_bounds__(kWave, rr_mixed_waves(NU, ND)) void k_measure_rr_mixed(DevSys s, DevState st, int block_size) {
-    measure_rr_refined_body<NU, ND, GPL>(s, st, blockIdx.x, block_size);
+// kTrips: the refinement's rows in one trip, at most two walkers of equal spins
+// to a SIMD, or in two (RRMixedShared).  7 polarised electrons have the
+// structure factor's values in registers.
+constexpr int rr_mixed_waves(int n_up, int n_dn, int trips) {
+    return trips == 1 ? (n_dn > 0 ? 2 : 1) : n_up + n_dn > kRRChunk ? 4 : 1;
 }
 
-template <int NU, int ND, int GPL>
-__global__ __launch_bounds__(kWave, rr_mixed_waves(NU, ND)) void k_measure_rr_mixed_parts(DevSys s, DevState st, double *parts) {
-    measure_rr_refined_body<NU, ND, GPL>(s, st, blockIdx.x, 1, parts);
+template <int NU, int ND, int GPL, int kTrips>
+__global__ __launch_bounds__(kWave, rr_mixed_waves(NU, ND, kTrips)) void k_measure_rr_mixed(DevSys s, DevState st, int block_size) {
+    measure_rr_refined_body<NU, ND, GPL, kTrips>(s, st, blockIdx.x, block_size);
 }
 
-template <int NU, int ND, int GPL>
-__global__ __launch_bounds__(kWave, rr_mixed_waves(NU, ND)) void k_measure_rr_mixed_b(const BatchItem *__restrict__ items, int n_items,
+template <int NU, int ND, int GPL, int kTrips>
+__global__ __launch_bounds__(kWave, rr_mixed_waves(NU, ND, kTrips)) void k_measure_rr_mixed_parts(DevSys s, DevState st, double *parts) {
+    measure_rr_refined_body<NU, ND, GPL, kTrips>(s, st, blockIdx.x, 1, parts);
+}
+
+template <int NU, int ND, int GPL, int kTrips>
+__global__ __launch_bounds__(kWave, rr_mixed_waves(NU, ND, kTrips)) void k_measure_rr_mixed_b(const BatchItem *__restrict__ items, int n_items,
                                                               int block_size) {
     const BatchItem &it = items[batch_find(items, n_items, blockIdx.x)];
-    measure_rr_refined_body<NU, ND, GPL>(it.s, it.st, blockIdx.x - it.walker_begin, block_size);
+    measure_rr_refined_body<NU, ND, GPL, kTrips>(it.s, it.st, blockIdx.x - it.walker_begin, block_size);
 }
 
 // Batch forms: one launch covers the walkers of every system of a batch group
