@@ -96,3 +96,49 @@ def test_several_sweeps_in_one_launch_are_those_of_single_launches(vmc):
         e.close()
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n_up,n_dn,first", [(10, 10, 0), (10, 10, 5), (19, 7, 0), (19, 7, 6), (65, 65, 4), (161, 0, 0),
+                                             (161, 0, 9)],
+                         ids=["10+10_0", "10+10_5", "19+7_0", "19+7_6", "65+65_4", "161+0_0", "161+0_9"])
+def test_a_move_away_from_a_node_keeps_the_inverse(vmc, oracle, n_up, n_dn, first):
+    """Two electrons of one spin 1e-5 L apart, one of which (the first mover or
+    one in mid-block) moves away: its ratio R is about 1e5 and the inverse
+    shrinks by as much.  One rank-1 update leaves an error of a few R roundings
+    of the new inverse (n of them in the sums); a flush that multiplied rows R
+    times too large by a rounded 1 - (1 - 1/R) left R^2 of them, 1e-6."""
+    N = n_up + n_dn
+    L = vmc.box_length_from_rs(2.0, N)
+    s = vmc.System(n_up, n_dn, L, 0.25, 0.5, 1.0, 5.0 / L, 25, 0.5 * L, vmc.ERFC_EXACT, vmc.MOVE_GAUSSIAN,
+                   vmc.PREC_FP64, 0)
+    osys = oracle_system(oracle, s)
+    rng = np.random.default_rng(31 * N + first)
+    W = 3
+    pos = np.stack([oracle.init_positions(osys, 5 + w, w)[0] for w in range(W)])
+    pos[:, first] = pos[:, first + 2] + 1e-5 * L * np.array([0.6, -0.5, 0.62])
+    pos -= L * np.floor(pos / L)
+    prop = pos + rng.normal(0.0, 0.1 * L / N ** (1 / 3), pos.shape)
+    prop[:, first] = rng.uniform(0.0, L, (W, 3))
+    prop -= L * np.floor(prop / L)
+    u = rng.uniform(0.0, 1.0, (W, N))
+    u[:, first] = 1e-30
+    for kernel in (vmc.KERNEL_DELAYED, vmc.KERNEL_GENERIC):
+        e = vmc.Ensemble(s, W, 1)
+        e.set_kernel(kernel)
+        e.set_positions(pos)
+        trace = e.sweep_given(prop, u)
+        inv, after = e.inverse(), e.positions()
+        e.close()
+        assert np.all(trace[:, first, 2] == 1.0)
+        seen = 0
+        for w in range(W):
+            R = np.abs(trace[w, :, 0]).max()
+            if R < 1e3:  # (its new place is near a node as well)
+                continue
+            seen += 1
+            ref = oracle.Walker(osys, after[w]).inverse(0)
+            got = inv[w, :n_up * n_up].reshape(n_up, n_up)
+            err = np.abs(got - ref).max() / np.abs(ref).max()
+            print(f"kernel {kernel} R {R:.1e} error {err:.1e}", flush=True)
+            assert err <= 16 * n_up * 2.2e-16 * R, (kernel, w)
+        assert seen >= 2

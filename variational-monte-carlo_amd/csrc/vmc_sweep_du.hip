@@ -22,11 +22,11 @@
 //     test, one row of X, one row broadcast and 31 FMAs per pair of moves.
 //   - A flush applies the m <= 16 accepted moves to all n rows of invT on the
 //     matrix cores, 16 rows per wavefront at a time:
-//       Z = Phi'_acc invT[rows]^T - E, Y = Cinv Z, invT[rows] -= Y^T P_acc,
-//     each row read once and written once (E: unit entries at the movers' own
-//     rows; P_acc: the accepted movers' old rows, copied to LDS first).
+//       Z = Phi'_acc invT[rows]^T, Y = Cinv Z, invT[rows] -= Y^T P_acc,
+//     each row read once and written once (P_acc: the accepted movers' old rows,
+//     copied to LDS first; the movers' own rows become Cinv^T P_acc).
 // A block ends early when 16 moves are accepted in one determinant or when
-// the product of its accepted ratios exceeds 16 (kDuGrowth).
+// the product of its accepted ratios exceeds a limit (du_growth_limit).
 //
 // What bounds it (N = 294, 1024 walkers, 1.70 ms a sweep): FP64 VALU work (43 %
 // of the cycles, the pair terms above all) and FP64 MFMA issue (24 %) of two
@@ -56,10 +56,31 @@ typedef double du_v4u __attribute__((ext_vector_type(4), aligned(8)));
 constexpr int kG = 8;  // decisions per unrolled group
 constexpr int kDuMaxAcc = 16;  // accepted moves per determinant between flushes: one MFMA tile
 // A flush forms invT as the difference of terms that grow with the product of
-// the accepted ratios since the last one (the determinant's growth); walkers
-// leaving a near-singular start accept ratios of 5 to 12.  In 1/256 of log2:
-// the block ends above a growth of 16.
-constexpr int kDuGrowth = 4 * 256;
+// the accepted ratios since the last one, from its lowest point on (the
+// determinant's growth G): it loses G^2 roundings where one accepted move after
+// another loses G, and walkers leaving a near-singular start accept ratios of 5
+// and far more.  A block therefore ends above a growth of 4, and of 16 for equal
+// spins above 64 and one determinant above 96; log2 in 1/256.  Stored inverse
+// against an 80-bit one, max|error| / max|inverse|, mean over walkers after one
+// sweep from uniform starts and after 36, in 1e-15: rank-1 updates of every
+// accepted move -> limit 4 (limit 16)
+//   10 + 10  4.8 -> 5.6 (19) and 1.2 -> 1.2 (1.4)    33 + 27  15 -> 22 (64) and 3.8 -> 5.3 (7.0)
+//   13 + 13  5.9 -> 7.9 (73) and 1.5 -> 1.8 (2.0)    50 + 50  20 -> 27 (39) and 8.6 -> 9.1 (16)
+//   19 + 7   5.4 -> 7.3 (15) and 1.5 -> 1.9 (2.2)    161      200 -> 210 (2300) and 70 -> 56 (210)
+// the largest of 512 walkers at 13 + 13 1.0e-12 -> 1.1e-12 (5.2e-11); windows of 8
+// accepted moves -> limit 16: 70 + 70 440 -> 62 and 600 -> 24, 123 + 123 160 -> 100 and
+// 1000 -> 48, 147 230 -> 83 and 3400 -> 53.  Limit 4 against 16 costs 8 % of a sweep
+// at 19 + 7, 24 % at 50 + 50 and 21 % at 485, more where each sweep is a launch of
+// its own, as long as its slowest walker.
+template <int TH, bool kTwo>
+__device__ __forceinline__ int du_growth_limit(const DevSys &s) {
+    const bool wide = kTwo ? TH >= 6 : TH >= 8 && s.ndet == 1;
+    return wide ? 4 * 256 : 2 * 256;
+}
+// A move that would pass the limit by this factor (a walker leaving a node, by
+// a ratio of 1e3 and more) waits for the flush of those before it and is then
+// alone in its block, where the flush is a rank-1 update.
+constexpr int kDuFar = 4 * 256;
 
 // Dynamic LDS of a walker, in doubles from its start.  TH > 0: rows of up to
 // 16 TH columns, so every offset but those of the arrays
@@ -312,9 +333,13 @@ __device__ __forceinline__ void du_flush(const DuLds<NB, TH, kTwo, NW> &l, doubl
     // stands for: register q of group g then holds column 16 jt + 4 g + q, so
     // a lane's four values are consecutive in memory.
     const double *pr = prow + g * l.pitch + 4 * (r & 3) + (r >> 2);
-    int own[4];  // the row of mover 4 q + g, where Z loses 1
+    // A mover's own row k is Cinv's column times P: Z of its column is -e_k and
+    // the row itself is left out (C's column times Cinv is e_k, so that the row
+    // would meet itself and leave 1/R of it, R roundings worse).
+    int own[4];  // the row of mover 4 q + g
 #pragma unroll
     for (int q = 0; q < 4; ++q) own[q] = 4 * q + g < m ? q0 + list[4 * q + g] : -1;
+    const unsigned movers = (unsigned)reinterpret_cast<const int *>(sm + Lay::ctl)[h];
     for (int kt = wave; kt < R; kt += NW) {
         const int k = 16 * kt + r;
         double *row = row_of(kt);
@@ -339,9 +364,10 @@ __device__ __forceinline__ void du_flush(const DuLds<NB, TH, kTwo, NW> &l, doubl
             for (int q = 0; q < 4; ++q)
                 c = __builtin_amdgcn_mfma_f64_16x16x4f64(pr[4 * q * l.pitch + 16 * jt], y[q], c, 0, 0, 0);
         };
+        const bool moved = (unsigned)(k - q0) < 32u && ((movers >> (k - q0)) & 1u);
         const auto solve = [&]() {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) z[q] = own[q] == k ? z[q] - 1.0 : z[q];
+            for (int q = 0; q < 4; ++q) z[q] = moved ? (own[q] == k ? -1.0 : 0.0) : z[q];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 y = __builtin_amdgcn_mfma_f64_16x16x4f64(cinv[r * (kDuMaxAcc + 1) + 4 * q + g], z[q], y, 0, 0, 0);
@@ -355,6 +381,12 @@ __device__ __forceinline__ void du_flush(const DuLds<NB, TH, kTwo, NW> &l, doubl
                 if (jt % 2) __builtin_amdgcn_sched_barrier(0);
             }
             solve();
+            if (__any(moved)) {
+#pragma unroll
+                for (int jt = 0; jt < TH; ++jt)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) c[jt][q] = moved ? 0.0 : c[jt][q];
+            }
 #pragma unroll
             for (int jt = 0; jt < TH; ++jt) {
                 update(jt, c[jt]);
@@ -382,6 +414,8 @@ __device__ __forceinline__ void du_flush(const DuLds<NB, TH, kTwo, NW> &l, doubl
 #pragma unroll 1
             for (int jt = 0; jt < T; ++jt) {
                 const du_v4d nx = load(row, jt + 1 < T ? jt + 1 : jt);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) cc[q] = moved ? 0.0 : cc[q];
                 update(jt, cc);
                 store(jt, cc);
                 cc = nx;
@@ -624,7 +658,13 @@ __device__ void du_sweep_walker(const DevSys &s, const DevState &st, int w, int 
                     for (int i = 0; i < kSub; ++i) dj += part[i * kSlots + slot];
                     const double ua = prop[3 * kSlots + slot];
                     unsigned mask[2] = {0u, 0u};
-                    int grow[2] = {0, 0};  // log2 of the accepted ratios' product, in 1/256
+                    // log2 of the accepted ratios' product since its lowest point, in 1/256
+                    int grow[2] = {0, 0};
+                    const int limit = du_growth_limit<TH, kTwo>(s);
+                    // Growth after a move of log2 ratio lg, and whether the move is to
+                    // wait for the flush of those accepted before it.
+                    const auto grown = [&](int hh, int lg) { return (grow[hh] > 0 ? grow[hh] : 0) + lg; };
+                    const auto waits = [&](int hh, int lg) { return mask[hh] && grown(hh, lg) > limit + kDuFar; };
                     double rec_r = 1.0, rec_j = 0.0;
                     int steps = cnt;
                     // Eight columns at a time by their registers, then the
@@ -639,12 +679,19 @@ __device__ void du_sweep_walker(const DevSys &s, const DevState &st, int w, int 
                             const double R = T[k], irl = rcp_nr(R);
                             const bool pivot = r == i;
                             const int au = du_decide(R, dj, ua, i);
+                            // (from within the limit only a ratio above kDuFar gets there)
+                            const unsigned long long far =
+                                __ballot(fabs(R) >= 16.0) & ((kTwo ? 0x100000001ull : 1ull) << i);
+                            if (far && ((au && waits(0, du_log2(R, i))) || (kTwo && waits(1, du_log2(R, 32 + i))))) {
+                                steps = i;
+                                break;
+                            }
                             rec_r = pivot ? R : rec_r;
                             rec_j = pivot && h == 0 ? dj : rec_j;
                             double f = 0.0;
                             if (au) {
                                 mask[0] |= 1u << i;
-                                grow[0] += du_log2(R, i);
+                                grow[0] = grown(0, du_log2(R, i));
                                 dj += X[i * kSlots + slot];
                                 const double ir = du_readlane(irl, i);
                                 f = kTwo && h ? 0.0 : du_factor(pivot, R, ir);
@@ -655,7 +702,7 @@ __device__ void du_sweep_walker(const DevSys &s, const DevState &st, int w, int 
                                 rec_j = pivot && h == 1 ? dj : rec_j;
                                 if (ad) {
                                     mask[1] |= 1u << i;
-                                    grow[1] += du_log2(R, 32 + i);
+                                    grow[1] = grown(1, du_log2(R, 32 + i));
                                     dj += X[(NB + i) * kSlots + slot];
                                     const double ir = du_readlane(irl, 32 + i);
                                     const double fd = h ? du_factor(pivot, R, ir) : 0.0;
@@ -664,10 +711,12 @@ __device__ void du_sweep_walker(const DevSys &s, const DevState &st, int w, int 
                                 }
                             }
                             // The mover's column is done: it takes the row
-                            // operations' own column.
-                            T[k] = pivot ? 1.0 - f : -f;
+                            // operations' own column (1/R itself for the mover:
+                            // 1 - f has lost R roundings, which the flush
+                            // multiplies by rows that are R times too large).
+                            T[k] = pivot ? (f != 0.0 ? irl : 1.0) : -f;
                             const int full = (int)(__popc(mask[0]) >= kDuMaxAcc) | (int)(__popc(mask[1]) >= kDuMaxAcc) |
-                                             (int)(grow[0] > kDuGrowth) | (int)(grow[1] > kDuGrowth);
+                                             (int)(grow[0] > limit) | (int)(grow[1] > limit);
                             steps = full ? i + 1 : steps;
                         }
                         double head[kG];
