@@ -239,7 +239,7 @@ int vmc_ensemble_get_inverse(vmc_ensemble *e, double *inv, void *stream);
  * and applies accepted moves as delayed Woodbury updates on the matrix cores,
  * a block of moves at a time.  VMC_KERNEL_AUTO (default) takes the register
  * kernel whenever it applies, else, in FP64, the delayed-update kernel
- * where it fits and is the faster for the electrons and walkers (from seven
+ * where it fits and is the faster for the electrons and walkers (from eight
  * electrons on, more with many walkers), else the generic kernel.  No reference counterpart: the
  * reference has a single CPU code path (its rank-1 update,
  * slater_plane_wave.cpp:367-423); this is the autotuner's knob.  VMC_ERR_INVALID if the system does not fit

@@ -35,11 +35,11 @@ def test_the_reported_kernel_can_be_set(vmc, n_up, n_dn):
 
 # Electrons up and down, walkers, and whether AUTO takes the delayed-update kernel:
 # both sides of the lines that its rule has.
-LINES = [(3, 3, 8, False), (4, 4, 8, True), (4, 4, 513, False), (5, 5, 513, True), (5, 5, 1281, False),
-         (8, 8, 1281, True), (16, 16, 1281, True), (17, 17, 1280, True), (17, 17, 1281, False),
-         (24, 24, 1281, True), (6, 0, 8, False), (8, 0, 1280, True), (8, 0, 1281, False), (12, 0, 1281, True),
-         (5, 2, 8, False), (8, 1, 512, True), (8, 1, 513, False), (12, 4, 1280, True), (19, 7, 1281, False),
-         (33, 8, 1281, True)]
+LINES = [(4, 4, 8, False), (5, 5, 512, True), (5, 5, 513, False), (6, 6, 1280, True), (6, 6, 1281, False),
+         (12, 12, 1281, True), (16, 16, 1281, True), (17, 17, 1280, True), (17, 17, 1281, False),
+         (32, 32, 1281, True), (6, 0, 8, False), (8, 0, 512, True), (8, 0, 513, False), (9, 0, 1280, True),
+         (14, 0, 1281, True), (17, 0, 1281, False), (24, 0, 1281, True), (8, 1, 8, False), (8, 4, 512, True),
+         (8, 4, 513, False), (12, 4, 1280, True), (19, 7, 1281, False), (27, 19, 1281, True)]
 
 
 @pytest.mark.parametrize("n_up,n_dn,W,delayed", LINES, ids=[f"{a}+{b}_{w}" for a, b, w, _ in LINES])

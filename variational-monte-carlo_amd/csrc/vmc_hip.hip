@@ -853,26 +853,29 @@ bool rrw_supported(const DevSys &d, int real_bytes) {
 // of these sizes in LDS.  A block of moves costs a fixed dozen phases, so it
 // takes more electrons to pay the more walkers share the chip: a walker is one
 // wavefront of the generic kernel and four or more of the block's, so beyond
-// 1024 walkers the blocks queue first.  One determinant or equal spins of up to
-// 32 electrons are one block a sweep (32 movers; 16 up to 16 per spin), unequal
-// spins two.  Time of
-// the generic sweep over the delayed one's, unmeasured / measured:
-//   up to 512 walkers   equal 3 + 3 1.24 / 0.93, 4 + 4 1.54 / 1.20; one determinant
-//                       6 1.46 / 0.99, 7 1.67 / 1.17; unequal 5 + 2 0.89 / 0.86, 8 + 1
-//                       1.11 / 1.08
-//   1280 walkers        4 + 4 0.93 / 0.95, 5 + 5 1.08 / 1.14, 23 + 23 1.53 / 1.66; 7 1.02 /
-//                       0.97, 8 1.13 / 1.07; 8 + 6 0.90 / 1.15, 12 + 4 1.06 / 1.31
-//   4096 walkers        6 + 6 0.91 / 0.98, 8 + 8 1.09 / 1.21, 16 + 16 1.87 / 1.88, 17 + 17
-//                       0.82 / 0.99, 20 + 20 0.92 / 1.08, 24 + 24 1.13 / 1.39; 10 1.01 /
-//                       0.96, 12 1.15 / 1.12; 19 + 7 0.91 / 1.09, 33 + 8 1.09 / 1.46
-//   16384 walkers       8 + 8 0.94 / 1.20, 12 1.00 / 1.10, 19 + 7 0.75 / 1.04, 25 + 5 0.87 /
-//                       1.16 (8192: 23 + 23 0.81 / 1.03, 24 + 24 0.93 / 1.17, 27 + 19 1.16 / 1.50)
-// and beyond, 40 + 40 at 4096 walkers 2.6 / 3.2 and 485 electrons at eight 31.
+// 1024 walkers the blocks queue first.  Unequal spins take a block for each
+// determinant; above 16 per spin the block of equal spins takes 68 KB of LDS
+// instead of 40, two walkers to a CU instead of four.  Time of the generic sweep
+// over the delayed one's, unmeasured / measured:
+//   256 walkers    equal 4 + 4 1.40 / 0.91, 5 + 5 1.65 / 1.12; one determinant 7 1.50 / 0.93,
+//                  8 1.64 / 1.06; unequal 6 + 4 1.11 / 0.97, 8 + 4 1.26 / 1.12
+//   1280 walkers   5 + 5 0.97 / 0.96, 6 + 6 1.11 / 1.10, 23 + 23 1.16 / 1.33; 8 1.00 / 0.93, 9
+//                  1.09 / 1.00; 8 + 6 0.84 / 1.02, 12 + 4 0.95 / 1.15, 14 + 5 1.05 / 1.26
+//   4096 walkers   10 + 10 1.02 / 1.16, 12 + 12 1.13 / 1.27, 16 + 16 1.47 / 1.55, 17 + 17 0.67 /
+//                  0.82, 30 + 30 0.94 / 1.28, 32 + 32 1.79 / 1.85; 12 1.01 / 1.01, 14 1.11 /
+//                  1.13, 17 0.93 / 1.01, 24 1.23 / 1.25; 19 + 7 0.78 / 0.96, 33 + 8 1.02 /
+//                  1.35, 27 + 19 1.16 / 1.51
+//   8192 walkers   10 + 10 0.91 / 1.16, 12 + 12 0.99 / 1.26, 30 + 30 0.94 / 1.27, 34 + 34 1.32 /
+//                  1.80; 14 0.98 / 1.12, 20 0.91 / 1.09, 24 1.05 / 1.23; 33 + 8 0.84 / 1.16,
+//                  27 + 19 0.98 / 1.32
+// and beyond, 50 + 50 at 4096 walkers 2.7 / 3.3 and 485 electrons at eight 80 / 30.
 bool du_pays(const DevSys &d, int64_t W) {
     const bool one = d.ndet == 1, equal = !one && d.n_up == d.n_dn;
-    if (W > 1280) return equal ? d.N >= 16 && (d.N <= 32 || d.N >= 48) : d.N >= (one ? 12 : 40);
-    if (W > 512) return d.N >= (equal ? 10 : one ? 8 : 16);
-    return d.N >= (equal ? 8 : one ? 7 : 9);
+    const int N = d.N;
+    if (W <= 512) return N >= (equal ? 10 : one ? 8 : 12);
+    if (W <= 1280) return N >= (equal ? 12 : one ? 9 : 16);
+    if (equal) return (N >= 24 && N <= 32) || N >= 64;
+    return one ? (N >= 14 && N <= 16) || N >= 24 : N >= 46;
 }
 
 // Sweep kernel family of an ensemble: the register-resident kernels where an
