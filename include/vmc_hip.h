@@ -248,9 +248,8 @@ int vmc_ensemble_set_kernel(vmc_ensemble *e, int32_t kernel);
 /* The kernel the next sweep launch will use (VMC_KERNEL_GENERIC, _REGISTER
  * or _DELAYED). */
 int vmc_ensemble_get_kernel(const vmc_ensemble *e, int32_t *kernel);
-/* Register-kernel build variant, 0 or 1: both are the same kernel now that
- * every one fits 128 VGPRs (4 waves per SIMD) without spills.  No reference
- * counterpart. */
+/* Register-kernel build variant, 0 or 1 (a saved tuning may hold either):
+ * both select the one build there is.  No reference counterpart. */
 int vmc_ensemble_set_rr_variant(vmc_ensemble *e, int32_t variant);
 /* Walker groups of the register kernels' measured sweeps: the walkers are
  * split into `groups` contiguous ranges (1 to 8; default 1), each swept and
@@ -394,7 +393,7 @@ int vmc_ensemble_footprint(const vmc_system *sys, int64_t n_walkers, int64_t *by
 typedef struct vmc_tuning {
     int32_t kernel;            /* VMC_KERNEL_GENERIC, _REGISTER or _DELAYED */
     int32_t walker_threads;    /* generic kernel: 64, 128 or 256 threads per walker */
-    int32_t rr_variant;        /* register kernel build variant */
+    int32_t rr_variant;        /* 0 (vmc_ensemble_set_rr_variant) */
     int32_t inv_placement;     /* generic kernel: 1 LDS, 2 HBM */
     int32_t reinvert_interval; /* chosen K (mixed); the system's own value in FP64 */
     double moves_per_s;        /* electron-moves/s of the chosen settings */

@@ -1863,9 +1863,9 @@ struct vmc_batch {
 
 namespace {
 
-// Kernel family of a batch member, by the rule the ensemble's own sweep
-// uses: register-resident when an instantiation exists and the member does
-// not ask for the generic kernel.
+// Kernel family of a batch member: register-resident when an instantiation
+// exists and the member does not ask for the generic kernel, else the generic
+// one (an FP64 system that alone would take the delayed-update kernel as well).
 int batch_family(const vmc_ensemble *e) {
     const DevSys &d = e->tables.dev;
     if (e->kernel == VMC_KERNEL_GENERIC) return 0;

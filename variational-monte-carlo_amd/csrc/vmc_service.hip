@@ -68,7 +68,7 @@ namespace {
 int walker_threads_for(const vmc_system &s) { return vmc_default_walker_threads(&s); }
 
 struct Candidate {
-    int kernel, variant, placement, threads;
+    int kernel, placement, threads;
 };
 
 // Device time of `sweeps` measured sweeps of a fresh ensemble with the given
@@ -79,8 +79,7 @@ double time_candidate(const vmc_system &sys, int64_t W, const Candidate &c, int 
     if (vmc_ensemble_create(&sys, W, 12345, 0.1 * sys.box_length, &e)) return -1.0;
     double ms = -1.0;
     hipEvent_t a = nullptr, b = nullptr;
-    if (!vmc_ensemble_set_kernel(e, c.kernel) && !vmc_ensemble_set_rr_variant(e, c.variant) &&
-        !vmc_ensemble_set_inverse_placement(e, c.placement) &&
+    if (!vmc_ensemble_set_kernel(e, c.kernel) && !vmc_ensemble_set_inverse_placement(e, c.placement) &&
         !vmc_ensemble_set_walker_threads(e, c.threads) && !vmc_ensemble_init_positions(e, s) &&
         !vmc_ensemble_sweep(e, 2, VMC_SWEEP_ADAPT, 1, s) && hipEventCreate(&a) == hipSuccess &&
         hipEventCreate(&b) == hipSuccess && hipEventRecord(a, s) == hipSuccess &&
@@ -115,13 +114,13 @@ int vmc_autotune(const vmc_system *sys, int64_t n_walkers, double drift_tol, int
         int rc = vmc_ensemble_create(sys, 1, 1, 0.1 * sys->box_length, &e);
         if (rc) return rc;
         if (!vmc_ensemble_set_kernel(e, VMC_KERNEL_REGISTER)) {
-            cands.push_back({VMC_KERNEL_REGISTER, 0, 0, 64});
+            cands.push_back({VMC_KERNEL_REGISTER, 0, 64});
         }
-        if (!vmc_ensemble_set_kernel(e, VMC_KERNEL_DELAYED)) cands.push_back({VMC_KERNEL_DELAYED, 0, 0, 64});
+        if (!vmc_ensemble_set_kernel(e, VMC_KERNEL_DELAYED)) cands.push_back({VMC_KERNEL_DELAYED, 0, 64});
         const bool lds_ok = !vmc_ensemble_set_inverse_placement(e, 1);
         for (int th : {64, 128, 256}) {
-            if (lds_ok) cands.push_back({VMC_KERNEL_GENERIC, 0, 1, th});
-            cands.push_back({VMC_KERNEL_GENERIC, 0, 2, th});
+            if (lds_ok) cands.push_back({VMC_KERNEL_GENERIC, 1, th});
+            cands.push_back({VMC_KERNEL_GENERIC, 2, th});
         }
         vmc_ensemble_destroy(e);
     }
@@ -148,7 +147,7 @@ int vmc_autotune(const vmc_system *sys, int64_t n_walkers, double drift_tol, int
             best = rate;
             out->kernel = c.kernel;
             out->walker_threads = c.threads;
-            out->rr_variant = c.variant;
+            out->rr_variant = 0;
             out->inv_placement = c.placement;
         }
     }

@@ -271,23 +271,6 @@ __device__ __forceinline__ Cx<Real> axis_phasor(double x, double inv_L) {
     return p;
 }
 
-// Compile-time power a^n (n >= 0).
-template <int NPOW, typename Real>
-__device__ __forceinline__ Cx<Real> cpow_ct(Cx<Real> a) {
-    if constexpr (NPOW == 0) {
-        return Cx<Real>{(Real)1, (Real)0};
-    } else if constexpr (NPOW == 1) {
-        return a;
-    } else {
-        return cmul(a, cpow_ct<NPOW - 1, Real>(a));
-    }
-}
-
-template <typename Real>
-__device__ __forceinline__ Cx<Real> cconj(Cx<Real> a) {
-    return {a.re, -a.im};
-}
-
 // Orbital phasor e^{2 pi i n.u} from the three axis phasors and their squares.
 template <typename Real>
 __device__ __forceinline__ Cx<Real> orbital_phasor(int nx, int ny, int nz, const Cx<Real> a[3],
@@ -301,11 +284,6 @@ __device__ __forceinline__ Cx<Real> orbital_phasor3(int nx, int ny, int nz, cons
                                                     const Cx<Real> a2[3], const Cx<Real> a3[3]) {
     return cmul(cmul(cpow3(nx, a[0], a2[0], a3[0]), cpow3(ny, a[1], a2[1], a3[1])),
                 cpow3(nz, a[2], a2[2], a3[2]));
-}
-
-template <typename Real>
-__device__ __forceinline__ Real jastrow_pair(Real r, Real a, Real b) {
-    return a * r / ((Real)1 + b * r);
 }
 
 }  // namespace rr
