@@ -442,10 +442,12 @@ size_t measure64_lds(const DevSys &d) {
 constexpr int kMsMinN = 6;
 bool measure64_fits(const DevSys &d) { return d.N >= kMsMinN && measure64_lds(d) <= kMeasure64LdsLimit; }
 
-// Dynamic LDS above 64 KB has to be asked for, kernel by kernel.
+// Dynamic LDS above 64 KB has to be asked for, kernel by kernel; always up to
+// the limit, so that two threads with systems of different sizes ask for the
+// same.
 static bool ms_allow(const void *kernel, size_t lds) {
-    return lds <= 64 * 1024 ||
-           hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    return lds <= 64 * 1024 || hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   (int)kMeasure64LdsLimit) == hipSuccess;
 }
 
 bool measure64(const DevSys &d, const DevState &st64, unsigned grid, int bs, double *parts, hipStream_t stream) {

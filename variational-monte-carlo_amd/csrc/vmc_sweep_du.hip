@@ -868,9 +868,10 @@ bool du_launch(const DevSys &d, const DevState &st, unsigned grid, int n_sweeps,
     const size_t lds = du_lds(d);
     const auto run = [&]<int NB, int TH, bool kTwo, int NW>() {
         const auto k = k_sweep_du<NB, TH, kTwo, NW>;
+        // (up to the limit: the same from every thread, whatever its system)
         if (lds > 64 * 1024 &&
             hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds) != hipSuccess)
+                                (int)kDuLdsLimit) != hipSuccess)
             return false;
         hipLaunchKernelGGL(k, dim3(grid), dim3(NW * kWave), lds, stream, d, st, n_sweeps, s0, flags, given);
         return true;

@@ -1534,7 +1534,7 @@ __device__ __forceinline__ void measure_rr_body(const DevSys &s, const DevState 
 // At 27 per spin one trip takes 19 KB, two walkers to a SIMD, and two trips 10 KB,
 // four: per measured sweep one trip against two, 1 walker 78 / 87 us, 1024 92 / 105,
 // 2048 114 / 130, 2560 162 / 153, 4096 213 / 192, 8192 371 / 342 (two trips build the
-// D rows in two half-empty passes and spill).  At 19 per spin one trip takes 9 KB:
+// D rows in two half-empty passes and spill).  At 19 per spin one trip takes 9.5 KB:
 // 62 / 67 at 1024, 117 / 122 at 4096 (147 with E's columns in LDS beside whole rows).
 template <int NU, int ND, int kTrips>
 struct RRMixedShared {
