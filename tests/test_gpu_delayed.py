@@ -1,8 +1,8 @@
 """GPU parity of the FP64 delayed-update sweep (vmc_sweep_du.hip).
 
 The delayed-update kernel keeps each determinant's FP64 inverse in HBM and
-applies accepted moves in windows of eight as Woodbury updates on the matrix
-cores; the reference updates the whole inverse on every accepted move
+applies accepted moves a block of up to 16 at a time as Woodbury updates on the
+matrix cores; the reference updates the whole inverse on every accepted move
 (slater_plane_wave.cpp:367-423).  In FP64 both are the same chain: the
 device follows the oracle's Philox twin move for move, with the local energy
 after every sweep within 1e-9 of the oracle's at the same positions.
@@ -42,7 +42,7 @@ def test_delayed_chain_follows_the_oracle_twin(vmc, oracle, N, rs, W, sweeps, fo
 
 def test_delayed_inverse_after_many_sweeps(vmc, oracle):
     """N = 294 (147 + 147) in FP64 over 30 adaptive sweeps of 64 walkers:
-    the inverse the windows leave in HBM equals a fresh FP64 inversion at the
+    the inverse the blocks leave in HBM equals a fresh FP64 inversion at the
     final positions to 1e-9 of its largest element, and log|det| tracked
     through the accepted ratios matches the fresh one."""
     s = vmc.System.heg(294, 2.0, 1.0)

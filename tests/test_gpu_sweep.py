@@ -46,6 +46,8 @@ def test_init_positions_match_oracle(vmc, oracle, name, factory):
         np.testing.assert_array_equal(gpu[w], pos)
 
 
+# (both build variants of the register kernel are one kernel now: the second row
+# holds the entry point to accepting either)
 KERNELS = [("generic", 1, 0), ("register", 2, 0), ("register_o4", 2, 1)]
 
 

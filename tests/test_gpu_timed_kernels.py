@@ -40,8 +40,8 @@ CASES = [
     ("heg162", lambda V, p: V.System.heg(162, 2.0, 1.0, precision=p), 32, "register"),
     ("heg54_generic", lambda V, p: V.System.heg(54, 2.0, 1.0, precision=p), 64, "generic"),
 ]
-# FP64 with the delayed-update kernel (inverse in HBM, rank-8 Woodbury
-# windows): forced at sizes the register kernels also run, and chosen by
+# FP64 with the delayed-update kernel (inverse in HBM, blocks of moves as
+# Woodbury updates): forced at sizes the register kernels also run, and chosen by
 # itself at 123 and 147 per spin.
 FP64_DELAYED = [
     ("heg14_delayed", lambda V, p: V.System.heg(14, 1.0, 1.0, precision=p), 64, "delayed"),

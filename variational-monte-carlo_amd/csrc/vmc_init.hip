@@ -12,10 +12,11 @@
 // then rotate by one, so every register index is a constant.
 //
 // What bounds it: the chain of n steps, each a workgroup maximum, two barriers
-// and the broadcast of the pivot row through LDS: 88 us for 1024 walkers at 33
-// per spin, 554 us for 1000 at 81, 2.2 ms for 1024 at 147; one wavefront per
-// walker with the matrix in memory took 435 us at 33 and 42.6 ms at 147.  Above
-// 160 a lane's row no longer fits its registers.
+// and the broadcast of the pivot row through LDS: 61 us for 1024 walkers at 33
+// per spin, 525 us for 1000 at 81, 1.28 ms for 1024 at 123 and 2.13 at 147; one
+// wavefront per walker with the matrix in memory took 435 us at 33 and 42.6 ms at
+// 147.  Above 128 a lane's row begins to spill (36 B of scratch per lane), above
+// 160 it is left to the kernel in memory.
 // FP64 inverses only: the elimination rounds in another order than k_init's, which
 // moves about one FP32 element in a million by its last place, and an FP32 chain
 // turns that into another accept decision now and then.

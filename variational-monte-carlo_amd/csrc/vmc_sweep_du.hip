@@ -28,14 +28,15 @@
 // A block ends early when 16 moves are accepted in one determinant or when
 // the product of its accepted ratios exceeds a limit (du_growth_limit).
 //
-// What bounds it (N = 294, 1024 walkers, 1.70 ms a sweep): FP64 VALU work (43 %
+// What bounds it (N = 294, 1024 walkers, 1.77 ms a sweep): FP64 VALU work (43 %
 // of the cycles, the pair terms above all) and FP64 MFMA issue (24 %) of two
 // resident workgroups; alone on its CU a walker takes 0.51 ms, of which the
 // decisions are a fifth, the flushes a third and T beside the pair terms 30 %.
 // Against one inverse row read, five barriers and an 8-entry window solved by
-// serial lane reads per move: 7.84 -> 1.70 ms a sweep at N = 294 and 3.88 -> 1.14
-// at N = 246 (1024 walkers), 0.46 -> 0.07 ms at 19 + 7 electrons (777 walkers,
-// against the generic kernel), 138 -> 3.5 ms at 485 (8 walkers, the same).
+// serial lane reads per move: 7.84 -> 1.77 ms a sweep at N = 294 and 3.88 -> 1.12
+// at N = 246 (1024 walkers); against the generic kernel 0.075 -> 0.050 ms at 19 + 7
+// electrons (777 walkers, several sweeps a launch; 0.078 one at a time) and 138
+// -> 4.3 at 485 (8 walkers).  20 to 112 B of spill per lane at 128 registers.
 //
 // The chain is the generic kernel's (vmc_hip.hip sweep_walker): the same
 // Philox draws, sweep order and FP64 accept test, so the FP64 trajectory

@@ -516,10 +516,11 @@ __device__ __forceinline__ void sweep_rrw_body(const DevSys &s, const DevState &
 }
 
 // Waves per SIMD the sweep kernel is compiled for.  57 + 57 and 81 + 81 in
-// FP32 take four (at most 128 VGPRs, 16 and 32 B of spill per lane): eight
-// and four walkers per CU, so 2048 and 1024 walkers are resident at once.
-// 123 + 123 takes three (168 VGPRs, 32 B of spill); 147 + 147 stays at two
-// (three would spill 144 B of its inverse row per lane and run at half speed).
+// FP32 take four (at most 128 VGPRs, 56 and 68 B of spill per lane; 84 and 68 in
+// a batch): eight and four walkers per CU, so 2048 and 1024 walkers are resident
+// at once.  123 + 123 takes three (168 VGPRs, 76 B of spill, 128 in a batch), FP64
+// 57 + 57 as well (168, 32 B); 147 + 147 stays at two (244 VGPRs; three would spill
+// 144 B of its inverse row per lane and run at half speed).
 template <typename Real, int NU, int ND, int WPS>
 constexpr int rrw_sweep_waves() {
     return (sizeof(Real) == 4 && ((NU == 57 && ND == 57) || (NU == 81 && ND == 81))) ? 4
