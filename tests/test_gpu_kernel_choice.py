@@ -87,3 +87,19 @@ def test_autotune_considers_the_delayed_kernel_for_unequal_spins(vmc):
     e.sweep(2, measure=True)
     assert np.all(e.stats()[:, vmc.STAT["NMEAS"]] == 2)
     e.close()
+
+
+def test_a_batch_member_reports_the_kernel_of_its_group(vmc):
+    """A batch takes the register kernels or the generic one: an FP64 member
+    that alone would take the delayed-update kernel reports the generic one."""
+    sy = [gas(vmc, 19, 7), gas(vmc, 27, 27), gas(vmc, 93, 93)]
+    b = vmc.Batch(sy, [4, 4, 2], [1, 2, 3])
+    fam, grp = b.groups()
+    want = [vmc.KERNEL_REGISTER if fam[g] else vmc.KERNEL_GENERIC for g in grp]
+    assert [b.member(i).kernel() for i in range(3)] == want
+    assert want == [vmc.KERNEL_GENERIC, vmc.KERNEL_REGISTER, vmc.KERNEL_GENERIC]
+    b.close()
+    for s, k in zip(sy, (vmc.KERNEL_DELAYED, vmc.KERNEL_REGISTER, vmc.KERNEL_DELAYED)):
+        e = vmc.Ensemble(s, 4, 1)
+        assert e.kernel() == k
+        e.close()

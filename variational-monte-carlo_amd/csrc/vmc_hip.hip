@@ -1580,8 +1580,9 @@ int vmc_ensemble_set_walker_threads(vmc_ensemble *e, int32_t threads) {
 int vmc_ensemble_get_kernel(const vmc_ensemble *e, int32_t *kernel) {
     if (!e || !kernel) return fail(VMC_ERR_INVALID, "NULL argument");
     const int fam = sweep_family(e);
+    // (a batch sweeps such a member with the generic kernel, batch_family)
     *kernel = fam == kFamRegister || fam == kFamMultiwave ? VMC_KERNEL_REGISTER
-              : fam == kFamDelayed                        ? VMC_KERNEL_DELAYED
+              : fam == kFamDelayed && !e->in_batch        ? VMC_KERNEL_DELAYED
                                                           : VMC_KERNEL_GENERIC;
     return VMC_OK;
 }
