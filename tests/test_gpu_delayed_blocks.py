@@ -17,7 +17,8 @@ from helpers import oracle_system
 pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 0), (2, 1), (8, 1), (16, 16), (17, 17), (19, 7), (7, 19), (32, 32), (34, 33), (48, 48), (49, 49),
-         (64, 64), (65, 65), (96, 96), (97, 97), (128, 0), (129, 129), (160, 160), (161, 0), (177, 5)]
+         (64, 64), (65, 65), (96, 96), (97, 97), (128, 0), (129, 129), (160, 160), (161, 0), (161, 161), (177, 5),
+         (161, 180)]
 
 
 @pytest.mark.parametrize("n_up,n_dn", SIZES, ids=[f"{a}+{b}" for a, b in SIZES])
